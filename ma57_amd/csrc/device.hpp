@@ -126,8 +126,19 @@ __host__ __device__ inline bool specFront(const FactorParams& p, int nE) { retur
 // panel column q at i + q m), from which a failed test restores them.
 constexpr int kSpecRec = 8 * kPanel + 2 * kPanel * kPanel;
 constexpr int kSpecRows = 256;  // rows below the block per workgroup (one per thread)
-__host__ __device__ inline int64_t panelWorkspace(int m, int nE, bool spec) {
+// The panel kernel keeps up to kPanelRegRows rows in registers; a front with
+// more eligible rows streams them through 16 more columns of its workspace.
+constexpr int kPanelRegRows = 2048;
+__host__ __device__ inline int64_t panelStreamOffset(int m, int nE, bool spec) {
   return 2 * static_cast<int64_t>(nE) + kSpecRec + (spec ? static_cast<int64_t>(m) * kPanel : 0);
 }
+__host__ __device__ inline int64_t panelWorkspace(int m, int nE, bool spec) {
+  return panelStreamOffset(m, nE, spec) + (nE > kPanelRegRows ? 16 * static_cast<int64_t>(nE) : 0);
+}
+// A front of at most kPanelAllRows rows has its panels' multipliers formed
+// for all its rows by the panel kernel itself (its few tiles cost less there
+// than another launch); spec: the front takes the speculative step instead.
+constexpr int kPanelAllRows = 256;
+__host__ __device__ inline bool panelHoldsAllRows(int m, bool spec) { return !spec && m <= kPanelAllRows; }
 
 }  // namespace symla_hip

@@ -14,6 +14,8 @@
 
 #include <cfloat>
 #include <cmath>
+#include <type_traits>
+#include <utility>
 
 namespace symla_hip {
 
@@ -564,6 +566,212 @@ size_t smallFrontSmemBytes(int m) {
 }
 
 // ---------------------------------------------------------------------------
+// Building blocks of the panel kernels.
+// ---------------------------------------------------------------------------
+// A front pointer read from the front table is generic; generic (flat)
+// accesses count against the LDS wait counter too, so every LDS wait would
+// also wait for them.  Front storage is global memory: this view makes the
+// accesses global ones.
+template <typename T>
+using GlobalPtr = __attribute__((address_space(1))) T*;
+template <typename T>
+__device__ inline GlobalPtr<T> globalView(void* p) {
+  return (GlobalPtr<T>)(p);
+}
+
+// Row values loaded in their storage type, every load issued before any is
+// used: each load is unconditional (a skipped element reads the front's first
+// entry, a valid address, and is zeroed afterwards), since a load under a
+// branch completes before the branch joins.
+template <int N, typename P, typename Off>
+__device__ inline void loadWiden(double (&x)[N], P base, Off off) {
+  decltype(+base[0]) raw[N];
+  bool ok[N];
+#pragma unroll
+  for (int q = 0; q < N; ++q) {
+    const int64_t o = off(q);
+    ok[q] = o >= 0;
+    raw[q] = base[ok[q] ? o : 0];
+  }
+#pragma unroll
+  for (int q = 0; q < N; ++q) x[q] = ok[q] ? static_cast<double>(raw[q]) : 0.0;
+}
+
+// 1 / d for a pivot on a dependent chain: the hardware reciprocal refined by
+// two Newton steps (within an ulp of the quotient), an IEEE division for
+// zero, denormal and non-finite d.
+__device__ inline double pivotRecip(double d) {
+  const double a = fabs(d);
+  double r = __builtin_amdgcn_rcp(d);
+  r = fma(fma(-d, r, 1.0), r, r);
+  r = fma(fma(-d, r, 1.0), r, r);
+  // (one branch for the wave, rarely taken)
+  const bool special = !(a >= DBL_MIN && a <= DBL_MAX);
+  if (__builtin_expect(__ballot(special) != 0, 0)) r = special ? 1.0 / d : r;
+  return r;
+}
+
+// A double of lane `src` (the same for the whole wave) in every lane.
+__device__ inline double readLane(double v, int src) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), src);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), src);
+  return __hiloint2double(hi, lo);
+}
+
+template <int CTRL>
+__device__ inline double dppMove(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+// Maximum over each group of 16 consecutive lanes, in all of them.
+__device__ inline double max16(double v) {
+  v = fmax(v, dppMove<0xB1>(v));   // lanes 1, 0, 3, 2 of a quad
+  v = fmax(v, dppMove<0x4E>(v));   // lanes 2, 3, 0, 1
+  v = fmax(v, dppMove<0x124>(v));  // 16-lane row rotated by 4
+  v = fmax(v, dppMove<0x128>(v));  // and by 8
+  return v;
+}
+
+// The panel kernels hold 16 rows x 16 panel columns as one FP64 MFMA result
+// of the transposed block: lane j + 16 c, register s is row j, column
+// 4 s + c.  That is also the layout of the instruction's second operand when
+// its step s takes the columns 4 s .. 4 s + 3, so a solved group of four
+// columns feeds the products with the later columns straight from the
+// registers it was formed in.
+typedef double v4d __attribute__((ext_vector_type(4)));
+__device__ inline v4d mfma64(double a, double b, v4d c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+
+// Inverse of a 4 x 4 unit lower block, rows 1 .. 3 of column k (column 0
+// first): m[r][k] for r > k.
+struct Inv4 {
+  double m10, m20, m21, m30, m31, m32;
+};
+__device__ inline Inv4 invUnit4(double l10, double l20, double l21, double l30, double l31, double l32) {
+  Inv4 v;
+  v.m10 = -l10;
+  v.m21 = -l21;
+  v.m32 = -l32;
+  v.m20 = fma(l21, l10, -l20);
+  v.m31 = fma(l32, l21, -l31);
+  v.m30 = -(l30 + l31 * v.m10 + l32 * v.m20);
+  return v;
+}
+
+// Waits for the matrix cores' results in x: 20 wait states cover an FP64
+// 16x16x4 product.  The compiler keeps that distance for reads in
+// straight-line code, but a register of a result that nothing reads may be
+// given another value after only 11 (the late result then lands on top of
+// it), and where a branch may be taken in between it can measure a read's
+// distance along the longer way.  So every result of which only a part is
+// used, or which is read after a branch, is settled whole.
+__device__ inline void settle(v4d& x) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x)); }
+
+// Workgroup barrier that orders LDS accesses only: stores to global memory
+// stay in flight across it.
+__device__ inline void ldsBarrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// One substitution step of a 16-column block held as above: x_s <- M_s x_s
+// for the four columns of group s, and the groups after it take
+// x -= L M_s x_s.  `a` is the step's operand (substOps); the groups before s
+// are left alone, so values of a later column never reach an earlier one.
+template <int S>
+__device__ inline void substStep(v4d& x, double a) {
+  v4d d = mfma64(a, x[S], x);
+  settle(d);
+#pragma unroll
+  for (int r = S; r < 4; ++r) x[r] = d[r];
+}
+
+// The substitution of one 16-row tile by a 16-column block: x becomes the
+// current values c_iq at each column's pivot.
+__device__ inline void substTile(v4d& x, const double (&op)[4]) {
+  substStep<0>(x, op[0]);
+  substStep<1>(x, op[1]);
+  substStep<2>(x, op[2]);
+  substStep<3>(x, op[3]);
+}
+
+// Lane J of each 16-lane group in every lane of the group.
+template <int J>
+__device__ inline double bcast16(double v) {
+  return __longlong_as_double(__builtin_amdgcn_update_dpp(0ll, __double_as_longlong(v), 0x150 + J, 0xf, 0xf, true));
+}
+// a += (lane J's v of each 16-lane group) * w in one instruction; the caller
+// leaves two wait states after the last write of v.
+template <int J>
+__device__ inline void fmaBcast16(double& a, double v, double w) {
+  asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(v), "v"(w), "n"(J));
+}
+
+template <int... I, typename Fn>
+__device__ inline void unrolled(std::integer_sequence<int, I...>, Fn&& fn) {
+  (fn(std::integral_constant<int, I>{}), ...);
+}
+
+// A 16 x 16 diagonal block's factorization and the operands of its
+// substitution, in LDS for every wave of the workgroup.
+struct Block16 {
+  double op[4][64];  // step s, lane i + 16 k: row i, column 4 s + k of [M_s - I within the group; -L M_s after it]
+  double akk[16];    // current diagonal at each pivot
+  double d[16], rd[16];  // the pivots (pivotOf) and their reciprocals
+};
+
+// LDL^T of a 16 x 16 block with 1x1 pivots in order, by one wave without
+// barriers or branches: lane i (mod 16; the four groups work alike) holds
+// row i of the lower triangle in a[], rows of a smaller block's padding those
+// of the identity.  pivotOf(q, a_qq) is the pivot (for a lane's own column
+// with q the lane).  Multipliers are rounded to the front's type T.  The
+// chain per pivot is one reciprocal and one product; a pivot row's
+// multipliers reach the other rows as DPP operands of the updates, one
+// instruction each (through lane reads into scalar registers, with a branch
+// or two per pivot, a block took 8000 cycles).  Only 4 x 4 blocks are
+// inverted for the substitution, so its rounding is close to that of a
+// column-by-column one.
+template <typename T, typename PivotOf>
+__device__ inline void blockFactor16(double (&a)[16], Block16& B, PivotOf pivotOf) {
+  const int lane = threadIdx.x & 63, i = lane & 15, k = lane >> 4;
+  auto stored = [](double c, double r) { return static_cast<double>(static_cast<T>(c * r)); };
+  unrolled(std::make_integer_sequence<int, 16>{}, [&](auto qq) {
+    constexpr int q = decltype(qq)::value;
+    double l = stored(a[q], pivotRecip(pivotOf(q, bcast16<q>(a[q]))));
+    const double c = -a[q];
+    asm volatile("s_nop 1" : "+v"(l));
+    unrolled(std::make_integer_sequence<int, 15 - q>{}, [&](auto jj) {
+      constexpr int j = q + 1 + decltype(jj)::value;
+      fmaBcast16<j>(a[j], l, c);
+    });
+  });
+  double akk = a[0];
+#pragma unroll
+  for (int q = 1; q < 16; ++q) akk = i == q ? a[q] : akk;
+  const double d = pivotOf(i, akk);
+  B.akk[i] = akk;  // (the four groups store the same values)
+  B.d[i] = d;
+  const double rd = pivotRecip(d);
+  B.rd[i] = rd;
+  unrolled(std::make_integer_sequence<int, 4>{}, [&](auto ss) {
+    constexpr int s = decltype(ss)::value, c = 4 * s;
+    // this row's multipliers in the group's columns (the values of the loop above)
+    const double l0 = stored(a[c], bcast16<c>(rd)), l1 = stored(a[c + 1], bcast16<c + 1>(rd));
+    const double l2 = stored(a[c + 2], bcast16<c + 2>(rd)), l3 = stored(a[c + 3], bcast16<c + 3>(rd));
+    const Inv4 v = invUnit4(bcast16<c + 1>(l0), bcast16<c + 2>(l0), bcast16<c + 2>(l1), bcast16<c + 3>(l0),
+                            bcast16<c + 3>(l1), bcast16<c + 3>(l2));
+    const double m0 = k == 0 ? 1.0 : 0.0;  // column k of M_s
+    const double m1 = k == 0 ? v.m10 : (k == 1 ? 1.0 : 0.0);
+    const double m2 = k == 0 ? v.m20 : (k == 1 ? v.m21 : (k == 2 ? 1.0 : 0.0));
+    const double m3 = k == 0 ? v.m30 : (k == 1 ? v.m31 : (k == 2 ? v.m32 : 1.0));
+    const double below = -(l0 * m0 + l1 * m1 + l2 * m2 + l3 * m3);
+    const int r = i - c;
+    B.op[s][lane] = r <= k ? 0.0 : (r == 1 ? m1 : (r == 2 ? m2 : (r == 3 ? m3 : below)));
+  });
+}
+
+// ---------------------------------------------------------------------------
 // Large fronts.
 // ---------------------------------------------------------------------------
 
@@ -589,46 +797,80 @@ __global__ __launch_bounds__(256) void k_front_maxabs(const int* list, int count
   if (lane == 0) atomicMaxNonNeg(fd.origMaxBits + s, v);
 }
 
-// Panel pivoting on the eligible rows [k, nE) of one front.  Columns not yet
-// pivoted are never modified in place in global memory: the current value of
-// a candidate column is its stored (pre-panel) value minus the correction of
-// this panel's pivots, like the reference's setColumnRaw
-// (dense_kernel.hpp:516-545).  Accepted pivots write their multipliers for
-// the eligible rows; the remaining rows are solved by k_panel_rows.
+// Panel pivoting of one front: one workgroup takes the panel's (up to 64)
+// pivots on the rows it holds, the eligible rows [k, nE), or every row
+// [k, m) of a front that panelHoldsAllRows.  Columns not yet pivoted are
+// never modified in place: the current value of a candidate column is its
+// stored (pre-panel) value minus the correction of this panel's pivots, like
+// the reference's setColumnRaw (dense_kernel.hpp:516-545).  Accepted pivots
+// write their multipliers for the held rows; the remaining rows are solved
+// by k_panel_rows.
 //
-// When every eligible row fits RM slots per thread (RM > 0), the next SW
-// columns from the current pivot (a sub-panel) are loaded into LDS with the
-// correction of the panel's earlier pivots applied once, then factored
-// right-looking inside LDS: a pivot accepted by the first Bunch-Kaufman test
-// (every static pivot) costs one barrier and no global reads.  Any other
-// decision runs the general code, which works on column buffers in global
-// memory, and the sub-panel is reloaded after it.
-template <int RM>
+// The next 16 columns from the current pivot are worked on at once.  Their
+// current values are formed on the FP64 matrix cores (16 rows x 16 columns
+// per tile, the panel's earlier pivots as the inner dimension), one wave
+// factors the 16 x 16 diagonal block with 1x1 pivots in order, the rows
+// below follow by MFMA substitution, and one reduction gives
+// lambda = max |a_ik| of every column.  The pivots before the first column
+// whose test |a_kk| >= alpha lambda fails are kept: the same decisions as
+// pivot by pivot, up to the order of rounding.  The failing column takes the
+// general step on column buffers, and the next block starts after it.
+//
+// What bounds it: the dependent chain (16 reciprocals per block, the
+// barriers, memory round trips), then for many rows the one CU's FP64 rate:
+// 64 columns of R rows take about 2048 R multiply-adds.  TPW 16-row tiles
+// per wave stay in registers (128 TPW rows); TPW = 0 streams any number of
+// rows eight tiles at a time, with the block's current values in the
+// workspace between the test and the multipliers.  A panel of few rows
+// (PanelShape::kInLds) lives in LDS from its first load to its write-back, so
+// the earlier multipliers, the interchanges and the general step's columns
+// cost no memory round trip.
+//
+// Measured per panel of 64 columns (FP64, before: sub-panels of eight columns
+// in LDS, each thread factoring the 8 x 8 block, rows loaded slot by slot):
+// 30x30x30 27-point fronts, few failing columns, <= 128 rows 103 -> 24 us,
+// <= 512 rows 103 -> 55, <= 2048 rows 153 -> 129; 100x100 5-point fronts, a
+// failing column in about every eight, 210 -> 105 us.  A block takes about
+// 15,000 cycles there (6,000 of them the diagonal block), a general step
+// 8,000.
+constexpr int kPanelCols = 16;  // columns per block
+template <int TPW, typename T>
 struct PanelShape {
-  // sub-panel width (a wider one saves reloads but costs LDS traffic on every pivot)
-  static constexpr int SW = RM <= 4 ? 8 : (RM <= 8 ? 4 : (RM <= 16 ? 2 : 1));
-  static constexpr int ROWS = RM > 0 ? RM * kPanelThreads : 0;
-  static constexpr size_t lds() { return sizeof(double) * static_cast<size_t>(ROWS) * SW; }
+  static constexpr int kRows = 128 * TPW;
+  // column stride in LDS: half the banks on from one column to the next, so
+  // the four columns of an operand read do not collide
+  static constexpr int kLd = kRows + 16;
+  static constexpr bool kInLds = TPW > 0 && sizeof(T) * kRows <= 2048;
+  static constexpr size_t lds() { return kInLds ? sizeof(T) * kPanel * kLd : 0; }
 };
-
-template <int RM, typename T>
+template <int TPW, typename T>
 __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int count, DevFronts fd, FactorParams prm,
                                                           double* wsBase, const int64_t* wsOff) {
+  using Shape = PanelShape<TPW, T>;
+  constexpr bool kInLds = Shape::kInLds;
+  constexpr int LD = Shape::kLd;
   constexpr int NT = kPanelThreads;
-  constexpr int SW = PanelShape<RM>::SW;
-  constexpr int CSR = PanelShape<RM>::ROWS;
-  extern __shared__ double Cs[];  // [SW][CSR]: sub-panel column j, row k0 + r at Cs[j * CSR + r]
-  __shared__ double Wsub[SW][kPanel + 2];
-  __shared__ double wvec[kPanel + 2];
-  __shared__ double pdd[kPanel + 2], pdo[kPanel + 2];
-  __shared__ int pkd[kPanel + 2];
-  __shared__ double redV[NT / 64 + 1];
-  __shared__ int redI[NT / 64 + 1];
-  __shared__ double fastV[2][NT / 64];
-  __shared__ int fastI[2][NT / 64];
-  __shared__ double blkV[NT / 64][SW];  // per-wave column maxima of a blocked step
+  constexpr int NW = NT / 64;
+  constexpr int SW = kPanelCols;
+  constexpr int CT = TPW > 0 ? TPW : 8;                  // tiles per wave of a chunk
+  constexpr int GT = CT < 4 ? CT : (TPW >= 16 ? 2 : 4);  // tiles whose loads are in flight together
+  constexpr int LR = TPW > 0 ? Shape::kRows : 1;         // rows of the column buffers kept in LDS
+  extern __shared__ double dynLds[];
+  T* const Lp = reinterpret_cast<T*>(dynLds);  // panel column k0 + q, row k0 + i at [q * LD + i]
+  __shared__ double bufK[LR], bufR[LR];        // current columns k and r of a general step, row k0 + i at [i]
+  __shared__ double Wc[kInLds ? 1 : SW][kPanel + 3];  // weights of the panel's earlier pivots at the block's rows
+  __shared__ double Ds[SW][SW + 1];            // diagonal block
+  __shared__ Block16 blk;
+  __shared__ double redM[NW][SW];              // per-wave column maxima
+  __shared__ double redS[NW], redT[NW], redV[NW + 1];
+  __shared__ int redI[NW];
+  // pivot q of the panel, at [q + 1]: (D L^T)(q, row) = pdd l_q + pnx l_(q+1) + ppv l_(q-1)
+  // (the neighbours: the other column of a 2x2 pivot)
+  __shared__ double pdd[kPanel + 3], pnx[kPanel + 3], ppv[kPanel + 3];
 
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lk = lane >> 4;
   if (static_cast<int>(blockIdx.x) >= count) return;
   const int s = list[blockIdx.x];
   double* ws = wsBase + wsOff[s];
@@ -638,7 +880,7 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
   }
   const int m = fd.m[s];
   const int nE = fd.nE[s];
-  T* F = static_cast<T*>(fd.F[s]);
+  const GlobalPtr<T> F = globalView<T>(fd.F[s]);
   const int64_t io = fd.idxOff[s];
   // after a speculative step the panel started p0 pivots before kcur
   const int kc = fd.kcur[s];
@@ -651,498 +893,565 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
   }
   const int nbEnd = min(k0 + kPanel, nE);
   if (kc >= nbEnd) return;
-  for (int q = tid; q < p0; q += NT) {
-    pdd[q] = fd.dDiag[io + k0 + q];
-    pdo[q] = fd.dOff[io + k0 + q];
-    pkd[q] = fd.pkind[io + k0 + q];
+  const bool allRows = panelHoldsAllRows(m, sp);
+  const int rEnd = allRows ? m : nE;  // rows held: [k, rEnd)
+  for (int q = tid; q < p0; q += NT) {  // the speculative step takes 1x1 pivots only
+    pdd[q + 1] = fd.dDiag[io + k0 + q];
+    pnx[q + 1] = 0.0;
+    ppv[q + 1] = 0.0;
   }
-  __syncthreads();
-  double* curK = ws;
-  double* curR = ws + nE;
-  auto Fat = [&](int i, int j) -> T& { return F[i + static_cast<size_t>(j) * m]; };
+  double* wsR = ws + nE;
+  double* cbuf = ws + panelStreamOffset(m, nE, sp);  // streamed rows: current value of row i, block column j at [i + j nE]
+  auto curK = [&](int i) -> double& {
+    if constexpr (TPW > 0)
+      return bufK[i - k0];
+    else
+      return ws[i];
+  };
+  auto curR = [&](int i) -> double& {
+    if constexpr (TPW > 0)
+      return bufR[i - k0];
+    else
+      return wsR[i];
+  };
+  auto at = [&](int i, int j) -> int64_t { return i + static_cast<int64_t>(j) * m; };
+  // entry (i, j), i >= j: panel columns of held rows live in LDS when kInLds
+  auto inLds = [&](int i, int j) { return kInLds && j >= k0 && j < k0 + kPanel && i < rEnd; };
+  auto ldsAt = [&](int i, int j) { return (j - k0) * LD + (i - k0); };
+  auto get = [&](int i, int j) -> T {
+    if constexpr (kInLds)
+      if (inLds(i, j)) return Lp[ldsAt(i, j)];
+    return F[at(i, j)];
+  };
+  auto put = [&](int i, int j, T v) {
+    if constexpr (kInLds)
+      if (inLds(i, j)) {
+        Lp[ldsAt(i, j)] = v;
+        return;
+      }
+    F[at(i, j)] = v;
+  };
+  // panel column q at a held row
+  auto panelEntry = [&](int i, int q) -> T {
+    if constexpr (kInLds)
+      return Lp[q * LD + (i - k0)];
+    else
+      return F[at(i, k0 + q)];
+  };
+  auto sync = [&]() {
+    if constexpr (kInLds)
+      ldsBarrier();
+    else
+      __syncthreads();
+  };
+  if constexpr (kInLds) {
+    // load the panel, eight columns per wave, every load in flight at once
+    const int pw = nbEnd - k0;
+    constexpr int RB = Shape::kRows / 64;
+    T v[RB][kPanel / NW];
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+      for (int u = 0; u < kPanel / NW; ++u) {
+        const int i = k0 + 64 * b + lane, q = wv + NW * u;
+        v[b][u] = F[i < rEnd && q < pw ? at(i, k0 + q) : 0];
+      }
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+      for (int u = 0; u < kPanel / NW; ++u) {
+        const int i = k0 + 64 * b + lane, q = wv + NW * u;
+        if (i < rEnd && q < pw) Lp[q * LD + (i - k0)] = v[b][u];
+      }
+  }
+  sync();
 
   const bool stat = prm.staticMode != 0;
   double origMax = bitsToDouble(fd.origMaxBits[s]);
   if (!stat && origMax < prm.zeroTol) origMax = 1.0;
   if (stat && origMax < prm.staticAbsFloor) origMax = 1.0;
+  const double isolatedFloor = fmax(prm.zeroTol, prm.relFloor * origMax);
   const double runMax0 = fmax(origMax, bitsToDouble(fd.runMaxBits[s]));
   double tmax = 0.0;
   const double delta = prm.staticDelta > 0.0 ? prm.staticDelta : sqrt(DBL_EPSILON) * origMax;
   const double sfloor = fmax(prm.staticAbsFloor, prm.staticRelFloor * origMax);
 
+  // counts of thread 0 (general steps) and of wave 0's lanes (blocks), summed at the end
   int npos = 0, nneg = 0, nzero = 0, npert = 0;
   double pert = 0.0;
   int k = kc, p = p0;
   bool stop = false;
+  bool has2 = false;       // the panel has a 2x2 pivot
+  bool farStores = false;  // kInLds: an interchange has stored to global memory since the last full barrier
 
   // (D L^T)(q, row) for this panel's pivot q and a given row
   auto weight = [&](int q, int row) -> double {
-    const int kind = pkd[q];
-    if (kind == 1) return pdd[q] * static_cast<double>(Fat(row, k0 + q));
-    if (kind == 2) return pdd[q] * static_cast<double>(Fat(row, k0 + q)) + pdo[q] * static_cast<double>(Fat(row, k0 + q + 1));
-    return pdo[q - 1] * static_cast<double>(Fat(row, k0 + q - 1)) + pdd[q] * static_cast<double>(Fat(row, k0 + q));
-  };
-  // weights of this panel's p pivots for one row (general path)
-  auto computeW = [&](int row) {
-    for (int q = tid; q < p; q += NT) wvec[q] = weight(q, row);
-    __syncthreads();
-  };
-  // out[i] = stored column `col` (rows >= k) minus the panel correction
-  auto currentColumn = [&](int col, double* out) {
-    for (int i = k + tid; i < nE; i += NT) {
-      const double raw = (i >= col) ? Fat(i, col) : Fat(col, i);
-      double acc = 0.0;
-      for (int q = 0; q < p; ++q) acc = fma(static_cast<double>(Fat(i, k0 + q)), wvec[q], acc);
-      out[i] = raw - acc;
-    }
-    __syncthreads();
+    const double l = static_cast<double>(panelEntry(row, q));
+    const double n = static_cast<double>(panelEntry(row, min(q + 1, p - 1)));
+    const double v = static_cast<double>(panelEntry(row, max(q - 1, 0)));
+    return pdd[q + 1] * l + (has2 ? pnx[q + 1] * n + ppv[q + 1] * v : 0.0);
   };
   // symmetric interchange of positions a < b in storage (all rows, incl. the
-  // factored part and the not-fully-summed rows) and in the column buffers
+  // factored part and the not-fully-summed rows)
   auto swapSym = [&](int a, int b) {
     for (int t = tid; t < m; t += NT) {
-      if (t < a) {
-        const T x = Fat(a, t);
-        Fat(a, t) = Fat(b, t);
-        Fat(b, t) = x;
-      } else if (t == a) {
-        const T x = Fat(a, a);
-        Fat(a, a) = Fat(b, b);
-        Fat(b, b) = x;
-      } else if (t < b) {
-        const T x = Fat(t, a);
-        Fat(t, a) = Fat(b, t);
-        Fat(b, t) = x;
-      } else if (t > b) {
-        const T x = Fat(t, a);
-        Fat(t, a) = Fat(t, b);
-        Fat(t, b) = x;
+      if (t == b) continue;
+      // (a, t) and (b, t), each read from the lower triangle; (a, a) and (b, b) for t = a
+      const int i1 = max(a, t), j1 = min(a, t);
+      const int i2 = t == a ? b : max(b, t), j2 = t == a ? b : min(b, t);
+      if constexpr (kInLds) {
+        // both values loaded before either is stored, one memory round trip
+        const bool in1 = inLds(i1, j1), in2 = inLds(i2, j2);
+        T x = Lp[in1 ? ldsAt(i1, j1) : 0], y = Lp[in2 ? ldsAt(i2, j2) : 0];
+        if (!in1 || !in2) {
+          const T gx = F[in1 ? 0 : at(i1, j1)], gy = F[in2 ? 0 : at(i2, j2)];
+          x = in1 ? x : gx;
+          y = in2 ? y : gy;
+        }
+        put(i1, j1, y);
+        put(i2, j2, x);
+      } else {
+        const T x = F[at(i1, j1)], y = F[at(i2, j2)];
+        F[at(i1, j1)] = y;
+        F[at(i2, j2)] = x;
       }
     }
     if (tid == 0) {
       const int tp = fd.perm[io + a];
       fd.perm[io + a] = fd.perm[io + b];
       fd.perm[io + b] = tp;
-      double x = curK[a];
-      curK[a] = curK[b];
-      curK[b] = x;
-      x = curR[a];
-      curR[a] = curR[b];
-      curR[b] = x;
     }
-    __syncthreads();
+    farStores = true;
+    sync();
   };
-  auto accept1 = [&](const double* col, double d) {
+  auto setPivot = [&](int q, double d, int kind, double next, double prev) {
+    fd.dDiag[io + k0 + q] = d;
+    fd.dOff[io + k0 + q] = next;
+    fd.pkind[io + k0 + q] = kind;
+    pdd[q + 1] = d;
+    pnx[q + 1] = next;
+    ppv[q + 1] = prev;
+  };
+  // 1x1 pivot d at k with current column col(i)
+  auto accept1 = [&](auto&& col, double d) {
     if (tid == 0) {
-      fd.dDiag[io + k] = d;
-      fd.dOff[io + k] = 0.0;
-      fd.pkind[io + k] = 1;
-      pdd[p] = d;
-      pdo[p] = 0.0;
-      pkd[p] = 1;
-      Fat(k, k) = static_cast<T>(d);
+      setPivot(p, d, 1, 0.0, 0.0);
+      put(k, k, static_cast<T>(d));
+      countInertia(d, npos, nneg, nzero);
     }
-    countInertia(d, npos, nneg, nzero);
     tmax = fmax(tmax, fabs(d));
-    for (int i = k + 1 + tid; i < nE; i += NT) {
-      const double c = col[i];
+    for (int i = k + 1 + tid; i < rEnd; i += NT) {
+      const double c = col(i);
       tmax = fmax(tmax, fabs(c));
-      Fat(i, k) = static_cast<T>(c / d);
+      put(i, k, static_cast<T>(c / d));
     }
-    __syncthreads();
+    sync();
     ++k;
     ++p;
   };
-
-  // Sub-panel [c0, c0 + sw): current values of the eligible rows >= k.
-  int c0 = k, sw = 0;
-  auto loadSub = [&]() {
-    c0 = k;
-    sw = min(SW, nbEnd - k);
-    for (int e = tid; e < sw * p; e += NT) {
-      const int j = e % sw, q = e / sw;
-      Wsub[j][q] = weight(q, c0 + j);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int jj = 0; jj < (RM > 0 ? RM : 1); ++jj) {
-      const int i = k0 + tid + jj * NT;
-      if (i < k || i >= nE) continue;
-      double acc[SW];
-      loadWiden<SW>(acc, static_cast<const T*>(F), [&](int j) -> int64_t {
-        const int col = c0 + j;
-        if (j >= sw) return -1;
-        return i >= col ? i + static_cast<int64_t>(col) * m : col + static_cast<int64_t>(i) * m;
-      });
-      constexpr int U = 8;
-      int q = 0;
-      for (; q + U <= p; q += U) {
-        double lv[U];
-        loadWiden<U>(lv, static_cast<const T*>(F), [&](int u) -> int64_t { return i + static_cast<int64_t>(k0 + q + u) * m; });
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int j = 0; j < SW; ++j) acc[j] = fma(-lv[u], Wsub[j][q + u], acc[j]);
-      }
-      for (; q < p; ++q) {
-        const double l = Fat(i, k0 + q);
-#pragma unroll
-        for (int j = 0; j < SW; ++j) acc[j] = fma(-l, Wsub[j][q], acc[j]);
-      }
-#pragma unroll
-      for (int j = 0; j < SW; ++j)
-        if (j < sw) Cs[j * CSR + (i - k0)] = acc[j];
-    }
-    __syncthreads();
-  };
-
-  int parity = 0;
-  if (RM > 0) loadSub();
-
-  // Blocked first test over the sub-panel's remaining columns [k, c0 + sw):
-  // every thread factors that block (at most SW x SW, from LDS) with 1x1
-  // pivots in order and runs the same recurrence over its own rows,
-  // c_ij = a_ij - sum_{q<j} l_iq d_q l_(k+j)q, so one reduction gives
-  // lambda for every column at once.  The pivots before the first column
-  // whose test fails are kept (the same decisions as pivot by pivot, up to
-  // the order of rounding); that column goes through the single-pivot path
-  // below.  Returns the number of pivots kept.
-  auto blockStep = [&]() -> int {
-    const int kk0 = k - c0, bw = sw - kk0;
-    double Wb[SW][SW], dq[SW], aq[SW];
-    {
-      double B[SW][SW];
-#pragma unroll
-      for (int a = 0; a < SW; ++a)
-#pragma unroll
-        for (int b = 0; b <= a; ++b) B[a][b] = (a < bw) ? Cs[(kk0 + b) * CSR + (k + a - k0)] : 0.0;
-#pragma unroll
-      for (int q = 0; q < SW; ++q) {
-        dq[q] = 1.0;
-        aq[q] = 0.0;
-        if (q < bw) {
-          aq[q] = B[q][q];
-          double d = aq[q];
-          if (stat) {
-            const int sign = prm.expectedSign ? prm.expectedSign[fd.frontIdx[io + k + q]] : 0;
-            double applied;
-            d = staticPivot(d, sign, delta, sfloor, applied);
-          }
-          dq[q] = d;
-          double la[SW];
-#pragma unroll
-          for (int a = q + 1; a < SW; ++a) {
-            la[a] = (a < bw) ? static_cast<double>(static_cast<T>(B[a][q] / d)) : 0.0;
-            Wb[a][q] = d * la[a];
-          }
-#pragma unroll
-          for (int a = q + 1; a < SW; ++a)
-#pragma unroll
-            for (int b = q + 1; b <= a; ++b) B[a][b] = fma(-la[a], Wb[b][q], B[a][b]);
-        }
-      }
-    }
-    // pass 1: column maxima over this thread's rows below each pivot
-    double vmax[SW];
-#pragma unroll
-    for (int j = 0; j < SW; ++j) vmax[j] = 0.0;
-#pragma unroll
-    for (int jj = 0; jj < (RM > 0 ? RM : 1); ++jj) {
-      const int i = k0 + tid + jj * NT;
-      if (i < k || i >= nE) continue;
-      double l[SW];
-#pragma unroll
-      for (int j = 0; j < SW; ++j) {
-        if (j < bw) {
-          double c = Cs[(kk0 + j) * CSR + (i - k0)];
-#pragma unroll
-          for (int q = 0; q < j; ++q) c = fma(-l[q], Wb[j][q], c);
-          if (i > k + j) vmax[j] = fmax(vmax[j], fabs(c));
-          l[j] = static_cast<double>(static_cast<T>(c / dq[j]));
-        }
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < SW; ++j) {
-      const double v = __ockl_wfred_max_f64(vmax[j]);
-      if ((tid & 63) == 0) blkV[tid >> 6][j] = v;
-    }
-    __syncthreads();
-    int qs = bw;
-    {
-      const double isolatedFloor = fmax(prm.zeroTol, prm.relFloor * origMax);
-      for (int j = 0; j < bw; ++j) {
-        double lam = 0.0;
-        for (int w = 0; w < NT / 64; ++w) lam = fmax(lam, blkV[w][j]);
-        const bool ok = stat || ((lam <= prm.zeroTol) ? fabs(aq[j]) > isolatedFloor : fabs(aq[j]) >= kAlpha * lam);
-        if (!ok) {
-          qs = j;
-          break;
-        }
-      }
-    }
-    if (qs == 0) return 0;  // blkV is rewritten only after the next block step's barrier
-    // pass 2: multipliers of the kept columns, current values of the others
-#pragma unroll
-    for (int jj = 0; jj < (RM > 0 ? RM : 1); ++jj) {
-      const int i = k0 + tid + jj * NT;
-      if (i < k || i >= nE) continue;
-      double x[SW], l[SW];
-#pragma unroll
-      for (int j = 0; j < SW; ++j) x[j] = (j < bw) ? Cs[(kk0 + j) * CSR + (i - k0)] : 0.0;
-#pragma unroll
-      for (int j = 0; j < SW; ++j) {
-        if (j < qs) {
-          double c = x[j];
-#pragma unroll
-          for (int q = 0; q < j; ++q) c = fma(-l[q], Wb[j][q], c);
-          l[j] = static_cast<double>(static_cast<T>(c / dq[j]));
-          if (i > k + j) {
-            tmax = fmax(tmax, fabs(c));
-            Fat(i, k + j) = static_cast<T>(l[j]);
-          }
-        } else if (j < bw) {
-          double y = x[j];
-#pragma unroll
-          for (int q = 0; q < SW; ++q)
-            if (q < qs) y = fma(-l[q], Wb[j][q], y);
-          Cs[(kk0 + j) * CSR + (i - k0)] = y;
-        }
-      }
-    }
-    for (int q = 0; q < qs; ++q) {
-      pdd[p + q] = dq[q];
-      pdo[p + q] = 0.0;
-      pkd[p + q] = 1;
-      countInertia(dq[q], npos, nneg, nzero);
-      tmax = fmax(tmax, fabs(dq[q]));
-      if (stat && dq[q] != aq[q]) {
-        pert += fabs(dq[q] - aq[q]);
-        ++npert;
-      }
-    }
-    if (tid == 0)
-      for (int q = 0; q < qs; ++q) {
-        fd.dDiag[io + k + q] = dq[q];
-        fd.dOff[io + k + q] = 0.0;
-        fd.pkind[io + k + q] = 1;
-        Fat(k + q, k + q) = static_cast<T>(dq[q]);
-      }
-    __syncthreads();  // the kept rows' Cs values are read by other threads next
-    return qs;
-  };
-  int skipAt = -1;
-
-  while (k < nbEnd) {
-    if (RM > 0 && SW > 1 && k != skipAt && k - c0 + 1 < sw) {
-      const int kept = blockStep();
-      if (kept == 0) {
-        skipAt = k;
-      } else {
-        k += kept;
-        p += kept;
-        if (k - c0 >= sw && k < nbEnd) {
-          __syncthreads();
-          loadSub();
-        }
-      }
-      continue;
-    }
-    double lv = 0.0;
-    int li = -1;
-    double akk;
-    const int kk = k - c0;
-    if (RM > 0) {
-      const double* col = Cs + kk * CSR;
-#pragma unroll
-      for (int jj = 0; jj < (RM > 0 ? RM : 1); ++jj) {
-        const int i = k0 + tid + jj * NT;
-        if (i > k && i < nE) {
-          const double v = fabs(col[i - k0]);
-          if (v > 0.0) argmaxCombine(lv, li, v, i);
-        }
-      }
-      waveArgmax(lv, li);
-      if ((tid & 63) == 0) {
-        fastV[parity][tid >> 6] = lv;
-        fastI[parity][tid >> 6] = li;
-      }
-      __syncthreads();
-      lv = 0.0;
-      li = -1;
-      for (int w = 0; w < NT / 64; ++w) argmaxCombine(lv, li, fastV[parity][w], fastI[parity][w]);
-      parity ^= 1;
-      akk = col[k - k0];
-    } else {
-      computeW(k);
-      currentColumn(k, curK);
-      if (!stat) {
-        for (int i = k + 1 + tid; i < nE; i += NT) {
-          const double v = fabs(curK[i]);
-          if (v > 0.0) argmaxCombine(lv, li, v, i);
-        }
-        blockArgmax<NT>(lv, li, redV, redI);
-      }
-      akk = curK[k];
-    }
-
-    // first Bunch-Kaufman tests (dense_kernel.hpp:601-618); static pivots
-    // are always accepted at k (dense_kernel.hpp:982-1011)
-    int action = -1;  // -1: sigma test needed
-    double dpiv = akk;
-    if (stat) {
-      const int sign = prm.expectedSign ? prm.expectedSign[fd.frontIdx[io + k]] : 0;
-      double applied;
-      dpiv = staticPivot(akk, sign, delta, sfloor, applied);
-      if (applied != 0.0) {
-        pert += fabs(applied);
-        ++npert;
-      }
-      action = 1;
-    } else if (lv <= prm.zeroTol) {
-      const double isolatedFloor = fmax(prm.zeroTol, prm.relFloor * origMax);
-      action = (fabs(akk) <= isolatedFloor) ? 0 : 1;
-    } else if (fabs(akk) >= kAlpha * lv) {
-      action = 1;
-    }
-    if (action == 0) {
+  // one general step at pivot k (sigma test, swaps, 1x1 or 2x2, or a stop);
+  // curK holds the current column k, lam = max |curK| over the eligible rows
+  // below k (attained)
+  auto generalStep = [&](double lam) {
+    const double akk = curK(k);
+    if (lam <= prm.zeroTol) {  // dense_kernel.hpp:601-616: the block test failed on the isolated-pivot floor
       stop = true;
-      break;
+      return;
     }
-    if (action == 1 && RM > 0) {
-      const double d = dpiv;
-      const double* col = Cs + kk * CSR;
-      // (D L^T)(k, c0 + j) for the sub-panel columns right of k, as the
-      // general path would form it from the stored multiplier
-      double wj[SW];
-#pragma unroll
-      for (int j = 0; j < SW; ++j)
-        wj[j] = (j > kk && j < sw) ? d * static_cast<double>(static_cast<T>(col[c0 + j - k0] / d)) : 0.0;
-      pdd[p] = d;  // every thread stores the same value
-      pdo[p] = 0.0;
-      pkd[p] = 1;
-      if (tid == 0) {
-        fd.dDiag[io + k] = d;
-        fd.dOff[io + k] = 0.0;
-        fd.pkind[io + k] = 1;
-        Fat(k, k) = static_cast<T>(d);
-      }
-      countInertia(d, npos, nneg, nzero);
-      tmax = fmax(tmax, fabs(d));
-#pragma unroll
-      for (int jj = 0; jj < (RM > 0 ? RM : 1); ++jj) {
-        const int i = k0 + tid + jj * NT;
-        if (i > k && i < nE) {
-          const double c = col[i - k0];
-          tmax = fmax(tmax, fabs(c));
-          const T lt = static_cast<T>(c / d);
-          Fat(i, k) = lt;
-          const double l = lt;
-#pragma unroll
-          for (int j = 0; j < SW; ++j)
-            if (j > kk && j < sw) Cs[j * CSR + (i - k0)] = fma(-l, wj[j], Cs[j * CSR + (i - k0)]);
-        }
-      }
-      // No barrier here: a thread updated only its own rows, and the values
-      // the next step reads from other threads' rows (a_kk, the sub-panel
-      // rows of the pivot column) are read after the next reduction's
-      // barrier.  A reload reads the multipliers just stored: it waits.
-      ++k;
-      ++p;
-      if (k - c0 >= sw && k < nbEnd) {
-        __syncthreads();
-        loadSub();
-      }
-      continue;
+    if (kInLds && farStores) {
+      __syncthreads();  // column r may have been stored by another thread's interchange
+      farStores = false;
     }
-    if (RM > 0) {
-      // the general path below works on the column buffers
-      const double* col = Cs + kk * CSR;
-      for (int i = k + tid; i < nE; i += NT) curK[i] = col[i - k0];
+    // r: the first row that attains lambda (found by every wave for itself
+    // where the column is in LDS)
+    int li = INT_MAX;
+    for (int i = k + 1 + (TPW > 0 ? lane : tid); i < nE; i += (TPW > 0 ? 64 : NT))
+      if (fabs(curK(i)) == lam) {
+        li = i;
+        break;
+      }
+    int r = __ockl_wfred_min_i32(li);
+    if constexpr (TPW == 0) {
+      if (lane == 0) redI[wv] = r;
       __syncthreads();
+      r = redI[0];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) r = min(r, redI[w]);
     }
-    if (action == 1) {
-      accept1(curK, dpiv);
-      if (RM > 0 && k < nbEnd) loadSub();
-      continue;
+    r = __builtin_amdgcn_readfirstlane(r);
+    if (r >= nE) {  // lambda is not a number: nothing to pivot on
+      stop = true;
+      return;
     }
-    const int r = li;
-    computeW(r);
-    currentColumn(r, curR);
-    // the reference mirrors column r into row r, so column k's entry at
-    // row r becomes column r's value at row k (dense_kernel.hpp:543)
-    if (tid == 0) curK[r] = curR[k];
-    __syncthreads();
+    // curR = current column r; sigma = its max over the eligible rows but r
+    // (dense_kernel.hpp:628-633); lane q keeps the weight of pivot q
+    const double wq = lane < p ? weight(lane, r) : 0.0;
     double sg = 0.0;
-    for (int i = k + tid; i < nE; i += NT)
-      if (i != r) sg = fmax(sg, fabs(curR[i]));
-    sg = blockMax<NT>(sg, redV);
-    if (fabs(akk) * sg >= kAlpha * lv * lv)
-      action = 1;
-    else if (fabs(curR[r]) >= kAlpha * sg)
-      action = 2;
-    else
-      action = 3;
-    if (action == 1) {
-      accept1(curK, curK[k]);
-      if (RM > 0 && k < nbEnd) loadSub();
-      continue;
+    for (int i0 = k + 64 * wv; i0 < rEnd; i0 += NT) {  // whole waves: the DPP operands come from every lane
+      const bool ok = i0 + lane < rEnd;
+      const int i = ok ? i0 + lane : rEnd - 1;
+      const double raw = static_cast<double>(i >= r ? get(i, r) : get(r, i));
+      double a0 = 0.0, a1 = 0.0;
+#pragma unroll 1
+      for (int q = 0; q < p; q += 16) {
+        const double w16 = __shfl(wq, q + lr, 64);  // the weights past p are zero
+        double lv[16];
+        if constexpr (kInLds) {
+#pragma unroll
+          for (int u = 0; u < 16; ++u) lv[u] = static_cast<double>(Lp[min(q + u, p - 1) * LD + (i - k0)]);
+        } else {
+          loadWiden<16>(lv, F, [&](int u) -> int64_t { return at(i, k0 + min(q + u, p - 1)); });
+        }
+        unrolled(std::make_integer_sequence<int, 8>{}, [&](auto uu) {
+          constexpr int u = 2 * decltype(uu)::value;
+          fmaBcast16<u>(a0, w16, lv[u]);
+          fmaBcast16<u + 1>(a1, w16, lv[u + 1]);
+        });
+      }
+      const double c = raw - (a0 + a1);
+      if (ok) curR(i) = c;
+      if (ok && i < nE && i != r) sg = fmax(sg, fabs(c));
     }
-    if (action == 2) {
+    sg = __ockl_wfred_max_f64(sg);
+    const double tm = __ockl_wfred_max_f64(tmax);
+    if (lane == 0) {
+      redS[wv] = sg;
+      redT[wv] = tm;
+    }
+    sync();
+    double rmax = runMax0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      sg = fmax(sg, redS[w]);
+      rmax = fmax(rmax, redT[w]);
+    }
+    const double crk = curR(k), crr = curR(r);
+    // the reference mirrors column r into row r, so column k's entry at row r
+    // is column r's value at row k (dense_kernel.hpp:543)
+    if (fabs(akk) * sg >= kAlpha * lam * lam) {
+      accept1([&](int i) { return i == r ? crk : curK(i); }, akk);
+      return;
+    }
+    if (fabs(crr) >= kAlpha * sg) {
+      // 1x1 at r after the interchange with k
       swapSym(k, r);
-      accept1(curR, curR[k]);
-      if (RM > 0 && k < nbEnd) loadSub();
-      continue;
+      accept1([&](int i) { return i == r ? crk : curR(i); }, crr);
+      return;
     }
-    // 2x2 at (k, r): bring r to k+1
-    if (r != k + 1) swapSym(k + 1, r);
-    const double d11 = curK[k];
-    const double d21 = curK[k + 1];
-    const double d22 = curR[k + 1];
+    // 2x2 at (k, r): r comes to k + 1
+    const double d11 = akk, d21 = crk, d22 = crr;
     const double det = d11 * d22 - d21 * d21;
-    const double rmax = fmax(runMax0, blockMax<NT>(tmax, redV));
+    const double ck1 = curK(k + 1), cr1 = curR(k + 1);
+    if (r != k + 1) swapSym(k + 1, r);
     if (fabs(det) <= prm.zeroTol * fmax(1.0, rmax) * fmax(1.0, rmax)) {
       stop = true;
-      break;
+      return;
     }
     tmax = fmax(tmax, fmax(fabs(d11), fmax(fabs(d21), fabs(d22))));
     if (tid == 0) {
-      fd.dDiag[io + k] = d11;
-      fd.dOff[io + k] = d21;
-      fd.dDiag[io + k + 1] = d22;
-      fd.dOff[io + k + 1] = 0.0;
-      fd.pkind[io + k] = 2;
-      fd.pkind[io + k + 1] = 0;
-      pdd[p] = d11;
-      pdo[p] = d21;
-      pkd[p] = 2;
-      pdd[p + 1] = d22;
-      pdo[p + 1] = 0.0;
-      pkd[p + 1] = 0;
-      Fat(k, k) = static_cast<T>(d11);
-      Fat(k + 1, k) = static_cast<T>(d21);
-      Fat(k + 1, k + 1) = static_cast<T>(d22);
+      setPivot(p, d11, 2, d21, 0.0);
+      setPivot(p + 1, d22, 0, 0.0, d21);
+      put(k, k, static_cast<T>(d11));
+      put(k + 1, k, static_cast<T>(d21));
+      put(k + 1, k + 1, static_cast<T>(d22));
+      countInertia2(d11, d22, det, npos, nneg);
     }
-    countInertia2(d11, d22, det, npos, nneg);
     const double inv11 = d22 / det, inv21 = -d21 / det, inv22 = d11 / det;
-    for (int i = k + 2 + tid; i < nE; i += NT) {
-      const double a0 = curK[i], a1 = curR[i];
+    for (int i = k + 2 + tid; i < rEnd; i += NT) {
+      // row r holds what was row k + 1
+      const double a0 = i == r ? ck1 : curK(i), a1 = i == r ? cr1 : curR(i);
       tmax = fmax(tmax, fmax(fabs(a0), fabs(a1)));
-      Fat(i, k) = static_cast<T>(a0 * inv11 + a1 * inv21);
-      Fat(i, k + 1) = static_cast<T>(a0 * inv21 + a1 * inv22);
+      put(i, k, static_cast<T>(a0 * inv11 + a1 * inv21));
+      put(i, k + 1, static_cast<T>(a0 * inv21 + a1 * inv22));
     }
-    __syncthreads();
+    sync();
+    has2 = true;
     k += 2;
     p += 2;
-    if (RM > 0 && k < nbEnd) loadSub();
-  }
-  __syncthreads();
+  };
 
+  // First row of tile t of this wave in chunk ch: tiles go to the waves in
+  // turn, so all of them keep rows as the panel moves down.
+  auto rowOf = [&](int ch, int t) { return k0 + 16 * ((ch * CT + t) * NW + wv); };
+  // Current values of the block's columns c0 .. c0 + sw - 1 at NTL tiles (16
+  // rows from row0(t)): stored values at and below the diagonal less the
+  // correction of the panel's p pivots; zero above the diagonal and past rEnd.
+  auto loadTiles = [&](auto& x, auto ntl, auto&& row0, int c0, int sw) {
+    constexpr int NTL = decltype(ntl)::value;
+    // panel column q, row `row` (any valid entry when !ok)
+    auto entry = [&](int row, int q, bool ok) -> T {
+      if constexpr (kInLds)
+        return Lp[ok ? q * LD + (row - k0) : 0];
+      else
+        return F[ok ? at(row, k0 + q) : 0];
+    };
+    T raw[NTL][4];
+#pragma unroll
+    for (int t = 0; t < NTL; ++t)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int row = row0(t) + lr, col = 4 * u + lk;
+        raw[t][u] = entry(row, c0 - k0 + col, row < rEnd && col < sw && row >= c0 + col);
+      }
+#pragma unroll
+    for (int t = 0; t < NTL; ++t)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int row = row0(t) + lr, col = 4 * u + lk;
+        x[t][u] = row < rEnd && col < sw && row >= c0 + col ? static_cast<double>(raw[t][u]) : 0.0;
+      }
+    // operands of 16 pivots
+    T lv[NTL][4], ln[NTL][4];
+    double w[4], wn[4];
+    auto fetch = [&](int q0, T (&l)[NTL][4], double (&wt)[4]) {
+#pragma unroll
+      for (int t = 0; t < NTL; ++t)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int row = row0(t) + lr, q = q0 + 4 * u + lk;
+          l[t][u] = entry(row, q, row >= c0 && row < rEnd && q < p);
+        }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int q = q0 + 4 * u + lk;
+        if constexpr (kInLds) {
+          // (columns past sw take weights that nothing uses)
+          const int qc = min(q, p - 1), i = min(c0 + lr, rEnd - 1);
+          wt[u] = -weight(qc, i);
+        } else {
+          wt[u] = -Wc[lr][q];
+        }
+      }
+    };
+    auto products = [&](int q0) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int t = 0; t < NTL; ++t) {
+          const int row = row0(t) + lr, q = q0 + 4 * u + lk;
+          const double l = row >= c0 && row < rEnd && q < p ? static_cast<double>(lv[t][u]) : 0.0;
+          x[t] = mfma64(w[u], l, x[t]);
+        }
+    };
+    if constexpr (TPW == 1 || TPW == 2) {  // (with more tiles the registers are worth more)
+      if (p > 0) fetch(0, ln, wn);
+      for (int q0 = 0; q0 < p; q0 += 16) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          w[u] = wn[u];
+#pragma unroll
+          for (int t = 0; t < NTL; ++t) lv[t][u] = ln[t][u];
+        }
+        if (q0 + 16 < p) fetch(q0 + 16, ln, wn);
+        products(q0);
+      }
+    } else {
+      for (int q0 = 0; q0 < p; q0 += 16) {
+        fetch(q0, lv, w);
+        products(q0);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NTL; ++t) settle(x[t]);
+  };
+
+  while (k < nbEnd && !stop) {
+    const int c0 = k, sw = min(SW, nbEnd - k);
+    if constexpr (!kInLds) {
+      // weights of the earlier pivots at the block's rows
+      for (int e = tid; e < SW * ((p + 15) & ~15); e += NT) {
+        const int j = e & (SW - 1), q = e / SW;
+        Wc[j][q] = (j < sw && q < p) ? weight(q, c0 + j) : 0.0;
+      }
+      sync();
+    }
+    v4d x[CT];
+    // chunk ch of this wave's tiles; a group of tiles past the held rows or
+    // above the block is skipped whole (zero)
+    auto loadChunk = [&](int ch) {
+#pragma unroll
+      for (int t0 = 0; t0 < CT; t0 += GT) {
+        if (rowOf(ch, t0) < rEnd && rowOf(ch, t0 + GT - 1) + 16 > c0) {
+          v4d xt[GT];
+          loadTiles(xt, std::integral_constant<int, GT>{}, [&](int t) { return rowOf(ch, t0 + t); }, c0, sw);
+#pragma unroll
+          for (int t = 0; t < GT; ++t) x[t0 + t] = xt[t];
+        } else {
+#pragma unroll
+          for (int t = 0; t < GT; ++t) x[t0 + t] = v4d{0.0, 0.0, 0.0, 0.0};
+        }
+      }
+    };
+    if constexpr (TPW > 0) {
+      loadChunk(0);
+#pragma unroll
+      for (int t = 0; t < CT; ++t) {
+        const int i = rowOf(0, t) + lr - c0;
+        if (i >= 0 && i < SW) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) Ds[i][4 * u + lk] = x[t][u];
+        }
+      }
+    } else if (wv == 0) {
+      v4d xd[1];
+      loadTiles(xd, std::integral_constant<int, 1>{}, [&](int) { return c0; }, c0, sw);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) Ds[lr][4 * u + lk] = xd[0][u];
+    }
+    sync();
+    if (wv == 0) {
+      double a[16];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) a[q] = Ds[lr][q];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) a[q] = lr < sw ? (q <= lr ? a[q] : 0.0) : (q == lr ? 1.0 : 0.0);
+      if (!stat) {
+        blockFactor16<T>(a, blk, [](int, double v) { return v; });
+      } else {
+        const int sgn = prm.expectedSign && lr < sw ? prm.expectedSign[fd.frontIdx[io + c0 + lr]] : 0;
+        blockFactor16<T>(a, blk, [&](int q, double v) {
+          double applied;
+          return staticPivot(v, __shfl(sgn, q, 64), delta, sfloor, applied);
+        });
+      }
+    }
+    sync();
+    double op[4], rdc[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      op[u] = blk.op[u][lane];
+      rdc[u] = blk.rd[4 * u + lk];
+    }
+    const double akk = blk.akk[lr];
+    // substitution of the held rows and the maxima over the eligible rows below each pivot
+    double vm[4] = {0.0, 0.0, 0.0, 0.0};
+    auto solveChunk = [&](int ch) {
+#pragma unroll
+      for (int t = 0; t < CT; ++t) {
+        const int row0 = rowOf(ch, t);
+        if (row0 < rEnd && row0 + 16 > c0) {
+          substTile(x[t], op);
+          const int row = row0 + lr;
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            vm[u] = fmax(vm[u], row < nE && row > c0 + 4 * u + lk ? fabs(x[t][u]) : 0.0);
+        }
+      }
+    };
+    const int nch = TPW > 0 ? 1 : (rEnd - k0 + 16 * NW * CT - 1) / (16 * NW * CT);
+    if constexpr (TPW > 0) {
+      solveChunk(0);
+    } else {
+      for (int ch = 0; ch < nch; ++ch) {
+        loadChunk(ch);
+        solveChunk(ch);
+#pragma unroll
+        for (int t = 0; t < CT; ++t) {
+          const int row = rowOf(ch, t) + lr;
+          if (row >= c0 && row < rEnd) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) cbuf[row + static_cast<int64_t>(4 * u + lk) * nE] = x[t][u];
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const double v = max16(vm[u]);
+      if (lr == 0) redM[wv][4 * u + lk] = v;
+    }
+    sync();
+    // first failing column (dense_kernel.hpp:601-618); static pivots are
+    // always accepted (dense_kernel.hpp:982-1011)
+    double lam = redM[0][lr];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) lam = fmax(lam, redM[w][lr]);
+    const bool pass = stat || ((lam <= prm.zeroTol) ? fabs(akk) > isolatedFloor : fabs(akk) >= kAlpha * lam);
+    const unsigned long long bad = __ballot(lane < sw && !pass);
+    const int qs = bad ? __ffsll(static_cast<long long>(bad)) - 1 : sw;
+    // keep the columns before it: multipliers, pivots, counts
+    auto acceptChunk = [&](int ch) {
+#pragma unroll
+      for (int t = 0; t < CT; ++t) {
+        const int row = rowOf(ch, t) + lr;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int q = 4 * u + lk;
+          if (q < qs && row > c0 + q && row < rEnd) {
+            tmax = fmax(tmax, fabs(x[t][u]));
+            const T l = static_cast<T>(x[t][u] * rdc[u]);
+            if constexpr (kInLds)
+              Lp[(c0 - k0 + q) * LD + (row - k0)] = l;
+            else
+              F[at(row, c0 + q)] = l;
+          }
+          // the failing column's current values for the general step
+          if (q == qs && row >= c0 + q && row < rEnd) curK(row) = x[t][u];
+        }
+      }
+    };
+    if constexpr (TPW > 0) {
+      acceptChunk(0);
+    } else {
+      for (int ch = 0; ch < nch; ++ch) {
+#pragma unroll
+        for (int t = 0; t < CT; ++t) {
+          const int row = rowOf(ch, t) + lr;
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            x[t][u] = (row >= c0 && row < rEnd) ? cbuf[row + static_cast<int64_t>(4 * u + lk) * nE] : 0.0;
+        }
+        acceptChunk(ch);
+      }
+    }
+    if (tid < qs) {
+      const int q = tid;
+      const double dpv = blk.d[q];
+      setPivot(p + q, dpv, 1, 0.0, 0.0);
+      put(k + q, k + q, static_cast<T>(dpv));
+      countInertia(dpv, npos, nneg, nzero);
+      tmax = fmax(tmax, fabs(dpv));
+      if (stat && dpv != akk) {
+        pert += fabs(dpv - akk);
+        ++npert;
+      }
+    }
+    const double lamF = readLane(lam, min(qs, SW - 1));
+    sync();
+    k += qs;
+    p += qs;
+    if (qs < sw) generalStep(lamF);
+  }
+
+  if constexpr (kInLds) {
+    ldsBarrier();
+    // write the panel back: accepted columns, and the others as the interchanges left them
+    const int pw = nbEnd - k0;
+    for (int i0 = k0; i0 < rEnd; i0 += 64) {
+      const int i = i0 + lane;
+#pragma unroll
+      for (int u = 0; u < kPanel / NW; ++u) {
+        const int q = wv + NW * u;
+        if (q < pw && i >= k0 + q && i < rEnd) F[at(i, k0 + q)] = Lp[q * LD + (i - k0)];
+      }
+    }
+  }
   const double bm = blockMax<NT>(tmax, redV);
+  if (tid < 64) {
+    for (int off = 8; off > 0; off >>= 1) {  // lanes 0 .. 15 counted
+      npos += __shfl_xor(npos, off, 64);
+      nneg += __shfl_xor(nneg, off, 64);
+      nzero += __shfl_xor(nzero, off, 64);
+      npert += __shfl_xor(npert, off, 64);
+      pert += __shfl_xor(pert, off, 64);
+    }
+  }
   if (tid == 0) {
     fd.kcur[s] = k;
+    fd.nF[s] = k;
     fd.pcount[s] = p;
     fd.stopped[s] = stop ? 1 : 0;
+    if (allRows) fd.cbDone[s] = 1;
     fd.inertia[3 * s] += npos;
     fd.inertia[3 * s + 1] += nneg;
     fd.inertia[3 * s + 2] += nzero;
@@ -1638,6 +1947,7 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel_mw(const int* list, int
   if (tid == 0) atomicMaxNonNeg(fd.runMaxBits + s, fmax(bm, origMax));
   if (lead && tid == 0) {
     fd.kcur[s] = k;
+    fd.nF[s] = k;
     fd.pcount[s] = p;
     fd.stopped[s] = stop ? 1 : 0;
     fd.inertia[3 * s] += npos;
@@ -1664,36 +1974,6 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel_mw(const int* list, int
 // rest (still holding current values) to the exact panel kernel, which
 // continues from there.
 // ---------------------------------------------------------------------------
-// Row values loaded in their storage type, every load issued before any is
-// used: each load is unconditional (a skipped element reads the front's first
-// entry, a valid address, and is zeroed afterwards), since a load under a
-// branch completes before the branch joins.
-template <int N, typename T, typename Off>
-__device__ inline void loadWiden(double (&x)[N], const T* base, Off off) {
-  T raw[N];
-  bool ok[N];
-#pragma unroll
-  for (int q = 0; q < N; ++q) {
-    const int64_t o = off(q);
-    ok[q] = o >= 0;
-    raw[q] = base[ok[q] ? o : 0];
-  }
-#pragma unroll
-  for (int q = 0; q < N; ++q) x[q] = ok[q] ? static_cast<double>(raw[q]) : 0.0;
-}
-
-// 1 / d for a pivot on a dependent chain: the hardware reciprocal refined by
-// two Newton steps (within an ulp of the quotient), an IEEE division for
-// zero, denormal and non-finite d.
-__device__ inline double pivotRecip(double d) {
-  const double a = fabs(d);
-  if (!(a >= DBL_MIN && a <= DBL_MAX)) return 1.0 / d;
-  double r = __builtin_amdgcn_rcp(d);
-  r = fma(fma(-d, r, 1.0), r, r);
-  r = fma(fma(-d, r, 1.0), r, r);
-  return r;
-}
-
 struct SpecRec {
   unsigned long long* colmax;  // [2][kPanel]
   unsigned long long* emax;
@@ -2141,6 +2421,7 @@ __global__ __launch_bounds__(kSpecRows) void k_spec_apply(const int* list, int c
       fd.pert[s] += pert;
       fd.npert[s] += npert;
       fd.kcur[s] = k0 + qs;
+      fd.nF[s] = k0 + qs;
       fd.pcount[s] = qs;
       fd.cbDone[s] = (qs == pw) ? 1 : 0;
       atomicMaxNonNeg(fd.runMaxBits + s, fmax(tmax, origMax));
@@ -2160,134 +2441,199 @@ __global__ void k_spec_reset(const int* list, int count, DevFronts fd, double* w
 
 // Multipliers of the rows that are not fully summed ([nE, m)) for the last
 // panel.  With U = D L^T of the panel, the multipliers of a row are
-// f U^{-1} = (f L^{-T}) D^{-1}: every workgroup forms M = L^{-1} of the
-// panel's unit lower block in LDS (one column per thread, no barriers), then
-// each thread maps one row: y = f M^T in registers, the running-max check on
-// y, and l = y D^{-1} for the 1x1 and 2x2 pivot blocks (dense_kernel.hpp:
-// 772-787 applied to the whole panel at once).
+// f U^{-1} = (f L^{-T}) D^{-1} (dense_kernel.hpp:772-787 applied to the whole
+// panel at once).  y = f L^{-T} is a substitution over the panel's columns in
+// groups of four: the operators [M_g - I; -L M_g] (M_g the inverse of group
+// g's 4 x 4 unit lower block) are formed in LDS once per workgroup, then every
+// wave takes 16 rows as 16 columns of the FP64 MFMA (layout above k_panel),
+// group after group, the solved group feeding the products of the later
+// columns from its own registers.  l = y D^{-1} follows for the 1x1 and 2x2
+// pivot blocks.  64 rows per workgroup: a front's rows spread over as many
+// CUs as they can; what is left is the latency of the panel block's loads
+// and of 16 dependent MFMA steps.
 template <typename T>
 __global__ __launch_bounds__(256) void k_panel_rows(const int* list, int count, const int* blockStart,
                                                      DevFronts fd) {
   constexpr int P = kPanel + 1;  // a 2x2 pivot at the panel's last column makes it 65
-  __shared__ double Lp[P][P + 1];
-  __shared__ double Mi[P][P + 1];
-  __shared__ double Tt[P - 32][33];  // L21 M11 of the blocked inverse
-  __shared__ double pdd[kPanel + 2], pdo[kPanel + 2];
-  __shared__ int pkd[kPanel + 2];
+  constexpr int G = (P + 3) / 4, PP = 4 * G;
+  constexpr int NB = (PP + 15) / 16;
+  __shared__ double Pm[16 * NB][PP + 1];  // the panel's unit lower block, then the operators
+  __shared__ double Mg[G][16];       // M_g, row-major
+  __shared__ double cSelf[PP], cNext[PP], cPrev[PP];  // l_q = y_q cSelf + y_{q+1} cNext + y_{q-1} cPrev
+  __shared__ int pkd[PP];
+  __shared__ int any2;
   if (static_cast<int>(blockIdx.x) >= blockStart[count]) return;
   const int f = findSegment(blockStart, count, blockIdx.x);
   const int s = list[f];
-  const int rowBlock = blockIdx.x - blockStart[f];
   const int p = fd.pcount[s];
-  if (p == 0 || fd.cbDone[s]) return;  // the speculative step already wrote these rows
+  if (p == 0 || fd.cbDone[s]) return;  // the panel already wrote these rows
   const int m = fd.m[s];
   const int nE = fd.nE[s];
   const int k1 = fd.kcur[s];
   const int k0 = k1 - p;
-  T* F = static_cast<T*>(fd.F[s]);
+  const GlobalPtr<T> F = globalView<T>(fd.F[s]);
   const int64_t io = fd.idxOff[s];
-  auto Fat = [&](int i, int j) -> T& { return F[i + static_cast<size_t>(j) * m]; };
-  for (int q = threadIdx.x; q < p; q += blockDim.x) {
-    pdd[q] = fd.dDiag[io + k0 + q];
-    pdo[q] = fd.dOff[io + k0 + q];
-    pkd[q] = fd.pkind[io + k0 + q];
-  }
-  __syncthreads();
-  // unit lower L of the panel; the (s+1, s) slot of a 2x2 block holds d21
-  for (int t = threadIdx.x; t < p * p; t += blockDim.x) {
-    const int r = t % p, c = t / p;
-    double v = 0.0;
-    if (r > c && !(r == c + 1 && pkd[c] == 2)) v = Fat(k0 + r, k0 + c);
-    Lp[r][c] = v;
-  }
-  __syncthreads();
-  // M = L^{-1} by 2 x 2 blocks (the first H columns and the rest): both
-  // diagonal blocks are inverted at once, column by column (column c:
-  // M[c][c] = 1, M[r][c] = -sum_{c <= t < r} L[r][t] M[t][c]) by threads 0.. and
-  // 64.. (two waves), then M21 = -M22 (L21 M11).
-  constexpr int H = 32;
-  const int h = min(H, p), nb = p - h;
-  auto invCol = [&](int base, int nrow, int c) {
-    Mi[base + c][base + c] = 1.0;
-    for (int r = c + 1; r < nrow; ++r) {
-      double a0 = Lp[base + r][base + c], a1 = 0.0, a2 = 0.0, a3 = 0.0;
-      int t = c + 1;
-      for (; t + 4 <= r; t += 4) {
-        a0 = fma(Lp[base + r][base + t], Mi[base + t][base + c], a0);
-        a1 = fma(Lp[base + r][base + t + 1], Mi[base + t + 1][base + c], a1);
-        a2 = fma(Lp[base + r][base + t + 2], Mi[base + t + 2][base + c], a2);
-        a3 = fma(Lp[base + r][base + t + 3], Mi[base + t + 3][base + c], a3);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int lr = lane & 15, lk = lane >> 4;
+  auto at = [&](int i, int j) -> int64_t { return i + static_cast<int64_t>(j) * m; };
+  // this wave's rows: column 16 b + 4 u + lk of the panel in register u of
+  // block b, all loads in flight together with the panel block's below
+  const int row = nE + (static_cast<int>(blockIdx.x) - blockStart[f]) * kPanelRowsWg + 16 * wv + lr;
+  T raw[NB][4];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int q = 16 * b + 4 * u + lk;
+      raw[b][u] = F[row < m && q < p ? at(row, k0 + q) : 0];
+    }
+  {
+    // panel block: row `lane`, columns wv, wv + 4, ...; row 64 by the last loads
+    T blk[kPanel / 4];
+#pragma unroll
+    for (int u = 0; u < kPanel / 4; ++u) {
+      const int c = wv + 4 * u;
+      blk[u] = F[lane < p && c < lane ? at(k0 + lane, k0 + c) : 0];
+    }
+    const T last = F[p > kPanel && tid < kPanel ? at(k0 + kPanel, k0 + tid) : 0];
+    if (tid == 0) any2 = 0;
+    for (int q = tid; q < PP; q += 256) pkd[q] = q < p ? fd.pkind[io + k0 + q] : 1;
+    __syncthreads();
+    for (int q = tid; q < PP; q += 256) {
+      double cs = 1.0, cn = 0.0, cp = 0.0;
+      if (q < p) {
+        const double d = fd.dDiag[io + k0 + q];
+        if (pkd[q] == 1) {
+          cs = 1.0 / d;
+        } else {
+          const int h = pkd[q] == 2 ? q : q - 1;  // first column of the 2x2 block
+          const double d11 = fd.dDiag[io + k0 + h], d21 = fd.dOff[io + k0 + h], d22 = fd.dDiag[io + k0 + h + 1];
+          const double det = d11 * d22 - d21 * d21;
+          cs = (h == q ? d22 : d11) / det;
+          (h == q ? cn : cp) = -d21 / det;
+          any2 = 1;
+        }
       }
-      for (; t < r; ++t) a0 = fma(Lp[base + r][base + t], Mi[base + t][base + c], a0);
-      Mi[base + r][base + c] = -((a0 + a1) + (a2 + a3));
+      cSelf[q] = cs;
+      cNext[q] = cn;
+      cPrev[q] = cp;
+    }
+    // unit lower L of the panel; the (q+1, q) slot of a 2x2 block holds d21
+#pragma unroll
+    for (int u = 0; u < kPanel / 4; ++u) {
+      const int c = wv + 4 * u;
+      Pm[lane][c] = (lane < p && c < lane && !(lane == c + 1 && pkd[c] == 2)) ? static_cast<double>(blk[u]) : 0.0;
+    }
+    if (tid < kPanel) {
+      Pm[kPanel][tid] = (p > kPanel && !(tid == kPanel - 1 && pkd[tid] == 2)) ? static_cast<double>(last) : 0.0;
+      for (int r = kPanel + 1; r < 16 * NB; ++r) Pm[r][tid] = 0.0;
+    }
+    if (tid < 16 * NB)
+      for (int c = kPanel; c < PP; ++c) Pm[tid][c] = 0.0;
+  }
+  __syncthreads();
+  if (tid < G) {
+    const int g = 4 * tid;
+    const Inv4 v = invUnit4(Pm[g + 1][g], Pm[g + 2][g], Pm[g + 2][g + 1], Pm[g + 3][g], Pm[g + 3][g + 1],
+                            Pm[g + 3][g + 2]);
+    const double mm[16] = {1, 0, 0, 0, v.m10, 1, 0, 0, v.m20, v.m21, 1, 0, v.m30, v.m31, v.m32, 1};
+#pragma unroll
+    for (int e = 0; e < 16; ++e) Mg[tid][e] = mm[e];
+  }
+  __syncthreads();
+  for (int e = tid; e < PP * G; e += 256) {
+    const int i = e % PP, g = e / PP, r = i - 4 * g;
+    double o[4];
+    if (r < 0) continue;  // above the group: zero, and not read
+    if (r < 4) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[k] = k < r ? Mg[g][4 * r + k] : 0.0;
+    } else {
+      const double l0 = Pm[i][4 * g], l1 = Pm[i][4 * g + 1], l2 = Pm[i][4 * g + 2], l3 = Pm[i][4 * g + 3];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[k] = -(l0 * Mg[g][k] + l1 * Mg[g][4 + k] + l2 * Mg[g][8 + k] + l3 * Mg[g][12 + k]);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) Pm[i][4 * g + k] = o[k];
+  }
+  __syncthreads();
+  v4d x[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      x[b][u] = (row < m && 16 * b + 4 * u + lk < p) ? static_cast<double>(raw[b][u]) : 0.0;
+  // group S of block B within the panel's first nb blocks
+  auto group = [&](auto nb, auto bb, auto ss) {
+    constexpr int N = decltype(nb)::value, B = decltype(bb)::value, S = decltype(ss)::value;
+    if constexpr (B < N && 16 * B + 4 * S < PP) {
+      const double y = x[B][S];
+      substStep<S>(x[B], Pm[16 * B + lr][16 * B + 4 * S + lk]);
+#pragma unroll
+      for (int rb = B + 1; rb < N; ++rb) x[rb] = mfma64(Pm[16 * rb + lr][16 * B + 4 * S + lk], y, x[rb]);
     }
   };
-  const int tid = threadIdx.x;
-  if (tid < h)
-    invCol(0, h, tid);
-  else if (tid >= 64 && tid < 64 + nb)
-    invCol(h, nb, tid - 64);
-  __syncthreads();
-  if (nb > 0) {
-    // T = L21 M11 (M11 unit lower)
-    for (int e = tid; e < nb * h; e += blockDim.x) {
-      const int i = e % nb, j = e / nb;
-      double a = 0.0;
-      for (int k = j; k < h; ++k) a = fma(Lp[h + i][k], Mi[k][j], a);
-      Tt[i][j] = a;
-    }
-    __syncthreads();
-    // M21 = -(M22 T) (M22 unit lower)
-    for (int e = tid; e < nb * h; e += blockDim.x) {
-      const int i = e % nb, j = e / nb;
-      double a = Tt[i][j];
-      for (int k = 0; k < i; ++k) a = fma(Mi[h + i][h + k], Tt[k][j], a);
-      Mi[h + i][j] = -a;
-    }
-  }
-  __syncthreads();
-  const int i = nE + rowBlock * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  double x[P];
-  loadWiden<P>(x, static_cast<const T*>(F), [&](int q) -> int64_t {
-    return (q < p) ? i + static_cast<int64_t>(k0 + q) * m : -1;
-  });
-  // y = x M^T in place, last column first (y_q needs x_0 .. x_q only)
+  auto solve = [&](auto nb) {  // no branches: see settle
+    auto block = [&](auto bb) {
+      group(nb, bb, std::integral_constant<int, 0>{});
+      group(nb, bb, std::integral_constant<int, 1>{});
+      group(nb, bb, std::integral_constant<int, 2>{});
+      group(nb, bb, std::integral_constant<int, 3>{});
+    };
+    block(std::integral_constant<int, 0>{});
+    block(std::integral_constant<int, 1>{});
+    block(std::integral_constant<int, 2>{});
+    block(std::integral_constant<int, 3>{});
+    block(std::integral_constant<int, 4>{});
 #pragma unroll
-  for (int q = P - 1; q > 0; --q) {
-    if (q < p) {
-      double a0 = x[q], a1 = 0.0;
-#pragma unroll
-      for (int qp = 0; qp < q; ++qp) {
-        if (qp & 1)
-          a1 = fma(x[qp], Mi[q][qp], a1);
-        else
-          a0 = fma(x[qp], Mi[q][qp], a0);
-      }
-      x[q] = a0 + a1;
-    }
-  }
+    for (int b = 0; b < decltype(nb)::value; ++b) settle(x[b]);
+  };
+  if (p > kPanel)
+    solve(std::integral_constant<int, 5>{});
+  else if (p > 32)
+    solve(std::integral_constant<int, 4>{});
+  else if (p > 16)
+    solve(std::integral_constant<int, 2>{});
+  else
+    solve(std::integral_constant<int, 1>{});
   double mx = 0.0;
 #pragma unroll
-  for (int q = 0; q < P; ++q) {
-    if (q < p) {
-      const int kind = pkd[q];
-      if (kind == 1) {
-        mx = fmax(mx, fabs(x[q]));
-        Fat(i, k0 + q) = static_cast<T>(x[q] / pdd[q]);
-      } else if (kind == 2 && q + 1 < P) {
-        const double x0 = x[q], x1 = x[q + 1];
-        mx = fmax(mx, fmax(fabs(x0), fabs(x1)));
-        const double d11 = pdd[q], d21 = pdo[q], d22 = pdd[q + 1];
-        const double det = d11 * d22 - d21 * d21;
-        const double inv11 = d22 / det, inv21 = -d21 / det, inv22 = d11 / det;
-        Fat(i, k0 + q) = static_cast<T>(x0 * inv11 + x1 * inv21);
-        Fat(i, k0 + q + 1) = static_cast<T>(x0 * inv21 + x1 * inv22);
-      }
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int q = 16 * b + 4 * u + lk;
+      if (q < p) mx = fmax(mx, fabs(x[b][u]));
     }
+  double l[NB][4];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) l[b][u] = x[b][u] * cSelf[min(16 * b + 4 * u + lk, PP - 1)];
+  if (any2) {
+    // columns q + 1 and q - 1 of the same row: the neighbouring 16-lane
+    // group, in the next or previous register where the group wraps
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int q = 16 * b + 4 * u + lk, qc = min(q, PP - 1);
+        const int bn = u < 3 ? b : b + 1, un = (u + 1) & 3, bp = u > 0 ? b : b - 1, up = (u + 3) & 3;
+        const double nOwn = __shfl(x[b][u], (lane + 16) & 63, 64);
+        const double nWrap = bn < NB ? __shfl(x[bn < NB ? bn : b][un], (lane + 16) & 63, 64) : 0.0;
+        const double pOwn = __shfl(x[b][u], (lane + 48) & 63, 64);
+        const double pWrap = bp >= 0 ? __shfl(x[bp >= 0 ? bp : b][up], (lane + 48) & 63, 64) : 0.0;
+        l[b][u] += (lk < 3 ? nOwn : nWrap) * cNext[qc] + (lk > 0 ? pOwn : pWrap) * cPrev[qc];
+      }
   }
-  for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
-  if ((threadIdx.x & 63) == 0) atomicMaxNonNeg(fd.runMaxBits + s, mx);
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int q = 16 * b + 4 * u + lk;
+      if (q < p && row < m) F[at(row, k0 + q)] = static_cast<T>(l[b][u]);
+    }
+  mx = __ockl_wfred_max_f64(row < m ? mx : 0.0);
+  if (lane == 0) atomicMaxNonNeg(fd.runMaxBits + s, mx);
 }
 
 // Trailing update T(k1:m, k1:m) -= (L D) L^T over the lower triangle, for
@@ -2322,17 +2668,6 @@ struct SchurMfma<float> {
   static __device__ inline v4 mma(float a, float b, v4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
   static __device__ inline int col(int lane, int r) { return 4 * (lane >> 4) + r; }
 };
-
-// A front pointer read from the front table is generic; generic (flat)
-// accesses count against the LDS wait counter too, so every LDS wait would
-// also wait for them.  Front storage is global memory: this view makes the
-// accesses global ones.
-template <typename T>
-using GlobalPtr = __attribute__((address_space(1))) T*;
-template <typename T>
-__device__ inline GlobalPtr<T> globalView(void* p) {
-  return (GlobalPtr<T>)(p);
-}
 
 template <typename T>
 __global__ __launch_bounds__(256, 4) void k_schur(const int* list, int count, const int* tileStart, const int* tileTp,
@@ -2599,11 +2934,6 @@ __global__ __launch_bounds__(256) void k_form_w(DevFronts fd, int s, int q0, int
   }
 }
 
-__global__ void k_front_finish(const int* list, int count, DevFronts fd) {
-  const int f = blockIdx.x * blockDim.x + threadIdx.x;
-  if (f < count) fd.nF[list[f]] = fd.kcur[list[f]];
-}
-
 // rowIdx = frontIdx[perm[i]] for every position of the listed fronts.
 __global__ void k_make_rowidx(const int* list, int count, DevFronts fd) {
   if (static_cast<int>(blockIdx.x) >= count) return;
@@ -2712,37 +3042,32 @@ void launchFrontMaxAbs(const int* list, int count, int maxM, const DevFronts& fd
     k_front_maxabs<double><<<count * bpf, 256, 0, st>>>(list, count, bpf, fd);
   hipCheck(hipGetLastError(), "launchFrontMaxAbs");
 }
-template <int RM, typename T>
+template <int TPW, typename T>
 static void panelLaunch(const int* list, int count, const DevFronts& fd, const FactorParams& prm, double* ws,
                         const int64_t* wsOff, hipStream_t st) {
-  const size_t lds = PanelShape<RM>::lds();
-  static bool attrSet = false;
-  if (!attrSet && lds > 0) {
-    hipCheck(hipFuncSetAttribute(reinterpret_cast<const void*>(k_panel<RM, T>),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
-             "k_panel LDS size");
-    attrSet = true;
-  }
-  k_panel<RM, T><<<count, kPanelThreads, lds, st>>>(list, count, fd, prm, ws, wsOff);
+  constexpr size_t lds = PanelShape<TPW, T>::lds();
+  static const hipError_t attr =
+      lds > 0 ? hipFuncSetAttribute(reinterpret_cast<const void*>(k_panel<TPW, T>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds))
+              : hipSuccess;
+  hipCheck(attr, "k_panel LDS size");
+  k_panel<TPW, T><<<count, kPanelThreads, lds, st>>>(list, count, fd, prm, ws, wsOff);
   hipCheck(hipGetLastError(), "panelLaunch");
 }
 template <typename T>
 static void panelT(const int* list, int count, int maxRows, const DevFronts& fd, const FactorParams& prm, double* ws,
                    const int64_t* wsOff, hipStream_t st) {
-  // register slots per thread for the eligible rows of the widest front
-  const int slots = (maxRows + kPanelThreads - 1) / kPanelThreads;
-  if (slots <= 1)
+  // tiles per wave for the rows of the widest front
+  if (maxRows <= kPanelRegRows / 16)
     panelLaunch<1, T>(list, count, fd, prm, ws, wsOff, st);
-  else if (slots <= 2)
+  else if (maxRows <= kPanelRegRows / 8)
     panelLaunch<2, T>(list, count, fd, prm, ws, wsOff, st);
-  else if (slots <= 4)
+  else if (maxRows <= kPanelRegRows / 4)
     panelLaunch<4, T>(list, count, fd, prm, ws, wsOff, st);
-  else if (slots <= 8)
+  else if (maxRows <= kPanelRegRows / 2)
     panelLaunch<8, T>(list, count, fd, prm, ws, wsOff, st);
-  else if (slots <= 16)
+  else if (maxRows <= kPanelRegRows)
     panelLaunch<16, T>(list, count, fd, prm, ws, wsOff, st);
-  else if (slots <= 32)
-    panelLaunch<32, T>(list, count, fd, prm, ws, wsOff, st);
   else
     panelLaunch<0, T>(list, count, fd, prm, ws, wsOff, st);
 }
@@ -2847,11 +3172,6 @@ void launchFormW(const DevFronts& fd, int s, int rows, int q0, int kc, void* W, 
   else
     k_form_w<double><<<grid, 256, 0, st>>>(fd, s, q0, kc, static_cast<double*>(W));
   hipCheck(hipGetLastError(), "launchFormW");
-}
-void launchFrontFinish(const int* list, int count, const DevFronts& fd, hipStream_t st) {
-  if (count <= 0) return;
-  k_front_finish<<<(count + 255) / 256, 256, 0, st>>>(list, count, fd);
-  hipCheck(hipGetLastError(), "launchFrontFinish");
 }
 void launchMakeRowIdx(const int* list, int count, const DevFronts& fd, hipStream_t st) {
   if (count <= 0) return;

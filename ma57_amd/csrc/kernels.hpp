@@ -20,6 +20,7 @@ void launchAssemble(const int4* tasks, int ntasks, const DevFronts& fd, const do
 void launchFactorSmall(const int* list, int count, int maxM, const DevFronts& fd, const FactorParams& prm,
                        hipStream_t st);
 void launchFrontMaxAbs(const int* list, int count, int maxM, const DevFronts& fd, hipStream_t st);
+// maxRows: most rows any listed front holds in this panel (all of them at most kPanelRegRows, or none)
 void launchPanel(const int* list, int count, int maxRows, const DevFronts& fd, const FactorParams& prm, double* ws,
                  const int64_t* wsOff, hipStream_t st);
 // cooperative panels: list[f] factored by workgroups [wgStart[f], wgStart[f+1]) with sync[f]
@@ -33,6 +34,7 @@ void launchSpecPanel(const int* list, int count, const int* wgStart, int blocks,
                      const FactorParams& prm, double* ws, const int64_t* wsOff, hipStream_t st);
 void launchSpecReset(const int* list, int count, const DevFronts& fd, double* ws, const int64_t* wsOff,
                      hipStream_t st);
+constexpr int kPanelRowsWg = 64;  // rows [nE, m) per workgroup
 void launchPanelRows(const int* list, int count, const int* blockStart, int totalBlocks, const DevFronts& fd,
                      hipStream_t st);
 // tileTp: per listed front, the planned 64-row tiles per side of its trailing block
@@ -41,7 +43,6 @@ void launchSyrk(const int* list, int count, const int* tileStart, const int* til
 // W = L(nE:m, q0:q0+kc) D of front s (rows = m - nE, column-major, ld = rows;
 // float for FP32 fronts), zero past the pivots taken
 void launchFormW(const DevFronts& fd, int s, int rows, int q0, int kc, void* W, hipStream_t st);
-void launchFrontFinish(const int* list, int count, const DevFronts& fd, hipStream_t st);
 void launchMakeRowIdx(const int* list, int count, const DevFronts& fd, hipStream_t st);
 void launchReduceStats(int numSN, const DevFronts& fd, long long* outI, double* outD, hipStream_t st);
 

@@ -550,7 +550,7 @@ LargeSched buildLargeSched(const std::vector<int>& fronts, const std::vector<int
     li.tileOff = static_cast<int64_t>(h.tileStart.size());
     int rb = 0, tl = 0, sb = 0;
     li.specOff = static_cast<int64_t>(h.specStart.size());
-    std::vector<int> reg, mw, mwW;
+    std::vector<int> reg, big, mw, mwW;
     int mwTotal = 0;
     for (int s : fronts) {
       if ((nE[s] + kPanel - 1) / kPanel <= it) continue;
@@ -558,10 +558,12 @@ LargeSched buildLargeSched(const std::vector<int>& fronts, const std::vector<int
       h.rowStart.push_back(rb);
       h.tileStart.push_back(tl);
       h.specStart.push_back(sb);
-      rb += (m[s] - nE[s] + 255) / 256;
+      const bool spec = specMinRows >= 0 && nE[s] > specMinRows;
+      const bool all = panelHoldsAllRows(m[s], spec);
+      if (!all) rb += (m[s] - nE[s] + kPanelRowsWg - 1) / kPanelRowsWg;
       // rows below this iteration's diagonal block (the block starts at or after it * kPanel)
       const int below = m[s] - it * kPanel - std::min(kPanel, nE[s] - it * kPanel);
-      if (specMinRows >= 0 && nE[s] > specMinRows) sb += std::max(1, (below + kSpecRows - 1) / kSpecRows);
+      if (spec) sb += std::max(1, (below + kSpecRows - 1) / kSpecRows);
       // trailing tiles: T per side from this iteration's panel start, column
       // blocks up to the cut
       const int T = (m[s] - it * kPanel + 63) / 64;
@@ -578,8 +580,10 @@ LargeSched buildLargeSched(const std::vector<int>& fronts, const std::vector<int
         mwW.push_back(W);
         mwTotal += W;
       } else {
-        reg.push_back(s);
-        li.regMaxNE = std::max(li.regMaxNE, nE[s]);
+        const int held = all ? m[s] - it * kPanel : rows;
+        (held > kPanelRegRows ? big : reg).push_back(s);
+        int& most = held > kPanelRegRows ? li.bigMaxRows : li.regMaxRows;
+        most = std::max(most, held);
       }
     }
     h.rowStart.push_back(rb);
@@ -587,11 +591,15 @@ LargeSched buildLargeSched(const std::vector<int>& fronts, const std::vector<int
     h.tileTp.push_back(0);  // keeps tileTp at the offsets of tileStart
     h.specStart.push_back(sb);
     li.specBlocks = sb;
+    if (sb > 0) ls.spec = true;
     li.rowBlocks = rb;
     li.tiles = tl;
     li.regOff = static_cast<int64_t>(h.lists.size());
     li.regCount = static_cast<int>(reg.size());
     h.lists.insert(h.lists.end(), reg.begin(), reg.end());
+    li.bigOff = static_cast<int64_t>(h.lists.size());
+    li.bigCount = static_cast<int>(big.size());
+    h.lists.insert(h.lists.end(), big.begin(), big.end());
     li.mwOff = static_cast<int64_t>(h.lists.size());
     li.mwCount = static_cast<int>(mw.size());
     h.lists.insert(h.lists.end(), mw.begin(), mw.end());
@@ -612,7 +620,7 @@ void runLargeSched(const LargeSched& ls, const LargeDev& dv, const DevFronts& fd
                    const int64_t* wsOff, hipStream_t st, const CbUpdate* cb, Plan* prof) {
   if (ls.allCount == 0) return;
   if (!dv.frontMaxDone) launchFrontMaxAbs(dv.lists + ls.allOff, ls.allCount, ls.maxM, fd, st);
-  if (prm.specPanel) launchSpecReset(dv.lists + ls.allOff, ls.allCount, fd, ws, wsOff, st);
+  if (ls.spec) launchSpecReset(dv.lists + ls.allOff, ls.allCount, fd, ws, wsOff, st);
   for (size_t t = 0; t < ls.iters.size(); ++t) {
     const LargeIter& it = ls.iters[t];
     const int* lst = dv.lists + it.listOff;
@@ -620,7 +628,8 @@ void runLargeSched(const LargeSched& ls, const LargeDev& dv, const DevFronts& fd
     if (prm.specPanel && it.specBlocks > 0)
       launchSpecPanel(lst, it.count, dv.specStart + it.specOff, it.specBlocks, static_cast<int>(t & 1), fd, prm, ws,
                       wsOff, st);
-    launchPanel(dv.lists + it.regOff, it.regCount, it.regMaxNE, fd, prm, ws, wsOff, st);
+    launchPanel(dv.lists + it.regOff, it.regCount, it.regMaxRows, fd, prm, ws, wsOff, st);
+    launchPanel(dv.lists + it.bigOff, it.bigCount, it.bigMaxRows, fd, prm, ws, wsOff, st);
     launchPanelMw(dv.lists + it.mwOff, it.mwCount, dv.mwStart + it.mwStartOff, it.mwBlocks, fd, prm, ws, wsOff,
                   dv.sync, dv.err, st);
     if (prof) prof->profEnd(Plan::kProfPanel);
@@ -633,7 +642,6 @@ void runLargeSched(const LargeSched& ls, const LargeDev& dv, const DevFronts& fd
     launchSyrk(lst, it.count, dv.tileStart + it.tileOff, dv.tileTp + it.tileOff, it.tiles, fd, st);
     if (prof) prof->profEnd(Plan::kProfSyrk);
   }
-  launchFrontFinish(dv.lists + ls.allOff, ls.allCount, fd, st);
   if (ls.cb.empty()) return;
   if (!cb || !cb->w || !cb->F) throw std::logic_error("symla: deferred contribution blocks without a workspace");
   const size_t esz = cb->fp32 ? sizeof(float) : sizeof(double);

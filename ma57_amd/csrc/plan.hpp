@@ -117,9 +117,12 @@ struct LargeIter {
   int rowBlocks = 0;
   int64_t tileOff = 0;
   int tiles = 0;
-  int64_t regOff = 0;  // single-workgroup panels
+  int64_t regOff = 0;  // single-workgroup panels whose rows stay in registers
   int regCount = 0;
-  int regMaxNE = 0;    // widest eligible-row count among them
+  int regMaxRows = 0;  // most rows held by one of them
+  int64_t bigOff = 0;  // single-workgroup panels with more than kPanelRegRows rows
+  int bigCount = 0;
+  int bigMaxRows = 0;
   int64_t mwOff = 0;   // cooperative panels: fronts, and workgroup starts at mwStartOff
   int mwCount = 0;
   int64_t mwStartOff = 0;
@@ -150,6 +153,7 @@ struct LargeSched {
   int64_t allOff = 0;
   int allCount = 0;
   int maxM = 0;
+  bool spec = false;  // some front takes the speculative step
   std::vector<LargeIter> iters;
   std::vector<CbTask> cb;  // fronts whose contribution block is updated after their last panel
 };
