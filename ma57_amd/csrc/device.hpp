@@ -118,14 +118,15 @@ __host__ __device__ inline bool specFront(const FactorParams& p, int nE) { retur
 //   dval[kPanel]       the pivot d_q (1 past the block)
 //   bmax[kPanel]       max |c_iq| over the block rows below q
 //   rdiv[kPanel]       1 / d_q (1 past the block)
-//   lblk[kPanel * kPanel]  multipliers of the block, l_iq at [i * kPanel + q]
-//   wmat[kPanel * kPanel]  d_j l_qj at [q * kPanel + j] (j < q): the row
-//                      substitution's coefficients
+//   ops[4 * 4 * 64]    the row substitution's operands of the block's four
+//                      16-column blocks (Block16::op each)
+//   wneg[6 * 4 * 64]   -d_q l_jq of the 16 x 16 tiles (column block b2, b < b2)
+//                      at 256 (b2 (b2 - 1) / 2 + b), in the MFMA operand's lane order
 // followed, for fronts that take the step, by the backup of the raw panel
-// values of the rows below the block (m x kPanel front elements, row i of
-// panel column q at i + q m), from which a failed test restores them.
-constexpr int kSpecRec = 8 * kPanel + 2 * kPanel * kPanel;
-constexpr int kSpecRows = 256;  // rows below the block per workgroup (one per thread)
+// values of the block's rows and those below (m x kPanel front elements, row
+// i of panel column q at i + q m), from which a failed test restores them.
+constexpr int kSpecRec = 8 * kPanel + (4 + 6) * 4 * 64;
+constexpr int kSpecRows = 64;  // rows below the block per workgroup (16 per wave)
 // The panel kernel keeps up to kPanelRegRows rows in registers; a front with
 // more eligible rows streams them through 16 more columns of its workspace.
 constexpr int kPanelRegRows = 2048;

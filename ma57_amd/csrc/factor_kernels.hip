@@ -126,20 +126,11 @@ __device__ inline void countInertia2(double d11, double d22, double det, int& po
 // Static pivot (dense_kernel.hpp:982-1011): returns the pivot to use and the
 // perturbation applied.
 __device__ inline double staticPivot(double a_kk, int sign, double delta, double floorv, double& applied) {
-  bool need;
-  if (sign > 0)
-    need = a_kk < floorv;
-  else if (sign < 0)
-    need = a_kk > -floorv;
-  else
-    need = fabs(a_kk) < floorv;
-  double d = a_kk;
-  applied = 0.0;
-  if (need) {
-    const double s = (sign != 0) ? static_cast<double>(sign) : (a_kk >= 0.0 ? 1.0 : -1.0);
-    d = a_kk + s * delta;
-    applied = d - a_kk;
-  }
+  // (selects, no branches: it is on the panels' dependent chain)
+  const double s = sign != 0 ? static_cast<double>(sign) : (a_kk >= 0.0 ? 1.0 : -1.0);
+  const double towards = sign != 0 ? a_kk * s : fabs(a_kk);
+  const double d = towards < floorv ? a_kk + s * delta : a_kk;
+  applied = d - a_kk;
   return d;
 }
 
@@ -1968,11 +1959,10 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel_mw(const int* list, int
 // at k (dense_kernel.hpp:982-1011).  When every pivot of a panel is taken
 // that way, the panel is an unpivoted LDL^T of its diagonal block followed by
 // the substitution of the rows below, and lambda_k is max |c_ik| over the
-// values c_ik the substitution forms.  k_spec_factor does that factorization
-// and the column maxima without writing the front; k_spec_apply finds the
-// first column whose test fails, keeps the columns before it, and leaves the
-// rest (still holding current values) to the exact panel kernel, which
-// continues from there.
+// values c_ik the substitution forms.  k_spec_block and k_spec_factor do
+// both, writing the multipliers over the raw values they back up, and form
+// the column maxima; k_spec_apply finds the first column whose test fails and
+// restores the columns from there on, and the exact panel kernel continues.
 // ---------------------------------------------------------------------------
 struct SpecRec {
   unsigned long long* colmax;  // [2][kPanel]
@@ -1982,8 +1972,8 @@ struct SpecRec {
   double* dval;
   double* bmax;
   double* rdiv;
-  double* lblk;
-  double* wmat;
+  double* ops;
+  double* wneg;
   double* backup;
 };
 __device__ inline SpecRec specRec(double* ws, int nE) {
@@ -1996,59 +1986,10 @@ __device__ inline SpecRec specRec(double* ws, int nE) {
   x.dval = r + 5 * kPanel;
   x.bmax = r + 6 * kPanel;
   x.rdiv = r + 7 * kPanel;
-  x.lblk = r + 8 * kPanel;
-  x.wmat = r + 8 * kPanel + kPanel * kPanel;
+  x.ops = r + 8 * kPanel;
+  x.wneg = x.ops + 4 * 4 * 64;
   x.backup = r + kSpecRec;
   return x;
-}
-
-// One row below the diagonal block: x holds its raw values in the panel
-// columns; for q < lim in order, c_q = x_q - sum_{j<q} l_j W[q][j] with
-// W[q][j] = d_j l_qj, then x[q] = l_q = T(c_q r_q), r_q = 1 / d_q (rdv: the
-// pivots' reciprocals, so the chain over q carries no division).  onC(q, c_q)
-// sees every current value; onGroup(g) runs after columns 16 g .. 16 g + 15
-// (every thread of the workgroup reaches it).
-//
-// The coefficients are broadcast LDS reads, 16 at a time: a chunk's reads are
-// all issued before its products (the empty asm statements keep the compiler
-// from interleaving them), so their latencies overlap.
-template <typename T, typename OnC, typename OnGroup>
-__device__ inline void specRow(double (&x)[kPanel], const double (*W)[kPanel], const double* rdv, int lim, OnC onC,
-                               OnGroup onGroup) {
-#pragma unroll
-  for (int g = 0; g < kPanel / 16; ++g) {
-#pragma unroll
-    for (int qq = 0; qq < 16; ++qq) {
-      const int q = 16 * g + qq;
-      if (q < lim) {
-        double c0 = x[q], c1 = 0.0;
-#pragma unroll
-        for (int j0 = 0; j0 < q; j0 += 16) {
-          double w[16];
-#pragma unroll
-          for (int u = 0; u < 16; ++u)
-            if (j0 + u < q) w[u] = W[q][j0 + u];
-#pragma unroll
-          for (int u = 0; u < 16; ++u)
-            if (j0 + u < q) asm volatile("" : "+v"(w[u]));
-#pragma unroll
-          for (int u = 0; u < 16; ++u) {
-            const int j = j0 + u;
-            if (j < q) {
-              if (j & 1)
-                c1 = fma(-x[j], w[u], c1);
-              else
-                c0 = fma(-x[j], w[u], c0);
-            }
-          }
-        }
-        const double c = c0 + c1;
-        onC(q, c);
-        x[q] = static_cast<double>(static_cast<T>(c * rdv[q]));
-      }
-    }
-    if (16 * g < lim) onGroup(g);
-  }
 }
 
 // Smallest float at or above v (v >= 0): a bound that is never below the value.
@@ -2059,17 +2000,26 @@ __device__ inline double roundUpToFloat(double v) {
 }
 
 // Pass 0: one workgroup per front factors the diagonal block (pw x pw,
-// pw = min(kPanel, nE - k0)) in registers, 1x1 pivots in order, and writes
-// the record: multipliers, pivots and their reciprocals, a_qq, the in-block
-// column maxima and W = (d_j l_qj) for the row passes.
+// pw = min(kPanel, nE - k0)), 1x1 pivots in order, as four blocks of 16
+// columns: wave w holds the block's rows 16 w .. 16 w + 15 as MFMA tiles, the
+// wave of the diagonal tile factors it (blockFactor16), the waves below
+// substitute their rows and update their later columns on the matrix cores.
+// The raw values go to the record's backup and the multipliers into the
+// front, where a failed test restores them; the record takes the pivots,
+// their reciprocals, a_qq, the in-block column maxima and the row pass's
+// operands.
+//
+// Bound by the dependent chain of 64 pivots: 4 x 6,000 cycles, 10 us of the
+// 22 on the 80^3 27-point workload (a barrier per two pivots on registers and
+// LDS took 37; 28 against 45 with static pivots).
 template <typename T>
 __global__ __launch_bounds__(256) void k_spec_block(const int* list, int count, DevFronts fd, FactorParams prm,
                                                     double* wsBase, const int64_t* wsOff) {
   constexpr int P = kPanel;
-  __shared__ double cvec[2][2][P];  // [step parity][column q, q + 1]
-  __shared__ double dv[P], rdv[P];
-  __shared__ int sgn[P];
-  __shared__ double red[4][P];
+  __shared__ double Ds[16][17];
+  __shared__ Block16 blk;
+  __shared__ double Ls[4][64][4];  // multipliers of the current 16 columns: wave w's tile, lane-major
+  __shared__ double redB[4][P];
   if (static_cast<int>(blockIdx.x) >= count) return;
   const int s = list[blockIdx.x];
   const int nE = fd.nE[s];
@@ -2078,141 +2028,133 @@ __global__ __launch_bounds__(256) void k_spec_block(const int* list, int count, 
   const int k0 = fd.kcur[s];
   if (k0 >= nE) return;
   const int pw = min(P, nE - k0);
-  const T* F = static_cast<const T*>(fd.F[s]);
+  const GlobalPtr<T> F = globalView<T>(fd.F[s]);
   const int64_t io = fd.idxOff[s];
   const SpecRec rec = specRec(wsBase + wsOff[s], nE);
-  const int tid = threadIdx.x;
+  T* const bk = reinterpret_cast<T*>(rec.backup);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lk = lane >> 4;
   const bool stat = prm.staticMode != 0;
   double origMax = bitsToDouble(fd.origMaxBits[s]);
   if (stat && origMax < prm.staticAbsFloor) origMax = 1.0;
   const double delta = prm.staticDelta > 0.0 ? prm.staticDelta : sqrt(DBL_EPSILON) * origMax;
   const double sfloor = fmax(prm.staticAbsFloor, prm.staticRelFloor * origMax);
-  for (int q = tid; q < pw; q += 256)
-    sgn[q] = (stat && prm.expectedSign) ? prm.expectedSign[fd.frontIdx[io + k0 + q]] : 0;
-  // block entry (i, j), i >= j: column j = tid % 64, rows i = tid / 64 + 4 r
-  const int j = tid & 63, ib = tid >> 6;
-  double a[16];
-  loadWiden<16>(a, F, [&](int r) -> int64_t {
-    const int i = ib + 4 * r;
-    return (i < pw && j < pw && i >= j) ? (k0 + i) + static_cast<int64_t>(k0 + j) * m : -1;
-  });
-  __syncthreads();
-  // Right-looking: a_ij -= c_iq l_jq (c_iq = d_q l_iq up to the rounding of
-  // the stored multiplier), l_jq = T(c_jq (1 / d_q)), two pivots per step.
-  // Columns q and q + 1 go through LDS whole after one barrier; every lane
-  // applies pivot q to its copy of column q + 1 (the same operations lane
-  // q + 1 applies to its own) before taking pivot q + 1, so the result is that
-  // of one pivot per step.  A column's lane updates all its rows: entries
-  // above the diagonal or past the block take values that nothing reads, and
-  // the lower-triangle entries combine lower-triangle entries only.
-  for (int q = 0; q < pw; q += 2) {
-    double* cv0 = cvec[(q >> 1) & 1][0];
-    double* cv1 = cvec[(q >> 1) & 1][1];
-    const bool two = q + 1 < pw;
-    if (j == q) {
+  const int row = 16 * wv + lr;  // of the block
+  const int sgn = stat && prm.expectedSign && row < pw ? prm.expectedSign[fd.frontIdx[io + k0 + row]] : 0;
+  T raw[4][4];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) cv0[ib + 4 * r] = a[r];
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int col = 16 * b + 4 * u + lk;
+      raw[b][u] = F[row < pw && col <= row ? (k0 + row) + static_cast<int64_t>(k0 + col) * m : 0];
     }
-    if (j == q + 1) {
+  v4d x[4];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) cv1[ib + 4 * r] = a[r];
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int col = 16 * b + 4 * u + lk;
+      const bool in = row < pw && col <= row;
+      if (in) bk[(k0 + row) + static_cast<int64_t>(col) * m] = raw[b][u];
+      x[b][u] = in ? static_cast<double>(raw[b][u]) : (col == row ? 1.0 : 0.0);
+    }
+  unrolled(std::make_integer_sequence<int, 4>{}, [&](auto bb) {
+    constexpr int b = decltype(bb)::value;
+    if (16 * b >= pw) return;
+    if (wv == b) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) Ds[lr][4 * u + lk] = x[b][u];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      double a[16];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) a[q] = Ds[lr][q];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) a[q] = q <= lr ? a[q] : 0.0;
+      if (!stat)
+        blockFactor16<T>(a, blk, [](int, double v) { return v; });
+      else
+        blockFactor16<T>(a, blk, [&](int q, double v) {
+          // (the identity padding is not a pivot)
+          double applied;
+          const double d = staticPivot(v, __shfl(sgn, q, 64), delta, sfloor, applied);
+          return 16 * b + q < pw ? d : v;
+        });
     }
     __syncthreads();
-    double ci0[16], ci1[16];
+    if (wv == b) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      ci0[r] = cv0[ib + 4 * r];
-      ci1[r] = cv1[ib + 4 * r];
-    }
-    const double cj0 = cv0[j];
-    double cj1 = cv1[j];
-    double d0 = cv0[q];
-    const double b10 = cv0[q + 1];  // c_{q+1,q}
-    double d1 = cv1[q + 1];
-    if (stat) {
-      double applied;
-      d0 = staticPivot(d0, sgn[q], delta, sfloor, applied);
-    }
-    const double rd0 = pivotRecip(d0);
-    const double lj0 = static_cast<double>(static_cast<T>(cj0 * rd0));
-    if (j > q && j < pw) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) a[r] = fma(-ci0[r], lj0, a[r]);
-    }
-    if (tid == 0) {
-      dv[q] = d0;
-      rdv[q] = rd0;
-    }
-    if (two) {
-      // column q + 1 after pivot q
-      const double l10 = static_cast<double>(static_cast<T>(b10 * rd0));
-#pragma unroll
-      for (int r = 0; r < 16; ++r) ci1[r] = fma(-ci0[r], l10, ci1[r]);
-      cj1 = fma(-cj0, l10, cj1);
-      d1 = fma(-b10, l10, d1);
-      if (stat) {
-        double applied;
-        d1 = staticPivot(d1, sgn[q + 1], delta, sfloor, applied);
-      }
-      const double rd1 = pivotRecip(d1);
-      const double lj1 = static_cast<double>(static_cast<T>(cj1 * rd1));
-      if (j > q + 1 && j < pw) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) a[r] = fma(-ci1[r], lj1, a[r]);
-      }
-      if (tid == 0) {
-        dv[q + 1] = d1;
-        rdv[q + 1] = rd1;
+      for (int u = 0; u < 4; ++u) rec.ops[(4 * b + u) * 64 + lane] = blk.op[u][lane];
+      if (lane < 16) {
+        rec.cdiag[16 * b + lane] = blk.akk[lane];
+        rec.dval[16 * b + lane] = blk.d[lane];
+        rec.rdiv[16 * b + lane] = blk.rd[lane];
       }
     }
-  }
-  // columns past the block: a neutral pivot for the branch-free row solve
-  for (int q = pw + tid; q < P; q += 256) {
-    dv[q] = 1.0;
-    rdv[q] = 1.0;
-  }
+    double vm[4];
+    if (wv >= b) {
+      double op[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) op[u] = blk.op[u][lane];
+      substTile(x[b], op);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int q = 4 * u + lk, col = 16 * b + q;
+        const T lt = static_cast<T>(x[b][u] * blk.rd[q]);
+        const double l = static_cast<double>(lt);
+        if (row < pw && col < row) F[(k0 + row) + static_cast<int64_t>(k0 + col) * m] = lt;
+        if (row < pw && col == row) F[(k0 + row) + static_cast<int64_t>(k0 + col) * m] = static_cast<T>(blk.d[q]);
+        vm[u] = row < pw && col < row ? fabs(x[b][u]) : 0.0;
+        if (wv > b) {
+          Ls[wv][lane][u] = l;
+          rec.wneg[((wv * (wv - 1) / 2 + b) * 4 + u) * 64 + lane] = row < pw ? -(blk.d[q] * l) : 0.0;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) vm[u] = 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const double v = max16(vm[u]);
+      if (lr == 0) redB[wv][16 * b + 4 * u + lk] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b2 = b + 1; b2 < 4; ++b2) {
+      if (wv >= b2) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[b2] = mfma64(-Ls[b2][lane][u], x[b][u], x[b2]);
+        settle(x[b2]);
+      }
+    }
+  });
   __syncthreads();
-  // a now holds c_ij (current value at pivot j) for i > j and a_jj^(j) on the diagonal
-  double bm = 0.0;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int i = ib + 4 * r;
-    if (j < pw && i < pw) {
-      if (i > j) {
-        const double l = static_cast<double>(static_cast<T>(a[r] * rdv[j]));
-        rec.wmat[i * P + j] = dv[j] * l;
-        rec.lblk[i * P + j] = l;
-        bm = fmax(bm, fabs(a[r]));
-      } else if (i == j) {
-        rec.cdiag[j] = a[r];
-      }
-    }
-  }
-  red[ib][j] = bm;
-  __syncthreads();
-  if (tid < P) {
-    rec.dval[tid] = dv[tid];
-    rec.rdiv[tid] = rdv[tid];
-    rec.bmax[tid] = fmax(fmax(red[0][tid], red[1][tid]), fmax(red[2][tid], red[3][tid]));
-  }
+  if (tid < pw) rec.bmax[tid] = fmax(fmax(redB[0][tid], redB[1][tid]), fmax(redB[2][tid], redB[3][tid]));
 }
 
 // Pass 1: every workgroup takes kSpecRows rows below the block of a front
-// (eligible rows [k0 + pw, nE) and rows [nE, m) alike), saves their raw panel
-// values in the record's backup, forms their multipliers for the whole block
-// and stores them in the front.  The column maxima of the current values go
-// to the record: over the eligible rows rounded up to float (colmax[parity],
-// the threshold test) and exact (emax), over the rows [nE, m) exact (nmax).
+// (eligible rows [k0 + pw, nE) and rows [nE, m) alike), 16 per wave as MFMA
+// tiles: saves their raw panel values in the record's backup, substitutes
+// them by the block's four 16-column blocks and stores the multipliers in the
+// front.  What a block takes off the later columns is the stored multiplier
+// times its pivot.  All operands come from the record in lane order, in
+// flight together with the rows, so the pass is one memory round trip, 40
+// dependent-chain MFMAs (2,600 cycles) and the stores.  The column maxima of
+// the current values go to the record: over the eligible rows rounded up to
+// float (colmax[parity], the threshold test) and exact (emax), over the rows
+// [nE, m) exact (nmax).
+//
+// (One row per thread with the coefficients broadcast from LDS took 31 us a
+// launch on the 80^3 27-point workload, this form 19.)
 template <typename T>
-__global__ __launch_bounds__(kSpecRows) void k_spec_factor(const int* list, int count, const int* wgStart, int parity,
-                                                     DevFronts fd, FactorParams prm, double* wsBase,
-                                                     const int64_t* wsOff) {
+__global__ __launch_bounds__(4 * kSpecRows) void k_spec_factor(const int* list, int count, const int* wgStart,
+                                                               int parity, DevFronts fd, FactorParams prm,
+                                                               double* wsBase, const int64_t* wsOff) {
   constexpr int P = kPanel;
-  constexpr int NT = kSpecRows;  // one row per thread
-  constexpr int NW = NT / 64;
-  __shared__ __align__(16) double W[P][P];  // whole 16-byte rows: broadcast reads of two coefficients at once
-  __shared__ double rdv[P];
-  __shared__ double cm[16][kSpecRows + 1];  // |c| (eligible rows) or -|c| (rows [nE, m)) of 16 columns
+  constexpr int NW = kSpecRows / 16;
   __shared__ double partE[NW][P], partN[NW][P];
   if (static_cast<int>(blockIdx.x) >= wgStart[count]) return;
   const int f = findSegment(wgStart, count, blockIdx.x);
@@ -2226,74 +2168,93 @@ __global__ __launch_bounds__(kSpecRows) void k_spec_factor(const int* list, int 
   const int pw = min(P, nE - k0);
   const int rBeg = k0 + pw + w * kSpecRows;
   if (rBeg >= m) return;
-  T* F = static_cast<T*>(fd.F[s]);
+  const GlobalPtr<T> F = globalView<T>(fd.F[s]);
   const SpecRec rec = specRec(wsBase + wsOff[s], nE);
-  const int tid = threadIdx.x;
-  const int i = rBeg + tid;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lk = lane >> 4;
+  const int i0 = rBeg + 16 * wv, i = i0 + lr;
   const bool valid = i < m;
-  const bool elig = i < nE;
-  // the block's substitution coefficients, the reciprocal pivots and the
-  // row's raw values all in flight together (coefficients outside the
-  // block's lower triangle and skipped row entries are read and dropped)
-  double wv[P * P / NT];
+  // the panel's first nb blocks of 16 columns
+  auto rows = [&](auto nb) {
+    constexpr int NB = decltype(nb)::value;
+    T raw[NB][4];
 #pragma unroll
-  for (int u = 0; u < P * P / NT; ++u) wv[u] = rec.wmat[tid + NT * u];
-  const double rv = rec.rdiv[tid & (P - 1)];
-  T raw[P];
-  bool ok[P];
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
-  for (int q = 0; q < P; ++q) {
-    ok[q] = valid && q < pw;
-    raw[q] = F[ok[q] ? i + static_cast<int64_t>(k0 + q) * m : 0];
-  }
+      for (int u = 0; u < 4; ++u) {
+        const int q = 16 * b + 4 * u + lk;
+        raw[b][u] = F[valid && q < pw ? i + static_cast<int64_t>(k0 + q) * m : 0];
+      }
+    double op[NB][4], wn[NB > 1 ? NB * (NB - 1) / 2 : 1][4], rd[NB][4];
 #pragma unroll
-  for (int u = 0; u < P * P / NT; ++u) {
-    const int e = tid + NT * u, q = e / P, j = e % P;
-    W[q][j] = (j < q && q < pw) ? wv[u] : 0.0;
-  }
-  if (tid < P) rdv[tid] = rv;
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        op[b][u] = rec.ops[(4 * b + u) * 64 + lane];
+        rd[b][u] = rec.rdiv[16 * b + 4 * u + lk];
+      }
+#pragma unroll
+    for (int b = 0; b < NB * (NB - 1) / 2; ++b)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) wn[b][u] = rec.wneg[(4 * b + u) * 64 + lane];
+    v4d x[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[b][u] = valid && 16 * b + 4 * u + lk < pw ? static_cast<double>(raw[b][u]) : 0.0;
+    // the raw values saved for the exact kernel
+    T* bk = reinterpret_cast<T*>(rec.backup);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int q = 16 * b + 4 * u + lk;
+        if (valid && q < pw) bk[i + static_cast<int64_t>(q) * m] = raw[b][u];
+      }
+    // no branches among the products: see settle
+    T l[NB][4];
+    unrolled(std::make_integer_sequence<int, NB>{}, [&](auto bb) {
+      constexpr int b = decltype(bb)::value;
+      substTile(x[b], op[b]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) l[b][u] = static_cast<T>(x[b][u] * rd[b][u]);
+#pragma unroll
+      for (int b2 = b + 1; b2 < NB; ++b2) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          x[b2] = mfma64(wn[b2 * (b2 - 1) / 2 + b][u], static_cast<double>(l[b][u]), x[b2]);
+      }
+    });
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int q = 16 * b + 4 * u + lk;
+        if (valid && q < pw) F[i + static_cast<int64_t>(k0 + q) * m] = l[b][u];
+      }
+    const bool anyE = i0 < nE, anyN = i0 + 16 > nE;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const double c = fabs(x[b][u]);
+        const int q = 16 * b + 4 * u + lk;
+        const double ve = anyE ? max16(i < nE ? c : 0.0) : 0.0;
+        const double vn = anyN ? max16(i >= nE && valid ? c : 0.0) : 0.0;
+        if (lr == 0) {
+          partE[wv][q] = ve;
+          partN[wv][q] = vn;
+        }
+      }
+  };
+  if (pw <= 16)
+    rows(std::integral_constant<int, 1>{});
+  else if (pw <= 32)
+    rows(std::integral_constant<int, 2>{});
+  else
+    rows(std::integral_constant<int, 4>{});
   __syncthreads();
-  double x[P];
-#pragma unroll
-  for (int q = 0; q < P; ++q) x[q] = ok[q] ? static_cast<double>(raw[q]) : 0.0;
-  // the raw values saved for the exact kernel (completed by the first
-  // column group's barrier, long before anything reads them)
-  T* bk = reinterpret_cast<T*>(rec.backup);
-#pragma unroll
-  for (int q = 0; q < P; ++q)
-    if (ok[q]) bk[i + static_cast<int64_t>(q) * m] = raw[q];
-  // column maxima through LDS, 16 columns at a time
-  specRow<T>(
-      x, W, rdv, pw,
-      [&](int q, double c) {
-        const double ac = fabs(c);
-        cm[q & 15][tid] = elig ? ac : -ac;
-      },
-      [&](int g) {
-        __syncthreads();
-        const int col = tid & 15, seg = tid >> 4;  // 16 rows per thread
-        double ve = 0.0, vn = 0.0;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const double v = cm[col][seg * 16 + r];
-          ve = fmax(ve, v);
-          vn = fmax(vn, -v);
-        }
-        ve = fmax(ve, __shfl_xor(ve, 16, 64));
-        ve = fmax(ve, __shfl_xor(ve, 32, 64));
-        vn = fmax(vn, __shfl_xor(vn, 16, 64));
-        vn = fmax(vn, __shfl_xor(vn, 32, 64));
-        if ((tid & 63) < 16) {
-          partE[tid >> 6][16 * g + col] = ve;
-          partN[tid >> 6][16 * g + col] = vn;
-        }
-        __syncthreads();
-      });
-  if (valid) {
-#pragma unroll
-    for (int q = 0; q < P; ++q)
-      if (q < pw) F[i + static_cast<int64_t>(k0 + q) * m] = static_cast<T>(x[q]);
-  }
   if (tid < pw) {
     double ve = partE[0][tid], vn = partN[0][tid];
 #pragma unroll
@@ -2309,6 +2270,7 @@ __global__ __launch_bounds__(kSpecRows) void k_spec_factor(const int* list, int 
   }
 }
 
+constexpr int kSpecApplyThreads = kSpecRows;
 // Pass 2: every workgroup finds the first column q* whose test fails (all of
 // them pass when static); when q* < pw it restores, for its rows, the raw
 // values the exact kernel continues from (columns [q*, pw) of the eligible
@@ -2317,7 +2279,7 @@ __global__ __launch_bounds__(kSpecRows) void k_spec_factor(const int* list, int 
 // maximum, sets kcur = k0 + q*, pcount = q*, and clears the other colmax
 // buffer and the exact maxima for the next panel.
 template <typename T>
-__global__ __launch_bounds__(kSpecRows) void k_spec_apply(const int* list, int count, const int* wgStart, int parity,
+__global__ __launch_bounds__(kSpecApplyThreads) void k_spec_apply(const int* list, int count, const int* wgStart, int parity,
                                                     DevFronts fd, FactorParams prm, double* wsBase,
                                                     const int64_t* wsOff) {
   constexpr int P = kPanel;
@@ -2365,18 +2327,19 @@ __global__ __launch_bounds__(kSpecRows) void k_spec_apply(const int* list, int c
   __syncthreads();
   const int qs = qsh;
   if (qs < pw) {
+    const T* bk = reinterpret_cast<const T*>(rec.backup);
     const int i = rBeg + tid;
     if (i < m) {
-      const T* bk = reinterpret_cast<const T*>(rec.backup);
       for (int q = (i < nE) ? qs : 0; q < pw; ++q) Fat(i, k0 + q) = bk[i + static_cast<int64_t>(q) * m];
     }
+    if (w == 0)  // the block's own rows
+      for (int e = tid; e < pw * P; e += kSpecApplyThreads) {
+        const int r = e & (P - 1), q = e / P;
+        if (q >= qs && r >= q && r < pw) Fat(k0 + r, k0 + q) = bk[(k0 + r) + static_cast<int64_t>(q) * m];
+      }
   }
   if (w != 0) return;
   double tmax = 0.0;
-  for (int e = tid; e < pw * pw; e += kSpecRows) {
-    const int q = e / pw, r = e % pw;  // column q, row r of the block
-    if (q < qs && r >= q) Fat(k0 + r, k0 + q) = static_cast<T>(r == q ? rec.dval[q] : rec.lblk[r * P + q]);
-  }
   if (tid < P) rec.colmax[(parity ^ 1) * P + tid] = 0ull;
   if (tid < 64) {
     // pivots, inertia, perturbation and the maxima of the kept columns: one column per lane
@@ -3117,15 +3080,15 @@ void launchSpecPanel(const int* list, int count, const int* wgStart, int blocks,
   if (fd.fp32) {
     k_spec_block<float><<<count, 256, 0, st>>>(list, count, fd, prm, ws, wsOff);
     hipCheck(hipGetLastError(), "k_spec_block");
-    k_spec_factor<float><<<blocks, kSpecRows, 0, st>>>(list, count, wgStart, parity, fd, prm, ws, wsOff);
+    k_spec_factor<float><<<blocks, 4 * kSpecRows, 0, st>>>(list, count, wgStart, parity, fd, prm, ws, wsOff);
     hipCheck(hipGetLastError(), "k_spec_factor");
-    k_spec_apply<float><<<blocks, kSpecRows, 0, st>>>(list, count, wgStart, parity, fd, prm, ws, wsOff);
+    k_spec_apply<float><<<blocks, kSpecApplyThreads, 0, st>>>(list, count, wgStart, parity, fd, prm, ws, wsOff);
   } else {
     k_spec_block<double><<<count, 256, 0, st>>>(list, count, fd, prm, ws, wsOff);
     hipCheck(hipGetLastError(), "k_spec_block");
-    k_spec_factor<double><<<blocks, kSpecRows, 0, st>>>(list, count, wgStart, parity, fd, prm, ws, wsOff);
+    k_spec_factor<double><<<blocks, 4 * kSpecRows, 0, st>>>(list, count, wgStart, parity, fd, prm, ws, wsOff);
     hipCheck(hipGetLastError(), "k_spec_factor");
-    k_spec_apply<double><<<blocks, kSpecRows, 0, st>>>(list, count, wgStart, parity, fd, prm, ws, wsOff);
+    k_spec_apply<double><<<blocks, kSpecApplyThreads, 0, st>>>(list, count, wgStart, parity, fd, prm, ws, wsOff);
   }
   hipCheck(hipGetLastError(), "launchSpecPanel");
 }

@@ -563,7 +563,10 @@ LargeSched buildLargeSched(const std::vector<int>& fronts, const std::vector<int
       if (!all) rb += (m[s] - nE[s] + kPanelRowsWg - 1) / kPanelRowsWg;
       // rows below this iteration's diagonal block (the block starts at or after it * kPanel)
       const int below = m[s] - it * kPanel - std::min(kPanel, nE[s] - it * kPanel);
-      if (spec) sb += std::max(1, (below + kSpecRows - 1) / kSpecRows);
+      if (spec) {
+        ++li.specCount;
+        sb += std::max(1, (below + kSpecRows - 1) / kSpecRows);
+      }
       // trailing tiles: T per side from this iteration's panel start, column
       // blocks up to the cut
       const int T = (m[s] - it * kPanel + 63) / 64;
@@ -628,12 +631,16 @@ void runLargeSched(const LargeSched& ls, const LargeDev& dv, const DevFronts& fd
     if (prm.specPanel && it.specBlocks > 0)
       launchSpecPanel(lst, it.count, dv.specStart + it.specOff, it.specBlocks, static_cast<int>(t & 1), fd, prm, ws,
                       wsOff, st);
-    launchPanel(dv.lists + it.regOff, it.regCount, it.regMaxRows, fd, prm, ws, wsOff, st);
-    launchPanel(dv.lists + it.bigOff, it.bigCount, it.bigMaxRows, fd, prm, ws, wsOff, st);
-    launchPanelMw(dv.lists + it.mwOff, it.mwCount, dv.mwStart + it.mwStartOff, it.mwBlocks, fd, prm, ws, wsOff,
-                  dv.sync, dv.err, st);
+    // static pivots are always taken: nothing is left for the exact panels then
+    const bool exact = !(prm.staticMode && it.specCount == it.count);
+    if (exact) {
+      launchPanel(dv.lists + it.regOff, it.regCount, it.regMaxRows, fd, prm, ws, wsOff, st);
+      launchPanel(dv.lists + it.bigOff, it.bigCount, it.bigMaxRows, fd, prm, ws, wsOff, st);
+      launchPanelMw(dv.lists + it.mwOff, it.mwCount, dv.mwStart + it.mwStartOff, it.mwBlocks, fd, prm, ws, wsOff,
+                    dv.sync, dv.err, st);
+    }
     if (prof) prof->profEnd(Plan::kProfPanel);
-    if (it.rowBlocks > 0) {
+    if (exact && it.rowBlocks > 0) {
       if (prof) prof->profBegin(Plan::kProfPanelRows);
       launchPanelRows(lst, it.count, dv.rowStart + it.rowOff, it.rowBlocks, fd, st);
       if (prof) prof->profEnd(Plan::kProfPanelRows);

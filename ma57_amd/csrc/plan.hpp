@@ -113,6 +113,7 @@ constexpr int kMwMaxBlocks = 240;  // cooperative workgroups per launch (all res
 struct LargeIter {
   int64_t listOff = 0;  // all fronts of the iteration (rows, trailing update)
   int count = 0;
+  int specCount = 0;    // those that take the speculative step
   int64_t rowOff = 0;
   int rowBlocks = 0;
   int64_t tileOff = 0;
