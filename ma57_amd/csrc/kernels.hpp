@@ -66,8 +66,12 @@ void launchFwdGather(const PosInfo* info, int64_t positions, int nrhs, const dou
 constexpr int kSolveBlock = 32;
 void launchDiagInverse(const int* list, int count, const int* blockStart, int blocks, const DevFronts& fd,
                        double* inv, const int64_t* invOff, hipStream_t st);
-// own rows, one workgroup per front (a short chain of own blocks)
-void launchFwdOwn(const int* list, int count, const DevFronts& fd, int nrhs, double* Z, double* Dl,
+// own rows, one workgroup per front (a short chain of own blocks, at most
+// maxBlocks <= kOwnMaxBlocks in a listed front): its products grow with the
+// square of the blocks (a chain of 10 took 83 us there, 50 with a workgroup
+// per block and flags between them)
+constexpr int kOwnMaxBlocks = 6;
+void launchFwdOwn(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* Z, double* Dl,
                   const int64_t* gOff, const double* inv, const int64_t* invOff, hipStream_t st);
 // own rows, one workgroup per own block (blockStart: ceil(nF / kSolveBlock) per front), dependency flags
 void launchFwdChain(const int* list, int count, const int* blockStart, int blocks, const DevFronts& fd, int nrhs,
@@ -80,7 +84,8 @@ void launchFwdDelta(const int* list, int count, const int* blockStart, int block
 void launchBwdAnc(const int* list, int count, const int* blockStart, int blocks, const DevFronts& fd, int nrhs,
                   const double* Z, const double* X, double* Dl, const int64_t* gOff, const AncPart* parts, int* err,
                   hipStream_t st);
-void launchBwdOwn(const int* list, int count, const DevFronts& fd, int nrhs, double* X, double* Dl,
+void launchBwdOwn(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* X,
+                  const double* Dl,
                   const int64_t* gOff, const AncPart* parts, const double* inv, const int64_t* invOff,
                   hipStream_t st);
 void launchBwdChain(const int* list, int count, const int* blockStart, int blocks, const DevFronts& fd, int nrhs,

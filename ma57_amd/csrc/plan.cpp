@@ -1127,7 +1127,7 @@ void Plan::ensureSolveLayout() {
           continue;
         }
         anc.push_back(s);
-        if ((nfs + kSolveBlock - 1) / kSolveBlock <= kOwnChainBlocks)
+        if ((nfs + kSolveBlock - 1) / kSolveBlock <= kOwnMaxBlocks)
           own.push_back(s);
         else
           chain.push_back(s);
@@ -1154,6 +1154,7 @@ void Plan::ensureSolveLayout() {
         partRows += static_cast<int64_t>(split - 1) * pa.stride;
       }
       addLaunch(lv.own, own, [](int) { return 1; });
+      for (int s : own) lv.own.maxBlocks = std::max(lv.own.maxBlocks, ownBlocks(s));
       addLaunch(lv.chain, chain, ownBlocks);
       addLaunch(lv.delta, delta, [&](int s) { return (hm_[s] - nfOf(s) + 63) / 64; });
       addLaunch(lv.anc, anc, [&](int s) { return ownBlocks(s) * parts[s].split; });
@@ -1218,7 +1219,7 @@ void Plan::solveCore(const double* dB, int64_t ldb, int nrhs, double* dX, int64_
     const SolveLevel& lv = solveLv_[L];
     profBegin(kProfFwd);
     launchFwdGather(dposInfo_.p + lv.posOff, lv.positions, nrhs, w.Bp, w.Dl, dmapRow_.p, stream_);
-    launchFwdOwn(lists + lv.own.list, lv.own.count, fd, nrhs, w.Z, w.Dl, dgOff_.p, dinv_.p, dinvOff_.p, stream_);
+    launchFwdOwn(lists + lv.own.list, lv.own.count, lv.own.maxBlocks, fd, nrhs, w.Z, w.Dl, dgOff_.p, dinv_.p, dinvOff_.p, stream_);
     launchFwdChain(lists + lv.chain.list, lv.chain.count, starts + lv.chain.start, lv.chain.blocks, fd, nrhs, w.Z,
                    w.Dl, dgOff_.p, dflagsF_.p, dflagOff_.p, dgen_.p, err, dinv_.p, dinvOff_.p, stream_);
     launchFwdDelta(lists + lv.delta.list, lv.delta.count, starts + lv.delta.start, lv.delta.blocks, fd, nrhs, w.Dl,
@@ -1231,7 +1232,7 @@ void Plan::solveCore(const double* dB, int64_t ldb, int nrhs, double* dX, int64_
     profBegin(kProfBwd);
     launchBwdAnc(lists + lv.anc.list, lv.anc.count, starts + lv.anc.start, lv.anc.blocks, fd, nrhs, w.Z, w.X, w.Dl,
                  dgOff_.p, dancPart_.p, err, stream_);
-    launchBwdOwn(lists + lv.own.list, lv.own.count, fd, nrhs, w.X, w.Dl, dgOff_.p, dancPart_.p, dinv_.p, dinvOff_.p,
+    launchBwdOwn(lists + lv.own.list, lv.own.count, lv.own.maxBlocks, fd, nrhs, w.X, w.Dl, dgOff_.p, dancPart_.p, dinv_.p, dinvOff_.p,
                  stream_);
     launchBwdChain(lists + lv.chain.list, lv.chain.count, starts + lv.chain.start, lv.chain.blocks, fd, nrhs, w.X,
                    w.Dl, dgOff_.p, dancPart_.p, dflagsB_.p, dflagOff_.p, dgen_.p, err, dinv_.p, dinvOff_.p,

@@ -139,9 +139,6 @@ struct LargeIter {
 constexpr int kCbMinCols = 256;
 constexpr int kCbMinRowsDefault = 2048;
 constexpr int kCbChunk = 2048;
-// fronts with at most this many 32-row own blocks solve their own rows on
-// one workgroup; longer chains take one workgroup per block
-constexpr int kOwnChainBlocks = 10;
 // the backward ancestors' product: chunks of at least this many rows, split
 // until a level has about kAncLevelBlocks workgroups, at most kAncMaxSplit
 constexpr int kAncChunkRows = 512;
@@ -402,6 +399,7 @@ class Plan {
   struct SolveLaunch {
     int64_t list = 0, start = 0;
     int count = 0, blocks = 0;
+    int maxBlocks = 0;  // own: most own blocks of a listed front
   };
   struct SolveLevel {
     int64_t posOff = 0, positions = 0;

@@ -71,6 +71,17 @@ constexpr int YW = 65;           // row stride of the right-hand-side tiles in L
 // Polls of a dependency flag before a chain block gives up (about a second).
 constexpr unsigned kSpinLimit = 1u << 22;
 
+// A front pointer read from the front table is generic; a generic (flat) load
+// may be an LDS access, so the compiler can only wait for all of them (and for
+// the LDS) at once.  Front storage is global memory: this view makes the loads
+// global ones, each waited for at its own use.
+template <typename T>
+using GlobalIn = const __attribute__((address_space(1))) T*;
+template <typename T>
+__device__ inline GlobalIn<T> globalIn(const T* p) {
+  return (GlobalIn<T>)(p);
+}
+
 // Front owning flat item b: start[f] <= b < start[f+1].
 template <typename I>
 __device__ inline int segmentOf(const I* start, int count, I b) {
@@ -135,8 +146,8 @@ __device__ inline void publishBlock(unsigned* f, unsigned gen) {
 
 // L(row, col) of a front with the (s+1, s) slot of a 2x2 pivot block read as
 // zero: that slot stores d21, not a multiplier (multifrontal.hpp:618-628).
-template <typename T>
-__device__ inline double lval(const T* F, int m, const int* pk, int row, int col) {
+template <typename P>
+__device__ inline double lval(P F, int m, const int* pk, int row, int col) {
   const double v = F[row + static_cast<size_t>(col) * m];
   return (row == col + 1 && pk[col] == 2) ? 0.0 : v;
 }
@@ -145,13 +156,13 @@ __device__ inline double lval(const T* F, int m, const int* pk, int row, int col
 // the block's first element (a valid address) is read and zero returned.  A
 // load under a branch completes before the branch joins, so conditional
 // loads would wait for one another; these are issued back to back.
-template <typename T>
-__device__ inline T ldOr0(const T* base, int64_t off, bool ok) {
-  const T v = base[ok ? off : 0];
-  return ok ? v : T(0);
+template <typename P>
+__device__ inline auto ldOr0(P base, int64_t off, bool ok) {
+  const auto v = +base[ok ? off : 0];
+  return ok ? v : decltype(v)(0);
 }
-template <typename T>
-__device__ inline double lvalOr0(const T* F, int m, const int* pk, int row, int col, bool ok) {
+template <typename P>
+__device__ inline double lvalOr0(P F, int m, const int* pk, int row, int col, bool ok) {
   const int r = ok ? row : 0, c = ok ? col : 0;
   const double v = F[r + static_cast<size_t>(c) * m];
   const int k = pk[c];
@@ -238,31 +249,13 @@ struct BlockLds {
   int pkA[SB + 1], rixA[SB + 1];  // their pivot kinds and final-order rows
 };
 
-// Work block rows of other blocks: read back by the workgroup that wrote
-// them (kShared false: ordered by its barriers) or published by another
-// workgroup of the launch (kShared true: device-coherent).
-template <bool kShared>
-__device__ inline double readRow(const double* p) {
-  if constexpr (kShared)
-    return loadShared(p);
-  else
-    return *p;
-}
-template <bool kShared>
-__device__ inline void writeRow(double* p, double v) {
-  if constexpr (kShared)
-    storeShared(p, v);
-  else
-    *p = v;
-}
-
 // Forward step of own block b of front s for right-hand sides rg .. rg + gw
 // (solve.hpp:349-361, :434-455): y_b = Ltop(b, b)^{-1} (y0_b - sum_{j<b}
 // L(b, j) y_j), y0_b in the block's work rows (from the gather), y_b written
 // over it, and z = D^{-1} y of the pivot blocks that end in this block into
-// Z.  With kShared the y_j come from other workgroups, waited for by flag
-// (on the first right-hand-side group only), and y_b is published when done.
-template <typename T, bool kShared>
+// Z.  The y_j come from other workgroups, waited for by flag (on the first
+// right-hand-side group only), and y_b is published when done.
+template <typename T>
 __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFronts& fd, int s, int b, int rg,
                             int gw, int nrhs, double* __restrict__ Z, double* Ds, const double* __restrict__ Mi,
                             unsigned* fl, unsigned gen, int* err, bool publish) {
@@ -274,7 +267,7 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
   const int nf = fd.nF[s];
   const int64_t io = fd.idxOff[s];
   const int* pk = fd.pkind + io;
-  const T* F = static_cast<const T*>(fd.F[s]);
+  const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
   const int r0 = b * SB, nr = min(SB, nf - r0);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   // wave wv owns output rows tr .. tr + 15 and right-hand sides tc .. tc + 31
@@ -311,7 +304,7 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
   double acc[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};  // FP64 sums of the per-tile products
   if (b > 0) loadL(0);
   for (int j = 0; j < b; ++j) {
-    if (kShared && rg == 0) waitBlock(fl + j, gen, err);
+    if (rg == 0) waitBlock(fl + j, gen, err);
     const int c0 = j * SB, cn = min(SB, nf - c0);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -321,7 +314,7 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
     for (int e = tid; e < SB * 64; e += NT) {
       const int c = e & 63, qq = e >> 6;
       const bool ok = qq < cn && c < gw;
-      const double v = readRow<kShared>(Ds + (ok ? static_cast<int64_t>(c0 + qq) * nrhs + rg + c : 0));
+      const double v = loadShared(Ds + (ok ? static_cast<int64_t>(c0 + qq) * nrhs + rg + c : 0));
       S.yt[qq][c] = ok ? static_cast<E>(v) : E(0);
     }
     if (j + 1 < b) loadL(j + 1);
@@ -365,13 +358,13 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
         const int r = tr + MD::row(lane, rr), c = tc + 16 * t + lr;
         if (r < nr && c < gw) {
           S.ys[r][c] = yv[t][rr];
-          writeRow<kShared>(Ds + static_cast<int64_t>(r0 + r) * nrhs + rg + c, yv[t][rr]);
+          storeShared(Ds + static_cast<int64_t>(r0 + r) * nrhs + rg + c, yv[t][rr]);
         }
       }
   }
   __syncthreads();
   // the later blocks need y only: release it before forming z
-  if (kShared && publish) publishBlock(fl + b, gen);
+  if (publish) publishBlock(fl + b, gen);
   // z = D^{-1} y for the pivot blocks that end in this block (slot r + 1 of
   // the staged pivot data is position r0 + r)
   for (int e = tid; e < nr * gw; e += NT) {
@@ -391,7 +384,7 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
       // second row of a 2x2 block that starts in the previous block
       const double d11 = S.dA[0], d21 = S.dB[0], d22 = S.dA[1];
       const double det = d11 * d22 - d21 * d21;
-      const double y0 = readRow<kShared>(Ds + static_cast<int64_t>(p - 1) * nrhs + cc), y1 = S.ys[0][c];
+      const double y0 = loadShared(Ds + static_cast<int64_t>(p - 1) * nrhs + cc), y1 = S.ys[0][c];
       Z[static_cast<int64_t>(S.rixA[0]) * nrhs + cc] = (d22 * y0 - d21 * y1) / det;
       Z[static_cast<int64_t>(S.rixA[1]) * nrhs + cc] = (-d21 * y0 + d11 * y1) / det;
     }
@@ -402,7 +395,7 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
 // Backward step of own block w of front s (solve.hpp:364-383): x_w =
 // Ltop(w, w)^{-T} (P_w - sum_{j>w} L(j, w)^T x_j), P_w (z less the
 // ancestors' part) in the block's work rows, x_w written over it and into X.
-template <typename T, bool kShared>
+template <typename T>
 __device__ void bwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFronts& fd, int s, int w, int rg,
                             int gw, int nrhs, double* __restrict__ X, double* Ds, const double* __restrict__ Dl,
                             const AncPart pa, const double* __restrict__ Mi, unsigned* fl, unsigned gen, int* err,
@@ -416,7 +409,7 @@ __device__ void bwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
   const int nOwn = (nf + SB - 1) / SB;
   const int64_t io = fd.idxOff[s];
   const int* pk = fd.pkind + io;
-  const T* F = static_cast<const T*>(fd.F[s]);
+  const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
   const int r0 = w * SB, nr = min(SB, nf - r0);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   // wave wv owns own columns tr .. tr + 15 and right-hand sides tc .. tc + 31
@@ -451,7 +444,7 @@ __device__ void bwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
   double acc[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
   if (nOwn - 1 > w) loadO(nOwn - 1);
   for (int j = nOwn - 1; j > w; --j) {
-    if (kShared && rg == 0) waitBlock(fl + j, gen, err);
+    if (rg == 0) waitBlock(fl + j, gen, err);
     const int i0 = j * SB, in = min(SB, nf - i0);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -461,7 +454,7 @@ __device__ void bwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
     for (int e = tid; e < SB * 64; e += NT) {
       const int c = e & 63, i = e >> 6;
       const bool ok = i < in && c < gw;
-      const double v = readRow<kShared>(Ds + (ok ? static_cast<int64_t>(i0 + i) * nrhs + rg + c : 0));
+      const double v = loadShared(Ds + (ok ? static_cast<int64_t>(i0 + i) * nrhs + rg + c : 0));
       S.yt[i][c] = ok ? static_cast<E>(v) : E(0);
     }
     if (j - 1 > w) loadO(j - 1);
@@ -504,13 +497,13 @@ __device__ void bwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
         const int qq = tr + MD::row(lane, rr), c = tc + 16 * t + lr;
         if (qq < nr && c < gw) {
           S.ys[qq][c] = xv[t][rr];
-          writeRow<kShared>(Ds + static_cast<int64_t>(r0 + qq) * nrhs + rg + c, xv[t][rr]);
+          storeShared(Ds + static_cast<int64_t>(r0 + qq) * nrhs + rg + c, xv[t][rr]);
         }
       }
   }
   __syncthreads();
   // the earlier blocks need x only through the work block: release it, then write X
-  if (kShared && publish) publishBlock(fl + w, gen);
+  if (publish) publishBlock(fl + w, gen);
   for (int e = tid; e < nr * gw; e += NT) {
     const int c = e % gw, r = e / gw;
     X[static_cast<int64_t>(S.rixA[r]) * nrhs + rg + c] = S.ys[r][c];
@@ -611,7 +604,7 @@ __global__ __launch_bounds__(64) void k_diag_inverse(const int* list, int count,
   const int nr = min(SB, nf - r0);
   const int64_t io = fd.idxOff[s];
   const int* pk = fd.pkind + io;
-  const T* F = static_cast<const T*>(fd.F[s]);
+  const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
   const int tid = threadIdx.x;
   for (int e = tid; e < SB * SB; e += 64) {
     const int r = e % SB, c = e / SB;
@@ -637,25 +630,297 @@ __global__ __launch_bounds__(64) void k_diag_inverse(const int* list, int count,
   for (int e = tid; e < SB * SB; e += 64) out[e] = Ms[e / SB][e % SB];
 }
 
-// Forward own rows of fronts with a short own-row chain: one workgroup per
-// front runs the blocks b = 0, 1, ... in order, reading the y_j it has
-// written back from the work block (its own barriers order those stores and
-// loads), so no block waits on another workgroup.
-template <typename T>
+// Own rows of fronts with a short own-row chain: one workgroup per front, one
+// wave per 16 right-hand sides, which runs the whole chain in registers.  A
+// 32-row block of right-hand sides is two FP64 MFMA results (lane j + 16 c,
+// register s of half h: row 16 h + 4 s + c, right-hand side j), which is also
+// the layout of the instruction's second operand when its step s takes the
+// rows 4 s .. 4 s + 3: a solved block feeds the products with the later
+// blocks from its own registers, and L and the inverted diagonal blocks are
+// read from memory in the first operand's order, ahead of the chain.  No LDS,
+// no barrier, no wave waits for another.  Products are FP64 for FP32 fronts
+// too (the chain's latency is in the loads and the dependent products).
+//
+// Measured (40^3 7-point, FP64, one right-hand side, a launch per level, up
+// to 6 blocks): forward 36 -> 20 us, backward 36 -> 18; 53x57x59 27-point,
+// FP32, 33 right-hand sides: 97 -> 46 and 116 -> 35 (blocks through LDS, four
+// waves and four barriers per product before).
+typedef double v4d __attribute__((ext_vector_type(4)));
+__device__ inline v4d ownMma(double a, double b, v4d c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+// An FP64 16x16x4 product's result before a branch: the compiler may count a
+// read's distance from it along the longer way only (20 wait states cover it).
+__device__ inline void ownSettle(v4d& x) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x)); }
+
+// NB: most own blocks of a listed front.  Forward (solve.hpp:349-361,
+// :434-455): y_b = L_bb^{-1} (y0_b - sum_{j<b} L_bj y_j), then z = D^{-1} y.
+template <typename T, int NB>
 __global__ __launch_bounds__(256) void k_fwd_own(const int* list, int count, DevFronts fd, int nrhs,
                                                  double* __restrict__ Z, double* __restrict__ Dl,
                                                  const int64_t* __restrict__ gOff, const double* __restrict__ inv,
                                                  const int64_t* __restrict__ invOff) {
-  __shared__ BlockLds<typename SweepMfma<T>::E> S;
   if (static_cast<int>(blockIdx.x) >= count) return;
   const int s = list[blockIdx.x];
-  const int nOwn = (fd.nF[s] + SB - 1) / SB;
+  const int m = fd.m[s], nf = fd.nF[s];
+  const int nOwn = (nf + SB - 1) / SB;
+  const int64_t io = fd.idxOff[s];
+  const int* pk = fd.pkind + io;
+  const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
+  const GlobalIn<double> Mi = globalIn(inv + invOff[s]);
   double* Ds = Dl + gOff[s] * nrhs;
-  for (int rg = 0; rg < nrhs; rg += 64) {
-    const int gw = min(64, nrhs - rg);
-    for (int b = 0; b < nOwn; ++b)
-      fwdOwnBlock<T, false>(S, fd, s, b, rg, gw, nrhs, Z, Ds, inv + invOff[s] + static_cast<int64_t>(b) * SB * SB,
-                            nullptr, 0u, nullptr, false);
+  const GlobalIn<double> Dr = globalIn(static_cast<const double*>(Ds));
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int c0 = 16 * wv; c0 < nrhs; c0 += 16 * (blockDim.x >> 6)) {
+    const int j = c0 + lr;
+    const bool jn = j < nrhs;
+    // operands of a step, loaded ahead of it
+    auto loadInv = [&](int b, double (&mi)[2][8], double (&y0)[2][4], int& k2) {
+      const int bb = min(b, nOwn - 1);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) mi[h][u] = Mi[bb * SB * SB + (16 * h + lr) * SB + 4 * u + lk];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int r = SB * bb + 16 * h + 4 * u + lk;
+          y0[h][u] = Dr[r < nf && jn ? static_cast<int64_t>(r) * nrhs + j : 0];
+        }
+      }
+      k2 = pk[min(SB * bb + SB - 1, nf - 1)];  // a 2x2 pivot across the next block's start: its slot of L holds d21
+    };
+    auto loadTile = [&](int b, int jb, T (&a)[2][8]) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int r = SB * b + 16 * h + lr, c = SB * jb + 4 * u + lk;
+          a[h][u] = F[r < nf && c < nf ? r + static_cast<int64_t>(c) * m : 0];
+        }
+    };
+    v4d acc[NB][2];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) acc[t][0] = acc[t][1] = v4d{0.0, 0.0, 0.0, 0.0};
+    double mi[2][8], y0[2][4];
+    T a[2][8], an[2][8];
+    int k2 = 1;
+    if (nOwn > 0) {
+      loadInv(0, mi, y0, k2);
+      if (NB > 1 && nOwn > 1) loadTile(1, 0, a);
+    }
+    for (int b = 0; b < nOwn; ++b) {
+      v4d r[2], y[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          r[h][u] = SB * b + 16 * h + 4 * u + lk < nf && jn ? y0[h][u] - acc[0][h][u] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        if (u < 4) y[0] = ownMma(mi[0][u], r[u >> 2][u & 3], y[0]);  // the inverse is lower triangular
+        y[1] = ownMma(mi[1][u], r[u >> 2][u & 3], y[1]);
+      }
+      ownSettle(y[0]);
+      ownSettle(y[1]);
+      const bool corner = k2 == 2;
+      if (b + 1 < nOwn) loadInv(b + 1, mi, y0, k2);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int row = SB * b + 16 * h + 4 * u + lk;
+          if (row < nf && jn) Ds[static_cast<int64_t>(row) * nrhs + j] = y[h][u];
+        }
+#pragma unroll
+      for (int t = 1; t < NB; ++t) {
+        if (b + t < nOwn) {
+          if (b + t + 1 < nOwn)
+            loadTile(b + t + 1, b, an);
+          else if (b + 2 < nOwn)
+            loadTile(b + 2, b + 1, an);  // the next step's first tile
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const bool d21 = t == 1 && h == 0 && u == 7 && lr == 0 && lk == 3 && corner;
+              acc[t][h] = ownMma(d21 ? 0.0 : static_cast<double>(a[h][u]), y[u >> 2][u & 3], acc[t][h]);
+            }
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            ownSettle(acc[t][h]);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a[h][u] = an[h][u];
+          }
+        }
+      }
+#pragma unroll
+      for (int t = 1; t < NB; ++t) {
+        acc[t - 1][0] = acc[t][0];
+        acc[t - 1][1] = acc[t][1];
+      }
+    }
+    // z = D^{-1} y, four rows per 16 lanes, from the rows just written
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    const int jc = min(j, nrhs - 1);
+    for (int p0 = 0; p0 < nf; p0 += 16) {
+      int kind[4], row[4];
+      double d[4], dn[4], dp[4], on[4], op[4], yc[4], yn[4], yp[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int pc = min(p0 + 4 * u + lk, nf - 1), pn = min(pc + 1, nf - 1), pp = max(pc - 1, 0);
+        kind[u] = pk[pc];
+        row[u] = fd.rowIdx[io + pc];
+        d[u] = fd.dDiag[io + pc];
+        dn[u] = fd.dDiag[io + pn];
+        dp[u] = fd.dDiag[io + pp];
+        on[u] = fd.dOff[io + pc];
+        op[u] = fd.dOff[io + pp];
+        yc[u] = Dr[static_cast<int64_t>(pc) * nrhs + jc];
+        yn[u] = Dr[static_cast<int64_t>(pn) * nrhs + jc];
+        yp[u] = Dr[static_cast<int64_t>(pp) * nrhs + jc];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        // the other row of a 2x2 pivot: the next one (kind 2) or the previous
+        const double dq = kind[u] == 2 ? dn[u] : dp[u], of = kind[u] == 2 ? on[u] : op[u];
+        const double yq = kind[u] == 2 ? yn[u] : yp[u];
+        const double num = kind[u] == 1 ? yc[u] : dq * yc[u] - of * yq;
+        const double den = kind[u] == 1 ? d[u] : d[u] * dq - of * of;
+        if (p0 + 4 * u + lk < nf && jn) Z[static_cast<int64_t>(row[u]) * nrhs + j] = num / den;
+      }
+    }
+  }
+}
+
+// Backward (solve.hpp:364-383): x_w = L_ww^{-T} (P_w - sum_{j>w} L_jw^T x_j),
+// P_w (z less the ancestors' part) in the front's work rows.
+template <typename T, int NB>
+__global__ __launch_bounds__(256) void k_bwd_own(const int* list, int count, DevFronts fd, int nrhs,
+                                                 double* __restrict__ X, const double* __restrict__ Dl,
+                                                 const int64_t* __restrict__ gOff, const AncPart* __restrict__ parts,
+                                                 const double* __restrict__ inv, const int64_t* __restrict__ invOff) {
+  if (static_cast<int>(blockIdx.x) >= count) return;
+  const int s = list[blockIdx.x];
+  const int m = fd.m[s], nf = fd.nF[s];
+  const int nOwn = (nf + SB - 1) / SB;
+  const int64_t io = fd.idxOff[s];
+  const int* pk = fd.pkind + io;
+  const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
+  const GlobalIn<double> Mi = globalIn(inv + invOff[s]);
+  const GlobalIn<double> Dr = globalIn(Dl + gOff[s] * nrhs), Dp = globalIn(Dl);
+  const AncPart pa = parts[s];
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int c0 = 16 * wv; c0 < nrhs; c0 += 16 * (blockDim.x >> 6)) {
+    const int j = c0 + lr;
+    const bool jn = j < nrhs;
+    auto loadInv = [&](int w, double (&mi)[2][8], double (&p0)[2][4], int (&rix)[2][4], int& k2) {
+      const int ww = max(w, 0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) mi[h][u] = Mi[ww * SB * SB + (4 * u + lk) * SB + 16 * h + lr];  // transposed
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int r = SB * ww + 16 * h + 4 * u + lk;
+          p0[h][u] = Dr[r < nf && jn ? static_cast<int64_t>(r) * nrhs + j : 0];
+          rix[h][u] = fd.rowIdx[io + min(r, nf - 1)];
+        }
+      }
+      k2 = pk[max(SB * ww - 1, 0)];
+    };
+    // L(w, jb)^T: the tile's rows are the product's inner dimension
+    auto loadTile = [&](int w, int jb, T (&a)[2][8]) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int r = SB * w + 4 * u + lk, c = SB * jb + 16 * h + lr;
+          a[h][u] = F[r < nf && c < nf ? r + static_cast<int64_t>(c) * m : 0];
+        }
+    };
+    v4d acc[NB][2];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) acc[t][0] = acc[t][1] = v4d{0.0, 0.0, 0.0, 0.0};
+    double mi[2][8], p0[2][4];
+    int rix[2][4], rixn[2][4];
+    T a[2][8], an[2][8];
+    int k2 = 1;
+    if (nOwn > 0) {
+      loadInv(nOwn - 1, mi, p0, rix, k2);
+      if (NB > 1 && nOwn > 1) loadTile(nOwn - 1, nOwn - 2, a);
+    }
+    for (int w = nOwn - 1; w >= 0; --w) {
+      // the other chunks of the ancestors' product, in chunk order
+      for (int k0 = 1; k0 < pa.split; k0 += 4) {
+        double part[4][2][4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int r = SB * w + 16 * h + 4 * u + lk;
+              part[k][h][u] = Dp[r < nf && jn && k0 + k < pa.split
+                                     ? (pa.off + static_cast<int64_t>(k0 + k - 1) * pa.stride + r) * nrhs + j
+                                     : 0];
+            }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) p0[h][u] -= k0 + k < pa.split ? part[k][h][u] : 0.0;
+      }
+      v4d r[2], x[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          r[h][u] = SB * w + 16 * h + 4 * u + lk < nf && jn ? p0[h][u] - acc[0][h][u] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        x[0] = ownMma(mi[0][u], r[u >> 2][u & 3], x[0]);
+        if (u >= 4) x[1] = ownMma(mi[1][u], r[u >> 2][u & 3], x[1]);  // the transposed inverse is upper triangular
+      }
+      ownSettle(x[0]);
+      ownSettle(x[1]);
+      const bool corner = k2 == 2;
+      if (w > 0) loadInv(w - 1, mi, p0, rixn, k2);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (SB * w + 16 * h + 4 * u + lk < nf && jn) X[static_cast<int64_t>(rix[h][u]) * nrhs + j] = x[h][u];
+          rix[h][u] = rixn[h][u];
+        }
+#pragma unroll
+      for (int t = 1; t < NB; ++t) {
+        if (w - t >= 0) {
+          if (w - t - 1 >= 0)
+            loadTile(w, w - t - 1, an);
+          else if (w >= 2)
+            loadTile(w - 1, w - 2, an);
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const bool d21 = t == 1 && h == 1 && u == 0 && lr == 15 && lk == 0 && corner;
+              acc[t][h] = ownMma(d21 ? 0.0 : static_cast<double>(a[h][u]), x[u >> 2][u & 3], acc[t][h]);
+            }
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            ownSettle(acc[t][h]);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a[h][u] = an[h][u];
+          }
+        }
+      }
+#pragma unroll
+      for (int t = 1; t < NB; ++t) {
+        acc[t - 1][0] = acc[t][0];
+        acc[t - 1][1] = acc[t][1];
+      }
+    }
   }
 }
 
@@ -683,7 +948,7 @@ __global__ __launch_bounds__(256) void k_fwd_chain(const int* list, int count, c
   double* Ds = Dl + gOff[s] * nrhs;
   for (int rg = 0; rg < nrhs; rg += 64) {
     const int gw = min(64, nrhs - rg);
-    fwdOwnBlock<T, true>(S, fd, s, b, rg, gw, nrhs, Z, Ds, inv + invOff[s] + static_cast<int64_t>(b) * SB * SB,
+    fwdOwnBlock<T>(S, fd, s, b, rg, gw, nrhs, Z, Ds, inv + invOff[s] + static_cast<int64_t>(b) * SB * SB,
                          flags + flagOff[s], gen, err, rg + 64 >= nrhs);
   }
 }
@@ -707,7 +972,7 @@ __device__ void fwdDeltaChunk(DeltaLds<typename SweepMfma<T>::E>& S, const DevFr
   const int m = fd.m[s];
   const int nf = fd.nF[s];
   const int i0 = nf + b * DT, ni = min(DT, m - i0);
-  const T* F = static_cast<const T*>(fd.F[s]);
+  const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32;
   const int lr = lane & 15, lk = lane >> 4;
@@ -819,7 +1084,7 @@ __device__ void bwdAncChunk(AncLds<typename SweepMfma<T>::E>& S, const DevFronts
   const int chunk = ((m - nf + pa.split - 1) / pa.split + DT - 1) / DT * DT;
   const int a0 = nf + k * chunk, a1 = min(m, a0 + chunk);
   const int64_t io = fd.idxOff[s];
-  const T* F = static_cast<const T*>(fd.F[s]);
+  const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int wu = __builtin_amdgcn_readfirstlane(wv);
   const int tr = (wv & 1) * 16, tc = (wv >> 1) * 32;
@@ -920,27 +1185,6 @@ __global__ __launch_bounds__(256) void k_bwd_anc(const int* list, int count, con
   bwdAncChunk<T>(S, fd, s, w, k, pa, nrhs, Z, X, Dl, Dl + gOff[s] * nrhs);
 }
 
-// Backward own rows of fronts with a short own-row chain: one workgroup per
-// front, blocks w = nOwn - 1 .. 0 in order, the x_j read back from the work
-// block this workgroup wrote.
-template <typename T>
-__global__ __launch_bounds__(256) void k_bwd_own(const int* list, int count, DevFronts fd, int nrhs,
-                                                 double* __restrict__ X, double* __restrict__ Dl,
-                                                 const int64_t* __restrict__ gOff, const AncPart* __restrict__ parts,
-                                                 const double* __restrict__ inv, const int64_t* __restrict__ invOff) {
-  __shared__ BlockLds<typename SweepMfma<T>::E> S;
-  if (static_cast<int>(blockIdx.x) >= count) return;
-  const int s = list[blockIdx.x];
-  const int nOwn = (fd.nF[s] + SB - 1) / SB;
-  double* Ds = Dl + gOff[s] * nrhs;
-  for (int rg = 0; rg < nrhs; rg += 64) {
-    const int gw = min(64, nrhs - rg);
-    for (int w = nOwn - 1; w >= 0; --w)
-      bwdOwnBlock<T, false>(S, fd, s, w, rg, gw, nrhs, X, Ds, Dl, parts[s],
-                            inv + invOff[s] + static_cast<int64_t>(w) * SB * SB, nullptr, 0u, nullptr, false);
-  }
-}
-
 // Backward own rows of fronts with a long own-row chain: one workgroup per
 // own block, taken from the last block to the first; block w waits for the
 // blocks j > w of its front (dispatched before it).
@@ -965,7 +1209,7 @@ __global__ __launch_bounds__(256) void k_bwd_chain(const int* list, int count, c
   double* Ds = Dl + gOff[s] * nrhs;
   for (int rg = 0; rg < nrhs; rg += 64) {
     const int gw = min(64, nrhs - rg);
-    bwdOwnBlock<T, true>(S, fd, s, w, rg, gw, nrhs, X, Ds, Dl, parts[s],
+    bwdOwnBlock<T>(S, fd, s, w, rg, gw, nrhs, X, Ds, Dl, parts[s],
                          inv + invOff[s] + static_cast<int64_t>(w) * SB * SB, flags + flagOff[s], gen, err,
                          rg + 64 >= nrhs);
   }
@@ -998,7 +1242,7 @@ __global__ __launch_bounds__(256) void k_fwd_tiny(const int* list, int count, De
   const int nf = fd.nF[s];
   const int64_t io = fd.idxOff[s];
   const int* pk = fd.pkind + io;
-  const T* F = static_cast<const T*>(fd.F[s]);
+  const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
   double* Dr = Dl + (gOff[s] + lane) * nrhs;  // this lane's work row
   const bool row = lane < m;
   const bool own = lane < nf;
@@ -1066,7 +1310,7 @@ __global__ __launch_bounds__(256) void k_bwd_tiny(const int* list, int count, De
   const int nf = fd.nF[s];
   const int64_t io = fd.idxOff[s];
   const int* pk = fd.pkind + io;
-  const T* F = static_cast<const T*>(fd.F[s]);
+  const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
   const bool own = lane < nf;
   // column `lane` of L below the diagonal, rows [lane + 1, m)
   double lc[64];
@@ -1452,13 +1696,28 @@ void launchDiagInverse(const int* list, int count, const int* blockStart, int bl
     k_diag_inverse<double><<<blocks, 64, 0, st>>>(list, count, blockStart, fd, inv, invOff);
   hipCheck(hipGetLastError(), "launchDiagInverse");
 }
-void launchFwdOwn(const int* list, int count, const DevFronts& fd, int nrhs, double* Z, double* Dl,
+// One wave per 16 right-hand sides, up to four; the variant for the most own
+// blocks of a listed front: two blocks (the fronts of one 64-column panel)
+// keep few registers.
+static int ownThreads(int nrhs) { return 64 * std::min(4, (nrhs + 15) / 16); }
+template <typename T>
+static void fwdOwnT(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* Z, double* Dl,
+                    const int64_t* gOff, const double* inv, const int64_t* invOff, hipStream_t st) {
+  auto go = [&](auto kernel) { kernel<<<count, ownThreads(nrhs), 0, st>>>(list, count, fd, nrhs, Z, Dl, gOff, inv, invOff); };
+  if (maxBlocks <= 2)
+    go(k_fwd_own<T, 2>);
+  else if (maxBlocks <= 4)
+    go(k_fwd_own<T, 4>);
+  else
+    go(k_fwd_own<T, kOwnMaxBlocks>);
+}
+void launchFwdOwn(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* Z, double* Dl,
                   const int64_t* gOff, const double* inv, const int64_t* invOff, hipStream_t st) {
   if (count <= 0 || nrhs <= 0) return;
   if (fd.fp32)
-    k_fwd_own<float><<<count, 256, 0, st>>>(list, count, fd, nrhs, Z, Dl, gOff, inv, invOff);
+    fwdOwnT<float>(list, count, maxBlocks, fd, nrhs, Z, Dl, gOff, inv, invOff, st);
   else
-    k_fwd_own<double><<<count, 256, 0, st>>>(list, count, fd, nrhs, Z, Dl, gOff, inv, invOff);
+    fwdOwnT<double>(list, count, maxBlocks, fd, nrhs, Z, Dl, gOff, inv, invOff, st);
   hipCheck(hipGetLastError(), "launchFwdOwn");
 }
 void launchFwdChain(const int* list, int count, const int* blockStart, int blocks, const DevFronts& fd, int nrhs,
@@ -1492,14 +1751,28 @@ void launchBwdAnc(const int* list, int count, const int* blockStart, int blocks,
     k_bwd_anc<double><<<blocks, 256, 0, st>>>(list, count, blockStart, fd, nrhs, Z, X, Dl, gOff, parts, err);
   hipCheck(hipGetLastError(), "launchBwdAnc");
 }
-void launchBwdOwn(const int* list, int count, const DevFronts& fd, int nrhs, double* X, double* Dl,
-                  const int64_t* gOff, const AncPart* parts, const double* inv, const int64_t* invOff,
-                  hipStream_t st) {
+template <typename T>
+static void bwdOwnT(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* X,
+                    const double* Dl, const int64_t* gOff, const AncPart* parts, const double* inv,
+                    const int64_t* invOff, hipStream_t st) {
+  auto go = [&](auto kernel) {
+    kernel<<<count, ownThreads(nrhs), 0, st>>>(list, count, fd, nrhs, X, Dl, gOff, parts, inv, invOff);
+  };
+  if (maxBlocks <= 2)
+    go(k_bwd_own<T, 2>);
+  else if (maxBlocks <= 4)
+    go(k_bwd_own<T, 4>);
+  else
+    go(k_bwd_own<T, kOwnMaxBlocks>);
+}
+void launchBwdOwn(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* X,
+                  const double* Dl, const int64_t* gOff, const AncPart* parts, const double* inv,
+                  const int64_t* invOff, hipStream_t st) {
   if (count <= 0 || nrhs <= 0) return;
   if (fd.fp32)
-    k_bwd_own<float><<<count, 256, 0, st>>>(list, count, fd, nrhs, X, Dl, gOff, parts, inv, invOff);
+    bwdOwnT<float>(list, count, maxBlocks, fd, nrhs, X, Dl, gOff, parts, inv, invOff, st);
   else
-    k_bwd_own<double><<<count, 256, 0, st>>>(list, count, fd, nrhs, X, Dl, gOff, parts, inv, invOff);
+    bwdOwnT<double>(list, count, maxBlocks, fd, nrhs, X, Dl, gOff, parts, inv, invOff, st);
   hipCheck(hipGetLastError(), "launchBwdOwn");
 }
 void launchBwdChain(const int* list, int count, const int* blockStart, int blocks, const DevFronts& fd, int nrhs,
