@@ -68,8 +68,8 @@ void launchDiagInverse(const int* list, int count, const int* blockStart, int bl
                        double* inv, const int64_t* invOff, hipStream_t st);
 // own rows, one workgroup per front (a short chain of own blocks, at most
 // maxBlocks <= kOwnMaxBlocks in a listed front): its products grow with the
-// square of the blocks (a chain of 10 took 83 us there, 50 with a workgroup
-// per block and flags between them)
+// square of the blocks (fronts of up to 10 took 83 us in one launch there;
+// the chain kernels take about 5 us a block)
 constexpr int kOwnMaxBlocks = 6;
 void launchFwdOwn(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* Z, double* Dl,
                   const int64_t* gOff, const double* inv, const int64_t* invOff, hipStream_t st);

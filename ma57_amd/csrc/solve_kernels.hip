@@ -641,10 +641,10 @@ __global__ __launch_bounds__(64) void k_diag_inverse(const int* list, int count,
 // no barrier, no wave waits for another.  Products are FP64 for FP32 fronts
 // too (the chain's latency is in the loads and the dependent products).
 //
-// Measured (40^3 7-point, FP64, one right-hand side, a launch per level, up
-// to 6 blocks): forward 36 -> 20 us, backward 36 -> 18; 53x57x59 27-point,
-// FP32, 33 right-hand sides: 97 -> 46 and 116 -> 35 (blocks through LDS, four
-// waves and four barriers per product before).
+// Measured (40^3 7-point, FP64, one right-hand side, all launches of a sweep):
+// forward 677 -> 297 us, backward 710 -> 279 (blocks through LDS, four waves
+// and four barriers per product before; 16 launches then, 15 now, as the level
+// whose fronts have up to 10 blocks went to the chain kernels).
 typedef double v4d __attribute__((ext_vector_type(4)));
 __device__ inline v4d ownMma(double a, double b, v4d c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
 // An FP64 16x16x4 product's result before a branch: the compiler may count a
