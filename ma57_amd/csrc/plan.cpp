@@ -396,11 +396,12 @@ void Plan::buildSchedule() {
     levelFrontOff_[L] = static_cast<int64_t>(all.size());
     for (int s : levelFronts_[L]) {
       all.push_back(s);
-      // column tiles: a large front gets narrower tiles so that it alone
-      // spreads over about 1024 workgroups (the top levels hold few fronts)
-      int w = tune_.asmTile;
-      while (w > 8 && (hm_[s] + w - 1) / w < 1024 && hm_[s] > 4 * tune_.asmTile) w >>= 1;
-      for (int c0 = 0; c0 < hm_[s]; c0 += w) tasks.push_back(make_int4(s, c0, std::min(c0 + w, hm_[s]), 0));
+      // assembly tiles of kAsmEntries entries, 16 columns by 256 rows (a
+      // child's column is read in runs of rows); a front that fits fewer rows
+      // gets more columns, so that a tiny one is one workgroup
+      const int w = std::min(tune_.asmTile, hm_[s] <= 64 ? 64 : hm_[s] <= 128 ? 32 : 16);
+      for (int c0 = 0; c0 < hm_[s]; c0 += w)
+        for (int r0 = c0; r0 < hm_[s]; r0 += kAsmEntries / w) tasks.push_back(make_int4(s, c0, c0 + w, r0));
       if (hm_[s] <= tune_.smallMax) {
         small.push_back(s);
         ls.smallMaxM = std::max(ls.smallMaxM, hm_[s]);

@@ -255,7 +255,7 @@ class Plan {
   bool hasGraph() const { return graphExec_ != nullptr; }
 
   // Scheduling choices: fronts of order <= smallMax take the LDS kernel,
-  // larger ones the panel path; assembly runs in column tiles of asmTile.
+  // larger ones the panel path; assembly tiles hold at most asmTile columns.
   struct Tuning {
     // fronts up to this order are factored whole in LDS; larger ones (also the
     // few mid-size fronts of the upper levels, where one workgroup per front
