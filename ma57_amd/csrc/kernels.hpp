@@ -48,6 +48,9 @@ void launchSyrk(const int* list, int count, const int* tileStart, const int* til
 // float for FP32 fronts), zero past the pivots taken
 void launchFormW(const DevFronts& fd, int s, int rows, int q0, int kc, void* W, hipStream_t st);
 void launchMakeRowIdx(const int* list, int count, const DevFronts& fd, hipStream_t st);
+// counts in outI[0..4], the perturbations' sum in outD[0]; the workgroups'
+// partial sums follow from outI[kStatsOutI] and outD[kStatsOutD]
+constexpr int kStatsParts = 256, kStatsOutI = 8, kStatsOutD = 4;
 void launchReduceStats(int numSN, const DevFronts& fd, long long* outI, double* outD, hipStream_t st);
 
 // solve_kernels.hip

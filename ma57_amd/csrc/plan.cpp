@@ -104,8 +104,8 @@ Plan::Plan(const SymbolicResult& sym, const int64_t* colptr, const int* rowidx) 
   dpert_.alloc(numSN_);
   dorigMax_.alloc(numSN_);
   drunMax_.alloc(numSN_);
-  dstatI_.alloc(8);
-  dstatD_.alloc(4);
+  dstatI_.alloc(kStatsOutI + 5 * kStatsParts);
+  dstatD_.alloc(kStatsOutD + kStatsParts);
   dvals_.alloc(nnzA_);
   uploadLayout();
   buildSchedule();
