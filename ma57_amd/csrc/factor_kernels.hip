@@ -2788,6 +2788,17 @@ __global__ __launch_bounds__(256) void k_panel_rows(const int* list, int count, 
 // read only when the walk enters a new front.  The product is formed
 // transposed (L operand first), so a register holds 16 consecutive rows of a
 // column: C is read and written in whole column segments.
+//
+// Bound by C's traffic (16 bytes per 128 flops in FP64) and by what a tile
+// does between its products: L D is formed in registers while the operands
+// are staged, behind one barrier and without branches (a neighbouring column
+// of a 2x2 block is the thread's own), and every load is unconditional, so
+// that the loads of a tile are in flight together.  Measured, all updates of
+// a factorization, before (L D through LDS, a branch per column) -> here:
+// 30^3 KKT, FP64, 56.1 -> 44.7 ms (17.6 -> 22 TFLOP/s); 64^3 27-point, FP64,
+// 16.4 -> 12.9 ms; 53x57x59 27-point, FP32, 6.9 -> 6.0 ms.  FP64 tiles need
+// 72 KiB of LDS, so two workgroups fit a CU and may use 256 registers a lane;
+// FP32 ones spill below 168.
 template <typename T>
 struct SchurMfma;
 template <>
@@ -2807,7 +2818,7 @@ struct SchurMfma<float> {
 };
 
 template <typename T>
-__global__ __launch_bounds__(256, 4) void k_schur(const int* list, int count, const int* tileStart, const int* tileTp,
+__global__ __launch_bounds__(256, sizeof(T) == 8 ? 2 : 3) void k_schur(const int* list, int count, const int* tileStart, const int* tileTp,
                                                DevFronts fd) {
   using M = SchurMfma<T>;
   constexpr int TS = 64;
@@ -2815,13 +2826,17 @@ __global__ __launch_bounds__(256, 4) void k_schur(const int* list, int count, co
   constexpr int KU = KP / 4;      // staged columns per thread
   __shared__ T As[TS][KP + 1];    // L D rows of the tile's row block
   __shared__ T Bs[TS][KP + 1];    // L rows of the tile's column block
-  __shared__ double pdd[kPanel + 2], pdo[kPanel + 2];
-  __shared__ int pkd[kPanel + 2];
+  // the panel's pivots: diagonal, coupling with the neighbour, its direction
+  // (0: 1x1); zero past the panel's columns
+  __shared__ double pdd[KP], pdn[KP];
+  __shared__ int pdir[KP];
   const int total = tileStart[count];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wr = (w >> 1) * 32, wc = (w & 1) * 32;
   const int lr = lane & 15, lk = lane >> 4;
-  const int sr = tid & 63, qb = tid >> 6;  // staging: row sr of both operand tiles, columns qb + 4u
+  // staging: row sr of both operand tiles, columns qb + u (a 2x2 block's
+  // neighbouring column is then in the thread's own registers)
+  const int sr = tid & 63, qb = (tid >> 6) * KU;
 
   // Geometry of tile t.  A front's tiles are numbered column block by
   // column block (tj, then ti = tj .. Tp-1 down the column), so the
@@ -2865,27 +2880,27 @@ __global__ __launch_bounds__(256, 4) void k_schur(const int* list, int count, co
   // a tile does work when its front took pivots and the tile lies in the
   // trailing block, left of the cut
   auto live = [&](const Tile& x) { return x.p > 0 && x.k1 + x.ti * TS < x.m && x.k1 + x.tj * TS < x.cut; };
-  T la[KU], lb[KU], cv[2][2][4];
+  T la[KU + 2], lb[KU], cv[2][2][4];  // la: columns qb - 1 .. qb + KU
   auto loadTile = [&](const Tile& x) {
     const int i0 = x.k1 + x.ti * TS, j0 = x.k1 + x.tj * TS;
-    const int ri = i0 + sr, rj = j0 + sr;
+    // every load is unconditional, at an address inside the front: rows past
+    // its end only make results that are not stored, columns past the pivots
+    // are zeroed when they are staged
+    const int ri = min(i0 + sr, x.m - 1), rj = min(j0 + sr, x.m - 1);
 #pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const int q = qb + 4 * u;
-      la[u] = (q < x.p && ri < x.m) ? x.F[ri + static_cast<size_t>(x.k0 + q) * x.m] : T(0);
-      lb[u] = (q < x.p && rj < x.m) ? x.F[rj + static_cast<size_t>(x.k0 + q) * x.m] : T(0);
-    }
+    for (int u = 0; u < KU + 2; ++u)
+      la[u] = x.F[ri + static_cast<size_t>(x.k0 + min(max(qb + u - 1, 0), x.p - 1)) * x.m];
+#pragma unroll
+    for (int u = 0; u < KU; ++u) lb[u] = x.F[rj + static_cast<size_t>(x.k0 + min(qb + u, x.p - 1)) * x.m];
 #pragma unroll
     for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
       for (int bj = 0; bj < 2; ++bj)
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
-          const int row = i0 + wr + bi * 16 + lr;
-          const int col = j0 + wc + bj * 16 + M::col(lane, rr);
-          cv[bi][bj][rr] = (row < x.m && col < x.cut && (x.ti != x.tj || row >= col))
-                               ? x.F[row + static_cast<size_t>(col) * x.m]
-                               : T(0);
+          const int row = min(i0 + wr + bi * 16 + lr, x.m - 1);
+          const int col = min(j0 + wc + bj * 16 + M::col(lane, rr), x.m - 1);
+          cv[bi][bj][rr] = x.F[row + static_cast<size_t>(col) * x.m];
         }
   };
 
@@ -2908,7 +2923,8 @@ __global__ __launch_bounds__(256, 4) void k_schur(const int* list, int count, co
   }
   if (t >= tEnd) return;
   Tile cur = tileOf(t, nullptr);
-  int pivFront = -1;  // front whose pivots are in pdd / pdo / pkd
+  int pivFront = -1;  // front whose pivots are in pdd / pdn / pdir
+  bool any2 = false;  // some of them 2x2
   // running max |F| of the updated entries: per lane over the tiles of one
   // front, folded into the front's record when the walk leaves it
   int mxFront = -1;
@@ -2923,12 +2939,17 @@ __global__ __launch_bounds__(256, 4) void k_schur(const int* list, int count, co
     const int tn = t + stride;
     if (live(cur)) {
       if (cur.s != pivFront) {
-        for (int q = tid; q < cur.p; q += blockDim.x) {
-          const int64_t io = fd.idxOff[cur.s];
-          pdd[q] = fd.dDiag[io + cur.k0 + q];
-          pdo[q] = fd.dOff[io + cur.k0 + q];
-          pkd[q] = fd.pkind[io + cur.k0 + q];
+        const int64_t io = fd.idxOff[cur.s] + cur.k0;
+        bool two = false;
+        if (tid < KP) {
+          const bool in = tid < cur.p;
+          const int kind = in ? fd.pkind[io + tid] : 1;
+          pdd[tid] = in && (kind != 0 || tid > 0) ? fd.dDiag[io + tid] : 0.0;
+          pdn[tid] = kind == 2 ? fd.dOff[io + tid] : kind == 0 && tid > 0 ? fd.dOff[io + tid - 1] : 0.0;
+          pdir[tid] = kind == 2 ? 1 : kind == 0 ? -1 : 0;
+          two = kind != 1;
         }
+        any2 = __syncthreads_or(two);
         pivFront = cur.s;
       }
       if (cur.ti == 0 && cur.tj == 0 && tid == 0 && fd.schurFlops) {
@@ -2937,33 +2958,26 @@ __global__ __launch_bounds__(256, 4) void k_schur(const int* list, int count, co
         const unsigned long long C = static_cast<unsigned long long>(cur.m - max(cur.cut, cur.k1));
         atomicAdd(fd.schurFlops, static_cast<unsigned long long>(cur.p) * (N * (N + 1) - C * (C + 1)));
       }
-      // stage the operands: raw L rows, then the L D scaling (a 2x2 block
-      // needs its neighbouring column, read back from LDS)
+      // stage the operands, L D formed on the way
+      auto stage = [&](auto two) {
 #pragma unroll
-      for (int u = 0; u < KU; ++u) {
-        As[sr][qb + 4 * u] = la[u];
-        Bs[sr][qb + 4 * u] = lb[u];
-      }
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < KU; ++u) {
-        const int q = qb + 4 * u;
-        double a = 0.0;
-        if (q < cur.p) {
-          const int kind = pkd[q];
-          const double l = static_cast<double>(la[u]);
-          if (kind == 1)
-            a = l * pdd[q];
-          else if (kind == 2)
-            a = l * pdd[q] + static_cast<double>(As[sr][q + 1]) * pdo[q];
-          else if (q > 0)
-            a = static_cast<double>(As[sr][q - 1]) * pdo[q - 1] + l * pdd[q];
+        for (int u = 0; u < KU; ++u) {
+          const int q = qb + u;
+          const double l = static_cast<double>(la[u + 1]);
+          double a = l * pdd[q];
+          if (decltype(two)::value) {
+            const int d = pdir[q];
+            const double n = static_cast<double>(d > 0 ? la[u + 2] : la[u]);
+            a = d != 0 ? l * pdd[q] + n * pdn[q] : a;
+          }
+          As[sr][q] = q < cur.p ? static_cast<T>(a) : T(0);
+          Bs[sr][q] = q < cur.p ? lb[u] : T(0);
         }
-        la[u] = static_cast<T>(a);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < KU; ++u) As[sr][qb + 4 * u] = la[u];
+      };
+      if (any2)
+        stage(std::true_type());
+      else
+        stage(std::false_type());
       __syncthreads();
     }
     // the next tile's operands and C travel while this tile computes
