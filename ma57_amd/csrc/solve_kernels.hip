@@ -169,6 +169,18 @@ __device__ inline double lvalOr0(P F, int m, const int* pk, int row, int col, bo
   return (ok && !(r == c + 1 && k == 2)) ? v : 0.0;
 }
 
+// Barrier for data in LDS: unlike __syncthreads it does not wait for the
+// thread's global loads and stores, so a tile's prefetched operands travel
+// across it.  With this barrier and operands held as loaded until they are
+// staged (all launches of three solves, 53x57x59 27-point, FP32): forward
+// chains 4.95 -> 3.02 ms, backward 4.91 -> 3.24, ancestors' parts 2.52 ->
+// 2.03, deltas 2.14 -> 1.79.
+__device__ inline void ldsBarrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // The solve's tile products on the matrix cores, in the storage type of the
 // factor: v_mfma_f64_16x16x4f64 for FP64 fronts, v_mfma_f32_16x16x4f32 for
 // FP32 fronts (operands rounded to FP32).  A[i][k] comes from lane i + 16k,
@@ -291,14 +303,20 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
       y0p[t][rr] = ldOr0(static_cast<const double*>(Ds), static_cast<int64_t>(r0 + r) * nrhs + rg + c, r < nr && c < gw);
     }
   // L(b, j) tiles four elements per thread, loaded one tile ahead
-  E lpre[4];
+  // (raw values and pivot kinds from addresses inside the front: a mask or a
+  // conversion next to a load would wait for it there, so both are applied
+  // when the values are staged)
+  T lpre[4];
+  int kpre[4];
   auto loadL = [&](int j) {
     const int c0 = j * SB, cn = min(SB, nf - c0);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int e = tid + u * NT;
       const int r = e % SB, qq = e / SB;
-      lpre[u] = static_cast<E>(lvalOr0(F, m, pk, r0 + r, c0 + qq, r < nr && qq < cn));
+      const int col = c0 + min(qq, cn - 1);
+      lpre[u] = F[r0 + min(r, nr - 1) + static_cast<int64_t>(col) * m];
+      kpre[u] = pk[col];
     }
   };
   double acc[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};  // FP64 sums of the per-tile products
@@ -306,19 +324,26 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
   for (int j = 0; j < b; ++j) {
     if (rg == 0) waitBlock(fl + j, gen, err);
     const int c0 = j * SB, cn = min(SB, nf - c0);
+    double yv[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int c = tid & 63, qq = (tid >> 6) + 4 * u;
+      yv[u] = loadShared(Ds + static_cast<int64_t>(c0 + min(qq, cn - 1)) * nrhs + rg + min(c, gw - 1));
+    }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int e = tid + u * NT;
-      S.Lt[e % SB][e / SB] = lpre[u];
+      const int r = e % SB, qq = e / SB;
+      const bool ok = r < nr && qq < cn && !(r0 + r == c0 + qq + 1 && kpre[u] == 2);
+      S.Lt[r][qq] = ok ? static_cast<E>(lpre[u]) : E(0);
     }
-    for (int e = tid; e < SB * 64; e += NT) {
-      const int c = e & 63, qq = e >> 6;
-      const bool ok = qq < cn && c < gw;
-      const double v = loadShared(Ds + (ok ? static_cast<int64_t>(c0 + qq) * nrhs + rg + c : 0));
-      S.yt[qq][c] = ok ? static_cast<E>(v) : E(0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int c = tid & 63, qq = (tid >> 6) + 4 * u;
+      S.yt[qq][c] = qq < cn && c < gw ? static_cast<E>(yv[u]) : E(0);
     }
     if (j + 1 < b) loadL(j + 1);
-    __syncthreads();
+    ldsBarrier();
     typename M::v4 part[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
     for (int kk = 0; kk < SB; kk += 4) {
@@ -330,7 +355,7 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) acc[t][rr] += static_cast<double>(part[t][rr]);
-    __syncthreads();
+    ldsBarrier();
   }
   // y_b = Ltop(b, b)^{-1} (y0_b - sum_j L(b, j) y_j), the inverse applied as
   // an FP64 tile product (rows past nr are zero so they add nothing)
@@ -341,7 +366,7 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
       const int r = tr + M::row(lane, rr), c = tc + 16 * t + lr;
       S.ys[r][c] = (r < nr && c < gw) ? y0p[t][rr] - acc[t][rr] : 0.0;
     }
-  __syncthreads();
+  ldsBarrier();
   {
     typename MD::v4 yv[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
@@ -350,7 +375,7 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
       yv[0] = MD::mma(av, S.ys[kk + lk][tc + lr], yv[0]);
       yv[1] = MD::mma(av, S.ys[kk + lk][tc + 16 + lr], yv[1]);
     }
-    __syncthreads();
+    ldsBarrier();
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -362,9 +387,11 @@ __device__ void fwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
         }
       }
   }
-  __syncthreads();
   // the later blocks need y only: release it before forming z
-  if (publish) publishBlock(fl + b, gen);
+  if (publish)
+    publishBlock(fl + b, gen);
+  else
+    __syncthreads();
   // z = D^{-1} y for the pivot blocks that end in this block (slot r + 1 of
   // the staged pivot data is position r0 + r)
   for (int e = tid; e < nr * gw; e += NT) {
@@ -431,14 +458,17 @@ __device__ void bwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
                    (pa.off + static_cast<int64_t>(k - 1) * pa.stride + r0 + qq) * nrhs + rg + c, ok);
       p0[t][rr] = v;
     }
-  E opre[4];
+  T opre[4];
+  int kpre[4];
   auto loadO = [&](int j) {
     const int i0 = j * SB, in = min(SB, nf - i0);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int e = tid + u * NT;
       const int i = e % SB, qq = e / SB;
-      opre[u] = static_cast<E>(lvalOr0(F, m, pk, i0 + i, r0 + qq, i < in && qq < nr));
+      const int col = r0 + min(qq, nr - 1);
+      opre[u] = F[i0 + min(i, in - 1) + static_cast<int64_t>(col) * m];
+      kpre[u] = pk[col];
     }
   };
   double acc[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
@@ -446,19 +476,26 @@ __device__ void bwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
   for (int j = nOwn - 1; j > w; --j) {
     if (rg == 0) waitBlock(fl + j, gen, err);
     const int i0 = j * SB, in = min(SB, nf - i0);
+    double xv[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int c = tid & 63, i = (tid >> 6) + 4 * u;
+      xv[u] = loadShared(Ds + static_cast<int64_t>(i0 + min(i, in - 1)) * nrhs + rg + min(c, gw - 1));
+    }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int e = tid + u * NT;
-      S.Lt[e % SB][e / SB] = opre[u];
+      const int i = e % SB, qq = e / SB;
+      const bool ok = i < in && qq < nr && !(i0 + i == r0 + qq + 1 && kpre[u] == 2);
+      S.Lt[i][qq] = ok ? static_cast<E>(opre[u]) : E(0);
     }
-    for (int e = tid; e < SB * 64; e += NT) {
-      const int c = e & 63, i = e >> 6;
-      const bool ok = i < in && c < gw;
-      const double v = loadShared(Ds + (ok ? static_cast<int64_t>(i0 + i) * nrhs + rg + c : 0));
-      S.yt[i][c] = ok ? static_cast<E>(v) : E(0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int c = tid & 63, i = (tid >> 6) + 4 * u;
+      S.yt[i][c] = i < in && c < gw ? static_cast<E>(xv[u]) : E(0);
     }
     if (j - 1 > w) loadO(j - 1);
-    __syncthreads();
+    ldsBarrier();
     typename M::v4 part[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
     for (int kk = 0; kk < SB; kk += 4) {
@@ -470,7 +507,7 @@ __device__ void bwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) acc[t][rr] += static_cast<double>(part[t][rr]);
-    __syncthreads();
+    ldsBarrier();
   }
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -479,7 +516,7 @@ __device__ void bwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
       const int qq = tr + M::row(lane, rr), c = tc + 16 * t + lr;
       S.ys[qq][c] = (qq < nr && c < gw) ? p0[t][rr] - acc[t][rr] : 0.0;
     }
-  __syncthreads();
+  ldsBarrier();
   {
     // x_w = L_ww^{-T} (...): the transposed inverse as an FP64 tile product
     typename MD::v4 xv[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
@@ -489,7 +526,7 @@ __device__ void bwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
       xv[0] = MD::mma(av, S.ys[kk + lk][tc + lr], xv[0]);
       xv[1] = MD::mma(av, S.ys[kk + lk][tc + 16 + lr], xv[1]);
     }
-    __syncthreads();
+    ldsBarrier();
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -501,9 +538,11 @@ __device__ void bwdOwnBlock(BlockLds<typename SweepMfma<T>::E>& S, const DevFron
         }
       }
   }
-  __syncthreads();
   // the earlier blocks need x only through the work block: release it, then write X
-  if (publish) publishBlock(fl + w, gen);
+  if (publish)
+    publishBlock(fl + w, gen);
+  else
+    __syncthreads();
   for (int e = tid; e < nr * gw; e += NT) {
     const int c = e % gw, r = e / gw;
     X[static_cast<int64_t>(S.rixA[r]) * nrhs + rg + c] = S.ys[r][c];
@@ -930,7 +969,7 @@ __global__ __launch_bounds__(256) void k_bwd_own(const int* list, int count, Dev
 // many workgroups at once.  A workgroup only waits for blocks of the same
 // front with a lower index, which were dispatched before it.
 template <typename T>
-__global__ __launch_bounds__(256) void k_fwd_chain(const int* list, int count, const int* blockStart, DevFronts fd,
+__global__ __launch_bounds__(256, 2) void k_fwd_chain(const int* list, int count, const int* blockStart, DevFronts fd,
                                                    int nrhs, double* __restrict__ Z, double* __restrict__ Dl,
                                                    const int64_t* __restrict__ gOff, unsigned* flags,
                                                    const int64_t* __restrict__ flagOff, const unsigned* genp,
@@ -978,20 +1017,20 @@ __device__ void fwdDeltaChunk(DeltaLds<typename SweepMfma<T>::E>& S, const DevFr
   const int lr = lane & 15, lk = lane >> 4;
   for (int rg = 0; rg < nrhs; rg += 64) {
     const int gw = min(64, nrhs - rg);
-    E lpre[8], ypre[8];
+    T lpre[8];  // as loaded: masked and converted when they are staged
+    double ypre[8];
     auto loadT = [&](int k0) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int e = tid + u * NT;
         const int i = e & (DT - 1), q = e / DT;
-        lpre[u] = static_cast<E>(ldOr0(F, (i0 + i) + static_cast<int64_t>(k0 + q) * m, i < ni && k0 + q < nf));
+        lpre[u] = F[i0 + min(i, ni - 1) + static_cast<int64_t>(min(k0 + q, nf - 1)) * m];
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int e = tid + u * NT;
         const int c = e & 63, q = e >> 6;
-        ypre[u] = static_cast<E>(ldOr0(static_cast<const double*>(Ds), static_cast<int64_t>(k0 + q) * nrhs + rg + c,
-                                        k0 + q < nf && c < gw));
+        ypre[u] = Ds[static_cast<int64_t>(min(k0 + q, nf - 1)) * nrhs + rg + min(c, gw - 1)];
       }
     };
     TileAcc<T, 4> acc;  // block (bi, bj) at 2 bi + bj
@@ -1001,11 +1040,13 @@ __device__ void fwdDeltaChunk(DeltaLds<typename SweepMfma<T>::E>& S, const DevFr
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int e = tid + u * NT;
-        S.Lt[e & (DT - 1)][e / DT] = lpre[u];
-        S.yt[e >> 6][e & 63] = ypre[u];
+        const int i = e & (DT - 1), q = e / DT;
+        S.Lt[i][q] = i < ni && k0 + q < nf ? static_cast<E>(lpre[u]) : E(0);
+        const int c = e & 63, qy = e >> 6;
+        S.yt[qy][c] = k0 + qy < nf && c < gw ? static_cast<E>(ypre[u]) : E(0);
       }
       if (k0 + SB < nf) loadT(k0 + SB);
-      __syncthreads();
+      ldsBarrier();
       typename M::v4* part = acc.begin();
 #pragma unroll 2
       for (int kk = 0; kk < SB; kk += 4) {
@@ -1017,7 +1058,7 @@ __device__ void fwdDeltaChunk(DeltaLds<typename SweepMfma<T>::E>& S, const DevFr
         part[3] = M::mma(a1, b1, part[3]);
       }
       acc.end();
-      __syncthreads();
+      ldsBarrier();
     }
     // g of the chunk's rows, all loaded before any is used
     double g[2][2][4];
@@ -1044,7 +1085,7 @@ __device__ void fwdDeltaChunk(DeltaLds<typename SweepMfma<T>::E>& S, const DevFr
 
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_fwd_delta(const int* list, int count, const int* blockStart, DevFronts fd,
+__global__ __launch_bounds__(256, 2) void k_fwd_delta(const int* list, int count, const int* blockStart, DevFronts fd,
                                                    int nrhs, double* __restrict__ Dl, const int64_t* __restrict__ gOff,
                                                    int* err) {
   __shared__ DeltaLds<typename SweepMfma<T>::E> S;
@@ -1061,8 +1102,7 @@ __global__ __launch_bounds__(256) void k_fwd_delta(const int* list, int count, c
 // Backward step, the ancestors' part (solve.hpp:364-383): for own block w of
 // a front, P_w = z_w - L(nF:m, w)^T x(nF:m), the ancestors' x final from the
 // levels above and read from X through the front's row indices (one
-// contiguous row each; the indices of a tile are read two tiles ahead, as
-// wave-uniform values).  The ancestors' rows are split in `split` chunks of
+// contiguous row each; the indices of a tile are read two tiles ahead).  The ancestors' rows are split in `split` chunks of
 // whole 64-row tiles: workgroup (w, k) takes chunk k of own block w, chunk 0
 // writing z_w less its part into the block's work rows, chunk k >= 1 its part
 // into the front's partial rows (AncPart).
@@ -1086,34 +1126,28 @@ __device__ void bwdAncChunk(AncLds<typename SweepMfma<T>::E>& S, const DevFronts
   const int64_t io = fd.idxOff[s];
   const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int wu = __builtin_amdgcn_readfirstlane(wv);
   const int tr = (wv & 1) * 16, tc = (wv >> 1) * 32;
   const int lr = lane & 15, lk = lane >> 4;
   for (int rg = 0; rg < nrhs; rg += 64) {
     const int gw = min(64, nrhs - rg);
-    // staging: thread (wave wu, lane) loads L rows i0 + lane of own columns
-    // wu + 4u, and x rows i0 + wu + 4u (right-hand side rg + lane)
-    E lpre[8], xpre[16];
-    int64_t rcur[16], rnext[16];
-    auto rows = [&](int i0, int64_t* out) {
-      // loaded unconditionally (a1 > i0 here) and held as loaded, so the
-      // sixteen loads are in flight together
-      int rr[16];
+    // staging: thread (wave wv, lane) loads L rows i0 + lane of own columns
+    // wv + 4u, and x rows i0 + wv + 4u (right-hand side rg + lane)
+    // (values and indices stay as loaded until the next use needs them)
+    T lpre[8];
+    double xpre[16];
+    int rcur[16], rnext[16];
+    auto rows = [&](int i0, int* out) {
 #pragma unroll
-      for (int u = 0; u < 16; ++u) rr[u] = fd.rowIdx[io + min(i0 + wu + 4 * u, a1 - 1)];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) asm volatile("" : "+v"(rr[u]));
-#pragma unroll
-      for (int u = 0; u < 16; ++u) out[u] = (i0 + wu + 4 * u < a1) ? static_cast<int64_t>(rr[u]) * nrhs : -1;
+      for (int u = 0; u < 16; ++u) out[u] = fd.rowIdx[io + min(i0 + wv + 4 * u, a1 - 1)];
     };
-    auto loadT = [&](int i0, const int64_t* xr) {
+    auto loadT = [&](int i0, const int* xr) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int q = wv + 4 * u;
-        lpre[u] = static_cast<E>(ldOr0(F, (i0 + lane) + static_cast<int64_t>(r0 + q) * m, i0 + lane < a1 && q < nr));
+        lpre[u] = F[min(i0 + lane, a1 - 1) + static_cast<int64_t>(r0 + min(q, nr - 1)) * m];
       }
 #pragma unroll
-      for (int u = 0; u < 16; ++u) xpre[u] = static_cast<E>(ldOr0(X, xr[u] + rg + lane, xr[u] >= 0 && lane < gw));
+      for (int u = 0; u < 16; ++u) xpre[u] = X[static_cast<int64_t>(xr[u]) * nrhs + rg + min(lane, gw - 1)];
     };
     double acc[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
     if (a0 < a1) {
@@ -1123,16 +1157,20 @@ __device__ void bwdAncChunk(AncLds<typename SweepMfma<T>::E>& S, const DevFronts
     }
     for (int i0 = a0; i0 < a1; i0 += DT) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) S.Lt[lane][wv + 4 * u] = lpre[u];
+      for (int u = 0; u < 8; ++u) {
+        const int q = wv + 4 * u;
+        S.Lt[lane][q] = i0 + lane < a1 && q < nr ? static_cast<E>(lpre[u]) : E(0);
+      }
 #pragma unroll
-      for (int u = 0; u < 16; ++u) S.xt[wv + 4 * u][lane] = xpre[u];
+      for (int u = 0; u < 16; ++u) {
+        const int i = wv + 4 * u;
+        S.xt[i][lane] = i0 + i < a1 && lane < gw ? static_cast<E>(xpre[u]) : E(0);
+      }
       if (i0 + DT < a1) {
         loadT(i0 + DT, rnext);
-#pragma unroll
-        for (int u = 0; u < 16; ++u) rcur[u] = rnext[u];
         if (i0 + 2 * DT < a1) rows(i0 + 2 * DT, rnext);
       }
-      __syncthreads();
+      ldsBarrier();
       typename M::v4 part[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll 4
       for (int kk = 0; kk < DT; kk += 4) {
@@ -1144,7 +1182,7 @@ __device__ void bwdAncChunk(AncLds<typename SweepMfma<T>::E>& S, const DevFronts
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) acc[t][rr] += static_cast<double>(part[t][rr]);
-      __syncthreads();
+      ldsBarrier();
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -1167,7 +1205,7 @@ __device__ void bwdAncChunk(AncLds<typename SweepMfma<T>::E>& S, const DevFronts
 
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_bwd_anc(const int* list, int count, const int* blockStart, DevFronts fd,
+__global__ __launch_bounds__(256, 2) void k_bwd_anc(const int* list, int count, const int* blockStart, DevFronts fd,
                                                  int nrhs, const double* __restrict__ Z, const double* __restrict__ X,
                                                  double* __restrict__ Dl, const int64_t* __restrict__ gOff,
                                                  const AncPart* __restrict__ parts, int* err) {
@@ -1189,7 +1227,7 @@ __global__ __launch_bounds__(256) void k_bwd_anc(const int* list, int count, con
 // own block, taken from the last block to the first; block w waits for the
 // blocks j > w of its front (dispatched before it).
 template <typename T>
-__global__ __launch_bounds__(256) void k_bwd_chain(const int* list, int count, const int* blockStart, DevFronts fd,
+__global__ __launch_bounds__(256, 2) void k_bwd_chain(const int* list, int count, const int* blockStart, DevFronts fd,
                                                    int nrhs, double* __restrict__ X, double* __restrict__ Dl,
                                                    const int64_t* __restrict__ gOff,
                                                    const AncPart* __restrict__ parts, unsigned* flags,
