@@ -122,10 +122,13 @@ __host__ __device__ inline bool specFront(const FactorParams& p, int nE) { retur
 //                      16-column blocks (Block16::op each)
 //   wneg[6 * 4 * 64]   -d_q l_jq of the 16 x 16 tiles (column block b2, b < b2)
 //                      at 256 (b2 (b2 - 1) / 2 + b), in the MFMA operand's lane order
+//   k0                 the panel's first pivot position, -1 when the front takes no
+//                      panel (written by the first pass: the last one advances
+//                      kcur while other workgroups of its launch have yet to start)
 // followed, for fronts that take the step, by the backup of the raw panel
 // values of the block's rows and those below (m x kPanel front elements, row
 // i of panel column q at i + q m), from which a failed test restores them.
-constexpr int kSpecRec = 8 * kPanel + (4 + 6) * 4 * 64;
+constexpr int kSpecRec = 8 * kPanel + (4 + 6) * 4 * 64 + 2;  // (even: 16-byte rows)
 constexpr int kSpecRows = 64;  // rows below the block per workgroup (16 per wave)
 // The panel kernel keeps up to kPanelRegRows rows in registers; a front with
 // more eligible rows streams them through 16 more columns of its workspace.

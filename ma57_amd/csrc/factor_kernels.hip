@@ -2148,6 +2148,7 @@ struct SpecRec {
   double* rdiv;
   double* ops;
   double* wneg;
+  int* k0;
   double* backup;
 };
 __device__ inline SpecRec specRec(double* ws, int nE) {
@@ -2162,6 +2163,7 @@ __device__ inline SpecRec specRec(double* ws, int nE) {
   x.rdiv = r + 7 * kPanel;
   x.ops = r + 8 * kPanel;
   x.wneg = x.ops + 4 * 4 * 64;
+  x.k0 = reinterpret_cast<int*>(x.wneg + 6 * 4 * 64);
   x.backup = r + kSpecRec;
   return x;
 }
@@ -2197,14 +2199,16 @@ __global__ __launch_bounds__(256) void k_spec_block(const int* list, int count, 
   if (static_cast<int>(blockIdx.x) >= count) return;
   const int s = list[blockIdx.x];
   const int nE = fd.nE[s];
-  if (!specFront(prm, nE) || fd.stopped[s]) return;
+  if (!specFront(prm, nE)) return;
   const int m = fd.m[s];
   const int k0 = fd.kcur[s];
-  if (k0 >= nE) return;
+  const SpecRec rec = specRec(wsBase + wsOff[s], nE);
+  const bool none = fd.stopped[s] || k0 >= nE;
+  if (threadIdx.x == 0) *rec.k0 = none ? -1 : k0;
+  if (none) return;
   const int pw = min(P, nE - k0);
   const GlobalPtr<T> F = globalView<T>(fd.F[s]);
   const int64_t io = fd.idxOff[s];
-  const SpecRec rec = specRec(wsBase + wsOff[s], nE);
   T* const bk = reinterpret_cast<T*>(rec.backup);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -2451,7 +2455,9 @@ constexpr int kSpecApplyThreads = kSpecRows;
 // rows, the whole block of the rows [nE, m)).  Workgroup 0 commits the block's
 // columns before q*, the pivots, inertia, perturbation counts and the running
 // maximum, sets kcur = k0 + q*, pcount = q*, and clears the other colmax
-// buffer and the exact maxima for the next panel.
+// buffer and the exact maxima for the next panel.  Nothing orders workgroup 0
+// against the others, so what they read is nothing that it writes: the panel's
+// position is the record's k0, not kcur.
 template <typename T>
 __global__ __launch_bounds__(kSpecApplyThreads) void k_spec_apply(const int* list, int count, const int* wgStart, int parity,
                                                     DevFronts fd, FactorParams prm, double* wsBase,
@@ -2466,8 +2472,9 @@ __global__ __launch_bounds__(kSpecApplyThreads) void k_spec_apply(const int* lis
   const int m = fd.m[s];
   const int nE = fd.nE[s];
   if (!specFront(prm, nE)) return;  // this front's panels are all exact
-  const int k0 = fd.kcur[s];
-  if (fd.stopped[s] || k0 >= nE) {
+  const SpecRec rec = specRec(wsBase + wsOff[s], nE);
+  const int k0 = *rec.k0;
+  if (k0 < 0) {
     if (w == 0 && tid == 0) {
       fd.pcount[s] = 0;
       fd.cbDone[s] = 0;
@@ -2480,7 +2487,6 @@ __global__ __launch_bounds__(kSpecApplyThreads) void k_spec_apply(const int* lis
   T* F = static_cast<T*>(fd.F[s]);
   auto Fat = [&](int i, int j) -> T& { return F[i + static_cast<size_t>(j) * m]; };
   const int64_t io = fd.idxOff[s];
-  const SpecRec rec = specRec(wsBase + wsOff[s], nE);
   const bool stat = prm.staticMode != 0;
   double origMax = bitsToDouble(fd.origMaxBits[s]);
   if (!stat && origMax < prm.zeroTol) origMax = 1.0;
