@@ -128,9 +128,10 @@ __device__ inline void countInertia2(double d11, double d22, double det, int& po
 __device__ inline double staticPivot(double a_kk, int sign, double delta, double floorv, double& applied) {
   // (selects, no branches: it is on the panels' dependent chain)
   const double s = sign != 0 ? static_cast<double>(sign) : (a_kk >= 0.0 ? 1.0 : -1.0);
-  const double towards = sign != 0 ? a_kk * s : fabs(a_kk);
-  const double d = towards < floorv ? a_kk + s * delta : a_kk;
-  applied = d - a_kk;
+  const double towards = sign > 0 ? a_kk : (sign < 0 ? -a_kk : fabs(a_kk));
+  const bool need = towards < floorv;  // false for NaN: such a pivot is taken as it is
+  const double d = need ? a_kk + s * delta : a_kk;
+  applied = need ? d - a_kk : 0.0;
   return d;
 }
 
