@@ -777,6 +777,32 @@ __device__ inline double pivotRecip(double d) {
   return r;
 }
 
+// c / d rounded to the front's type, r the reciprocal of d: one residual step
+// makes the quotient a correctly rounded one (c r alone is up to 1.5 ulp off,
+// and what a column takes off the later ones is c, so the factors' backward
+// error follows the multiplier's).  An FP32 multiplier hides it.  div_fixup
+// gives the quotients of zero, infinite and NaN operands.
+template <typename T>
+__device__ inline T multiplier(double c, double d, double r) {
+  double l = c * r;
+  if constexpr (sizeof(T) == 8) l = __builtin_amdgcn_div_fixup(fma(fma(-l, d, c), r, l), d, c);
+  return static_cast<T>(l);
+}
+
+// c / d with d on a dependent chain: one Newton step on the hardware
+// reciprocal (24 bits) and the residual step; an IEEE division when d is zero
+// or denormal or an operand is not finite.
+__device__ inline double pivotQuot(double c, double d) {
+  const double a = fabs(d);
+  double r = __builtin_amdgcn_rcp(d);
+  r = fma(fma(-d, r, 1.0), r, r);
+  double l = c * r;
+  l = fma(fma(-l, d, c), r, l);
+  const bool special = !(a >= DBL_MIN && a <= DBL_MAX && fabs(c) <= DBL_MAX);
+  if (__builtin_expect(__ballot(special) != 0, 0)) l = special ? c / d : l;
+  return l;
+}
+
 // A double of lane `src` (the same for the whole wave) in every lane.
 __device__ inline double readLane(double v, int src) {
   const int lo = __builtin_amdgcn_readlane(__double2loint(v), src);
@@ -808,22 +834,6 @@ __device__ inline double max16(double v) {
 typedef double v4d __attribute__((ext_vector_type(4)));
 __device__ inline v4d mfma64(double a, double b, v4d c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
 
-// Inverse of a 4 x 4 unit lower block, rows 1 .. 3 of column k (column 0
-// first): m[r][k] for r > k.
-struct Inv4 {
-  double m10, m20, m21, m30, m31, m32;
-};
-__device__ inline Inv4 invUnit4(double l10, double l20, double l21, double l30, double l31, double l32) {
-  Inv4 v;
-  v.m10 = -l10;
-  v.m21 = -l21;
-  v.m32 = -l32;
-  v.m20 = fma(l21, l10, -l20);
-  v.m31 = fma(l32, l21, -l31);
-  v.m30 = -(l30 + l31 * v.m10 + l32 * v.m20);
-  return v;
-}
-
 // Waits for the matrix cores' results in x: 20 wait states cover an FP64
 // 16x16x4 product.  The compiler keeps that distance for reads in
 // straight-line code, but a register of a result that nothing reads may be
@@ -841,16 +851,51 @@ __device__ inline void ldsBarrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// One substitution step of a 16-column block held as above: x_s <- M_s x_s
-// for the four columns of group s, and the groups after it take
-// x -= L M_s x_s.  `a` is the step's operand (substOps); the groups before s
-// are left alone, so values of a later column never reach an earlier one.
+// The four 16-lane rows of v, each in every lane's x[row].
+__device__ inline void rows16(double v, double (&x)[4]) {
+  uint32_t w[2] = {static_cast<uint32_t>(__double2loint(v)), static_cast<uint32_t>(__double2hiint(v))};
+  uint32_t r[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const auto p = __builtin_amdgcn_permlane16_swap(w[h], w[h], false, false);  // rows 0 0 2 2 and 1 1 3 3
+    const auto e = __builtin_amdgcn_permlane32_swap(p[0], p[0], false, false);
+    const auto o = __builtin_amdgcn_permlane32_swap(p[1], p[1], false, false);
+    r[h][0] = e[0];
+    r[h][1] = o[0];
+    r[h][2] = e[1];
+    r[h][3] = o[1];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) x[k] = __hiloint2double(static_cast<int>(r[1][k]), static_cast<int>(r[0][k]));
+}
+
+// One substitution step of a 16-column block held as above: the four columns
+// of group s are solved one after the other, then the groups after it take
+// x -= L x_s in one product.  `a` is the step's operand: -L(i, 4 s + k) in
+// lane i + 16 k.  A column only ever reaches later ones, so an infinity or a
+// NaN stays where a column-by-column substitution has it.
+//
+// (The inverse of the group's 4 x 4 unit block on the matrix cores in place
+// of the six dependent products is as accurate only while the multipliers
+// are bounded: static pivots, random dense fronts of 300 rows, componentwise
+// backward error 1600 u in the worst of six, against 1.5 u.)
 template <int S>
 __device__ inline void substStep(v4d& x, double a) {
-  v4d d = mfma64(a, x[S], x);
-  settle(d);
+  auto l = [&](int i, int k) { return readLane(a, 4 * S + i + 16 * k); };
+  const int k = (threadIdx.x >> 4) & 3;
+  double y[4];
+  rows16(x[S], y);
+  y[1] = fma(l(1, 0), y[0], y[1]);
+  y[2] = fma(l(2, 1), y[1], fma(l(2, 0), y[0], y[2]));
+  y[3] = fma(l(3, 2), y[2], fma(l(3, 1), y[1], fma(l(3, 0), y[0], y[3])));
+  const double v = k < 2 ? (k == 0 ? y[0] : y[1]) : (k == 2 ? y[2] : y[3]);
+  if constexpr (S < 3) {
+    v4d d = mfma64(a, v, x);
+    settle(d);
 #pragma unroll
-  for (int r = S; r < 4; ++r) x[r] = d[r];
+    for (int r = S + 1; r < 4; ++r) x[r] = d[r];
+  }
+  x[S] = v;
 }
 
 // The substitution of one 16-row tile by a 16-column block: x becomes the
@@ -882,7 +927,7 @@ __device__ inline void unrolled(std::integer_sequence<int, I...>, Fn&& fn) {
 // A 16 x 16 diagonal block's factorization and the operands of its
 // substitution, in LDS for every wave of the workgroup.
 struct Block16 {
-  double op[4][64];  // step s, lane i + 16 k: row i, column 4 s + k of [M_s - I within the group; -L M_s after it]
+  double op[4][64];  // step s, lane i + 16 k: -L(i, 4 s + k), zero on and above the diagonal
   double akk[16];    // current diagonal at each pivot
   double d[16], rd[16];  // the pivots (pivotOf) and their reciprocals
 };
@@ -892,49 +937,38 @@ struct Block16 {
 // row i of the lower triangle in a[], rows of a smaller block's padding those
 // of the identity.  pivotOf(q, a_qq) is the pivot (for a lane's own column
 // with q the lane).  Multipliers are rounded to the front's type T.  The
-// chain per pivot is one reciprocal and one product; a pivot row's
-// multipliers reach the other rows as DPP operands of the updates, one
-// instruction each (through lane reads into scalar registers, with a branch
-// or two per pivot, a block took 8000 cycles).  Only 4 x 4 blocks are
-// inverted for the substitution, so its rounding is close to that of a
-// column-by-column one.
+// chain per pivot is one quotient; a pivot row's multipliers reach the other
+// rows as DPP operands of the updates, one instruction each (through lane
+// reads into scalar registers, with a branch or two per pivot, a block took
+// 8000 cycles).  The block's multipliers that the front keeps are these, not
+// ones that the substitution forms again: all later products of the block's
+// columns use these, and where static pivots make them large a second
+// rounding of the same values is a backward error of its own.
 template <typename T, typename PivotOf>
 __device__ inline void blockFactor16(double (&a)[16], Block16& B, PivotOf pivotOf) {
   const int lane = threadIdx.x & 63, i = lane & 15, k = lane >> 4;
-  auto stored = [](double c, double r) { return static_cast<double>(static_cast<T>(c * r)); };
+  double akk = a[0];
   unrolled(std::make_integer_sequence<int, 16>{}, [&](auto qq) {
     constexpr int q = decltype(qq)::value;
-    double l = stored(a[q], pivotRecip(pivotOf(q, bcast16<q>(a[q]))));
+    double l = static_cast<double>(static_cast<T>(pivotQuot(a[q], pivotOf(q, bcast16<q>(a[q])))));
     const double c = -a[q];
+    if (q > 0) akk = i == q ? a[q] : akk;
     asm volatile("s_nop 1" : "+v"(l));
     unrolled(std::make_integer_sequence<int, 15 - q>{}, [&](auto jj) {
       constexpr int j = q + 1 + decltype(jj)::value;
       fmaBcast16<j>(a[j], l, c);
     });
+    a[q] = l;
   });
-  double akk = a[0];
-#pragma unroll
-  for (int q = 1; q < 16; ++q) akk = i == q ? a[q] : akk;
   const double d = pivotOf(i, akk);
   B.akk[i] = akk;  // (the four groups store the same values)
   B.d[i] = d;
-  const double rd = pivotRecip(d);
-  B.rd[i] = rd;
-  unrolled(std::make_integer_sequence<int, 4>{}, [&](auto ss) {
-    constexpr int s = decltype(ss)::value, c = 4 * s;
-    // this row's multipliers in the group's columns (the values of the loop above)
-    const double l0 = stored(a[c], bcast16<c>(rd)), l1 = stored(a[c + 1], bcast16<c + 1>(rd));
-    const double l2 = stored(a[c + 2], bcast16<c + 2>(rd)), l3 = stored(a[c + 3], bcast16<c + 3>(rd));
-    const Inv4 v = invUnit4(bcast16<c + 1>(l0), bcast16<c + 2>(l0), bcast16<c + 2>(l1), bcast16<c + 3>(l0),
-                            bcast16<c + 3>(l1), bcast16<c + 3>(l2));
-    const double m0 = k == 0 ? 1.0 : 0.0;  // column k of M_s
-    const double m1 = k == 0 ? v.m10 : (k == 1 ? 1.0 : 0.0);
-    const double m2 = k == 0 ? v.m20 : (k == 1 ? v.m21 : (k == 2 ? 1.0 : 0.0));
-    const double m3 = k == 0 ? v.m30 : (k == 1 ? v.m31 : (k == 2 ? v.m32 : 1.0));
-    const double below = -(l0 * m0 + l1 * m1 + l2 * m2 + l3 * m3);
-    const int r = i - c;
-    B.op[s][lane] = r <= k ? 0.0 : (r == 1 ? m1 : (r == 2 ? m2 : (r == 3 ? m3 : below)));
-  });
+  B.rd[i] = pivotRecip(d);
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const double l = k < 2 ? (k == 0 ? a[4 * s] : a[4 * s + 1]) : (k == 2 ? a[4 * s + 2] : a[4 * s + 3]);
+    B.op[s][lane] = i > 4 * s + k ? -l : 0.0;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1482,12 +1516,9 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
       }
     }
     sync();
-    double op[4], rdc[4];
+    double op[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      op[u] = blk.op[u][lane];
-      rdc[u] = blk.rd[4 * u + lk];
-    }
+    for (int u = 0; u < 4; ++u) op[u] = blk.op[u][lane];
     const double akk = blk.akk[lr];
     // substitution of the held rows and the maxima over the eligible rows below each pivot
     double vm[4] = {0.0, 0.0, 0.0, 0.0};
@@ -1536,16 +1567,34 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
     const unsigned long long bad = __ballot(lane < sw && !pass);
     const int qs = bad ? __ffsll(static_cast<long long>(bad)) - 1 : sw;
     // keep the columns before it: multipliers, pivots, counts
+    double dc[4], rdc[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      dc[u] = blk.d[4 * u + lk];
+      rdc[u] = blk.rd[4 * u + lk];
+    }
     auto acceptChunk = [&](int ch) {
 #pragma unroll
       for (int t = 0; t < CT; ++t) {
-        const int row = rowOf(ch, t) + lr;
+        const int row0 = rowOf(ch, t), row = row0 + lr;
+        T lt[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) lt[u] = multiplier<T>(x[t][u], dc[u], rdc[u]);
+        if (row0 < c0 + sw && row0 + 16 > c0) {
+          // the block's own rows keep the multipliers of its factorization
+          const int i = row - c0, ic = min(max(i, 0), sw - 1);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const T lb = static_cast<T>(-blk.op[u][ic + 16 * lk]);
+            lt[u] = i == ic ? lb : lt[u];
+          }
+        }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int q = 4 * u + lk;
           if (q < qs && row > c0 + q && row < rEnd) {
             tmax = fmax(tmax, fabs(x[t][u]));
-            const T l = static_cast<T>(x[t][u] * rdc[u]);
+            const T l = lt[u];
             if constexpr (kInLds)
               Lp[(c0 - k0 + q) * LD + (row - k0)] = l;
             else
@@ -2281,7 +2330,8 @@ __global__ __launch_bounds__(256) void k_spec_block(const int* list, int count, 
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int q = 4 * u + lk, col = 16 * b + q;
-        const T lt = static_cast<T>(x[b][u] * blk.rd[q]);
+        // the block's own rows keep the multipliers of its factorization
+        const T lt = wv == b ? static_cast<T>(-blk.op[u][lane]) : multiplier<T>(x[b][u], blk.d[q], blk.rd[q]);
         const double l = static_cast<double>(lt);
         if (row < pw && col < row) F[(k0 + row) + static_cast<int64_t>(k0 + col) * m] = lt;
         if (row < pw && col == row) F[(k0 + row) + static_cast<int64_t>(k0 + col) * m] = static_cast<T>(blk.d[q]);
@@ -2365,12 +2415,13 @@ __global__ __launch_bounds__(4 * kSpecRows) void k_spec_factor(const int* list, 
         const int q = 16 * b + 4 * u + lk;
         raw[b][u] = F[valid && q < pw ? i + static_cast<int64_t>(k0 + q) * m : 0];
       }
-    double op[NB][4], wn[NB > 1 ? NB * (NB - 1) / 2 : 1][4], rd[NB][4];
+    double op[NB][4], wn[NB > 1 ? NB * (NB - 1) / 2 : 1][4], dv[NB][4], rd[NB][4];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         op[b][u] = rec.ops[(4 * b + u) * 64 + lane];
+        dv[b][u] = rec.dval[16 * b + 4 * u + lk];
         rd[b][u] = rec.rdiv[16 * b + 4 * u + lk];
       }
 #pragma unroll
@@ -2397,7 +2448,7 @@ __global__ __launch_bounds__(4 * kSpecRows) void k_spec_factor(const int* list, 
       constexpr int b = decltype(bb)::value;
       substTile(x[b], op[b]);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) l[b][u] = static_cast<T>(x[b][u] * rd[b][u]);
+      for (int u = 0; u < 4; ++u) l[b][u] = multiplier<T>(x[b][u], dv[b][u], rd[b][u]);
 #pragma unroll
       for (int b2 = b + 1; b2 < NB; ++b2) {
 #pragma unroll
@@ -2587,23 +2638,21 @@ __global__ void k_spec_reset(const int* list, int count, DevFronts fd, double* w
 // panel.  With U = D L^T of the panel, the multipliers of a row are
 // f U^{-1} = (f L^{-T}) D^{-1} (dense_kernel.hpp:772-787 applied to the whole
 // panel at once).  y = f L^{-T} is a substitution over the panel's columns in
-// groups of four: the operators [M_g - I; -L M_g] (M_g the inverse of group
-// g's 4 x 4 unit lower block) are formed in LDS once per workgroup, then every
-// wave takes 16 rows as 16 columns of the FP64 MFMA (layout above k_panel),
-// group after group, the solved group feeding the products of the later
-// columns from its own registers.  l = y D^{-1} follows for the 1x1 and 2x2
-// pivot blocks.  64 rows per workgroup: a front's rows spread over as many
-// CUs as they can; what is left is the latency of the panel block's loads
-// and of 16 dependent MFMA steps.
+// groups of four (substStep), -L of the panel's block in LDS: every wave takes
+// 16 rows as 16 columns of the FP64 MFMA (layout above k_panel), group after
+// group, the solved group feeding the products of the later columns from its
+// own registers.  l = y D^{-1} follows for the 1x1 and 2x2 pivot blocks.  64
+// rows per workgroup: a front's rows spread over as many CUs as they can; what
+// is left is the latency of the panel block's loads and of 16 dependent steps.
 template <typename T>
 __global__ __launch_bounds__(256) void k_panel_rows(const int* list, int count, const int* blockStart,
                                                      DevFronts fd) {
   constexpr int P = kPanel + 1;  // a 2x2 pivot at the panel's last column makes it 65
   constexpr int G = (P + 3) / 4, PP = 4 * G;
   constexpr int NB = (PP + 15) / 16;
-  __shared__ double Pm[16 * NB][PP + 1];  // the panel's unit lower block, then the operators
-  __shared__ double Mg[G][16];       // M_g, row-major
+  __shared__ double Pm[16 * NB][PP + 1];  // -L of the panel's block, zero on and above its diagonal
   __shared__ double cSelf[PP], cNext[PP], cPrev[PP];  // l_q = y_q cSelf + y_{q+1} cNext + y_{q-1} cPrev
+  __shared__ double cDiv[PP];  // 1x1 pivots (cSelf their reciprocals): l_q = y_q / cDiv
   __shared__ int pkd[PP];
   __shared__ int any2;
   if (static_cast<int>(blockIdx.x) >= blockStart[count]) return;
@@ -2644,10 +2693,11 @@ __global__ __launch_bounds__(256) void k_panel_rows(const int* list, int count, 
     for (int q = tid; q < PP; q += 256) pkd[q] = q < p ? fd.pkind[io + k0 + q] : 1;
     __syncthreads();
     for (int q = tid; q < PP; q += 256) {
-      double cs = 1.0, cn = 0.0, cp = 0.0;
+      double cs = 1.0, cn = 0.0, cp = 0.0, cd = 1.0;
       if (q < p) {
         const double d = fd.dDiag[io + k0 + q];
         if (pkd[q] == 1) {
+          cd = d;
           cs = 1.0 / d;
         } else {
           const int h = pkd[q] == 2 ? q : q - 1;  // first column of the 2x2 block
@@ -2661,44 +2711,20 @@ __global__ __launch_bounds__(256) void k_panel_rows(const int* list, int count, 
       cSelf[q] = cs;
       cNext[q] = cn;
       cPrev[q] = cp;
+      cDiv[q] = cd;
     }
-    // unit lower L of the panel; the (q+1, q) slot of a 2x2 block holds d21
+    // (the (q+1, q) slot of a 2x2 block holds d21)
 #pragma unroll
     for (int u = 0; u < kPanel / 4; ++u) {
       const int c = wv + 4 * u;
-      Pm[lane][c] = (lane < p && c < lane && !(lane == c + 1 && pkd[c] == 2)) ? static_cast<double>(blk[u]) : 0.0;
+      Pm[lane][c] = (lane < p && c < lane && !(lane == c + 1 && pkd[c] == 2)) ? -static_cast<double>(blk[u]) : 0.0;
     }
     if (tid < kPanel) {
-      Pm[kPanel][tid] = (p > kPanel && !(tid == kPanel - 1 && pkd[tid] == 2)) ? static_cast<double>(last) : 0.0;
+      Pm[kPanel][tid] = (p > kPanel && !(tid == kPanel - 1 && pkd[tid] == 2)) ? -static_cast<double>(last) : 0.0;
       for (int r = kPanel + 1; r < 16 * NB; ++r) Pm[r][tid] = 0.0;
     }
     if (tid < 16 * NB)
       for (int c = kPanel; c < PP; ++c) Pm[tid][c] = 0.0;
-  }
-  __syncthreads();
-  if (tid < G) {
-    const int g = 4 * tid;
-    const Inv4 v = invUnit4(Pm[g + 1][g], Pm[g + 2][g], Pm[g + 2][g + 1], Pm[g + 3][g], Pm[g + 3][g + 1],
-                            Pm[g + 3][g + 2]);
-    const double mm[16] = {1, 0, 0, 0, v.m10, 1, 0, 0, v.m20, v.m21, 1, 0, v.m30, v.m31, v.m32, 1};
-#pragma unroll
-    for (int e = 0; e < 16; ++e) Mg[tid][e] = mm[e];
-  }
-  __syncthreads();
-  for (int e = tid; e < PP * G; e += 256) {
-    const int i = e % PP, g = e / PP, r = i - 4 * g;
-    double o[4];
-    if (r < 0) continue;  // above the group: zero, and not read
-    if (r < 4) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) o[k] = k < r ? Mg[g][4 * r + k] : 0.0;
-    } else {
-      const double l0 = Pm[i][4 * g], l1 = Pm[i][4 * g + 1], l2 = Pm[i][4 * g + 2], l3 = Pm[i][4 * g + 3];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) o[k] = -(l0 * Mg[g][k] + l1 * Mg[g][4 + k] + l2 * Mg[g][8 + k] + l3 * Mg[g][12 + k]);
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) Pm[i][4 * g + k] = o[k];
   }
   __syncthreads();
   v4d x[NB];
@@ -2711,13 +2737,13 @@ __global__ __launch_bounds__(256) void k_panel_rows(const int* list, int count, 
   auto group = [&](auto nb, auto bb, auto ss) {
     constexpr int N = decltype(nb)::value, B = decltype(bb)::value, S = decltype(ss)::value;
     if constexpr (B < N && 16 * B + 4 * S < PP) {
-      const double y = x[B][S];
       substStep<S>(x[B], Pm[16 * B + lr][16 * B + 4 * S + lk]);
+      const double y = x[B][S];
 #pragma unroll
       for (int rb = B + 1; rb < N; ++rb) x[rb] = mfma64(Pm[16 * rb + lr][16 * B + 4 * S + lk], y, x[rb]);
     }
   };
-  auto solve = [&](auto nb) {  // no branches: see settle
+  auto solve = [&](auto nb) __attribute__((always_inline)) {  // no branches: see settle
     auto block = [&](auto bb) {
       group(nb, bb, std::integral_constant<int, 0>{});
       group(nb, bb, std::integral_constant<int, 1>{});
@@ -2752,7 +2778,11 @@ __global__ __launch_bounds__(256) void k_panel_rows(const int* list, int count, 
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) l[b][u] = x[b][u] * cSelf[min(16 * b + 4 * u + lk, PP - 1)];
+    for (int u = 0; u < 4; ++u) {
+      const int q = min(16 * b + 4 * u + lk, PP - 1);
+      const double own = x[b][u] * cSelf[q];
+      l[b][u] = pkd[q] == 1 ? static_cast<double>(multiplier<T>(x[b][u], cDiv[q], cSelf[q])) : own;
+    }
   if (any2) {
     // columns q + 1 and q - 1 of the same row: the neighbouring 16-lane
     // group, in the next or previous register where the group wraps
