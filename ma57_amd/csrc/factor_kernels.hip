@@ -1254,8 +1254,13 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
   // below k (attained)
   auto generalStep = [&](double lam) {
     const double akk = curK(k);
-    if (lam <= prm.zeroTol) {  // dense_kernel.hpp:601-616: the block test failed on the isolated-pivot floor
-      stop = true;
+    if (lam <= prm.zeroTol) {
+      // dense_kernel.hpp:601-616: the block test failed on the isolated-pivot
+      // floor, which NaN does not lie below
+      if (fabs(akk) <= isolatedFloor)
+        stop = true;
+      else
+        accept1([&](int i) { return curK(i); }, akk);
       return;
     }
     if (kInLds && farStores) {
