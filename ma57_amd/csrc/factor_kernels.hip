@@ -912,11 +912,40 @@ template <int J>
 __device__ inline double bcast16(double v) {
   return __longlong_as_double(__builtin_amdgcn_update_dpp(0ll, __double_as_longlong(v), 0x150 + J, 0xf, 0xf, true));
 }
-// a += (lane J's v of each 16-lane group) * w in one instruction; the caller
-// leaves two wait states after the last write of v.
-template <int J>
-__device__ inline void fmaBcast16(double& a, double v, double w) {
-  asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(v), "v"(w), "n"(J));
+// a[j] += (lane j's v of each 16-lane group) * w for j = J .. J + N - 1, one
+// instruction each.  A DPP operand must have been written two wait states
+// before: they stand in the same asm statement as the reads, so no copy or
+// reload of v by the compiler can come between.
+template <int J, int N, int M>
+__device__ inline void fmaBcast16(double (&a)[M], double v, double w) {
+#define DPP_FMA(acc, src, mul, lane) "\n\tv_fmac_f64_dpp %" #acc ", %" #src ", %" #mul " row_newbcast:%" #lane " row_mask:0xf bank_mask:0xf"
+  if constexpr (N >= 4) {
+    asm("s_nop 1" DPP_FMA(0, 4, 5, 6) DPP_FMA(1, 4, 5, 7) DPP_FMA(2, 4, 5, 8) DPP_FMA(3, 4, 5, 9)
+        : "+&v"(a[J]), "+&v"(a[J + 1]), "+&v"(a[J + 2]), "+&v"(a[J + 3])
+        : "v"(v), "v"(w), "n"(J), "n"(J + 1), "n"(J + 2), "n"(J + 3));
+    fmaBcast16<J + 4, N - 4>(a, v, w);
+  } else if constexpr (N >= 2) {
+    asm("s_nop 1" DPP_FMA(0, 2, 3, 4) DPP_FMA(1, 2, 3, 5)
+        : "+&v"(a[J]), "+&v"(a[J + 1])
+        : "v"(v), "v"(w), "n"(J), "n"(J + 1));
+    fmaBcast16<J + 2, N - 2>(a, v, w);
+  } else if constexpr (N == 1) {
+    asm("s_nop 1" DPP_FMA(0, 1, 2, 3) : "+v"(a[J]) : "v"(v), "v"(w), "n"(J));
+  }
+#undef DPP_FMA
+}
+// a0 and a1 += (lane J's v of each 16-lane group) * b[J] for J = 0 .. 15, the
+// even J into a0 and the odd ones into a1
+__device__ inline void dotBcast16(double& a0, double& a1, double v, const double (&b)[16]) {
+#define DPP_FMA(acc, src, mul, lane) "\n\tv_fmac_f64_dpp %" #acc ", %" #src ", %" #mul " row_newbcast:" #lane " row_mask:0xf bank_mask:0xf"
+  asm("s_nop 1" DPP_FMA(0, 2, 3, 0) DPP_FMA(1, 2, 4, 1) DPP_FMA(0, 2, 5, 2) DPP_FMA(1, 2, 6, 3) DPP_FMA(0, 2, 7, 4)
+      DPP_FMA(1, 2, 8, 5) DPP_FMA(0, 2, 9, 6) DPP_FMA(1, 2, 10, 7) DPP_FMA(0, 2, 11, 8) DPP_FMA(1, 2, 12, 9)
+      DPP_FMA(0, 2, 13, 10) DPP_FMA(1, 2, 14, 11) DPP_FMA(0, 2, 15, 12) DPP_FMA(1, 2, 16, 13)
+      DPP_FMA(0, 2, 17, 14) DPP_FMA(1, 2, 18, 15)
+      : "+&v"(a0), "+&v"(a1)
+      : "v"(v), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]), "v"(b[8]),
+        "v"(b[9]), "v"(b[10]), "v"(b[11]), "v"(b[12]), "v"(b[13]), "v"(b[14]), "v"(b[15]));
+#undef DPP_FMA
 }
 
 template <int... I, typename Fn>
@@ -950,14 +979,10 @@ __device__ inline void blockFactor16(double (&a)[16], Block16& B, PivotOf pivotO
   double akk = a[0];
   unrolled(std::make_integer_sequence<int, 16>{}, [&](auto qq) {
     constexpr int q = decltype(qq)::value;
-    double l = static_cast<double>(static_cast<T>(pivotQuot(a[q], pivotOf(q, bcast16<q>(a[q])))));
+    const double l = static_cast<double>(static_cast<T>(pivotQuot(a[q], pivotOf(q, bcast16<q>(a[q])))));
     const double c = -a[q];
     if (q > 0) akk = i == q ? a[q] : akk;
-    asm volatile("s_nop 1" : "+v"(l));
-    unrolled(std::make_integer_sequence<int, 15 - q>{}, [&](auto jj) {
-      constexpr int j = q + 1 + decltype(jj)::value;
-      fmaBcast16<j>(a[j], l, c);
-    });
+    fmaBcast16<q + 1, 15 - q>(a, l, c);
     a[q] = l;
   });
   const double d = pivotOf(i, akk);
@@ -1307,11 +1332,7 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
         } else {
           loadWiden<16>(lv, F, [&](int u) -> int64_t { return at(i, k0 + min(q + u, p - 1)); });
         }
-        unrolled(std::make_integer_sequence<int, 8>{}, [&](auto uu) {
-          constexpr int u = 2 * decltype(uu)::value;
-          fmaBcast16<u>(a0, w16, lv[u]);
-          fmaBcast16<u + 1>(a1, w16, lv[u + 1]);
-        });
+        dotBcast16(a0, a1, w16, lv);
       }
       const double c = raw - (a0 + a1);
       if (ok) curR(i) = c;
