@@ -1051,6 +1051,14 @@ __global__ __launch_bounds__(256) void k_front_maxabs(const int* list, int count
 // the earlier multipliers, the interchanges and the general step's columns
 // cost no memory round trip.
 //
+// Where a wide panel's blocks (TPW >= 8 or streamed) keep fewer than four of
+// their columns, columns are formed one by one on the general step's buffers
+// until four in turn pass their test: a block of 4,000 rows costs 80 us
+// whatever it keeps, a column alone 15.  Random dense fronts (a failing column
+// in every second; blocks throughout -> here; sub-panels of four and eight
+// columns before the blocks): a panel of 4,000 rows 3.7 -> 1.9 ms (2.6),
+// 2,000 rows 2.0 -> 1.3 (1.9), 1,000 rows 1.26 -> 0.95 (1.3).
+//
 // Measured per panel of 64 columns (FP64, before: sub-panels of eight columns
 // in LDS, each thread factoring the 8 x 8 block, rows loaded slot by slot):
 // 30x30x30 27-point fronts, few failing columns, <= 128 rows 103 -> 24 us,
@@ -1059,6 +1067,7 @@ __global__ __launch_bounds__(256) void k_front_maxabs(const int* list, int count
 // 15,000 cycles there (6,000 of them the diagonal block), a general step
 // 8,000.
 constexpr int kPanelCols = 16;  // columns per block
+constexpr int kAloneRun = 4;    // a block that keeps fewer columns is followed by columns one by one
 template <int TPW, typename T>
 struct PanelShape {
   static constexpr int kRows = 128 * TPW;
@@ -1080,6 +1089,7 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
   constexpr int CT = TPW > 0 ? TPW : 8;                  // tiles per wave of a chunk
   constexpr int GT = CT < 4 ? CT : (TPW >= 16 ? 2 : 4);  // tiles whose loads are in flight together
   constexpr int LR = TPW > 0 ? Shape::kRows : 1;         // rows of the column buffers kept in LDS
+  constexpr bool kWide = TPW == 0 || TPW >= 8;           // columns one by one where the blocks keep few of theirs
   extern __shared__ double dynLds[];
   T* const Lp = reinterpret_cast<T*>(dynLds);  // panel column k0 + q, row k0 + i at [q * LD + i]
   __shared__ double bufK[LR], bufR[LR];        // current columns k and r of a general step, row k0 + i at [i]
@@ -1087,7 +1097,7 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
   __shared__ double Ds[SW][SW + 1];            // diagonal block
   __shared__ Block16 blk;
   __shared__ double redM[NW][SW];              // per-wave column maxima
-  __shared__ double redS[NW], redT[NW], redV[NW + 1];
+  __shared__ double redS[NW], redT[NW], redL[NW], redV[NW + 1];
   __shared__ int redI[NW];
   // pivot q of the panel, at [q + 1]: (D L^T)(q, row) = pdd l_q + pnx l_(q+1) + ppv l_(q-1)
   // (the neighbours: the other column of a 2x2 pivot)
@@ -1217,29 +1227,43 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
     return pdd[q + 1] * l + (has2 ? pnx[q + 1] * n + ppv[q + 1] * v : 0.0);
   };
   // symmetric interchange of positions a < b in storage (all rows, incl. the
-  // factored part and the not-fully-summed rows)
+  // factored part and the not-fully-summed rows), the values of S turns of a
+  // thread loaded before any is stored
   auto swapSym = [&](int a, int b) {
-    for (int t = tid; t < m; t += NT) {
-      if (t == b) continue;
-      // (a, t) and (b, t), each read from the lower triangle; (a, a) and (b, b) for t = a
-      const int i1 = max(a, t), j1 = min(a, t);
-      const int i2 = t == a ? b : max(b, t), j2 = t == a ? b : min(b, t);
-      if constexpr (kInLds) {
-        // both values loaded before either is stored, one memory round trip
-        const bool in1 = inLds(i1, j1), in2 = inLds(i2, j2);
-        T x = Lp[in1 ? ldsAt(i1, j1) : 0], y = Lp[in2 ? ldsAt(i2, j2) : 0];
-        if (!in1 || !in2) {
-          const T gx = F[in1 ? 0 : at(i1, j1)], gy = F[in2 ? 0 : at(i2, j2)];
-          x = in1 ? x : gx;
-          y = in2 ? y : gy;
+    constexpr int S = kInLds ? 1 : 4;
+    for (int t0 = tid; t0 < m; t0 += S * NT) {
+      T x[S], y[S];
+      int i1[S], j1[S], i2[S], j2[S];
+      bool ok[S];
+#pragma unroll
+      for (int u = 0; u < S; ++u) {
+        // (a, t) and (b, t), each read from the lower triangle; (a, a) and (b, b) for t = a
+        const int t = t0 + u * NT;
+        ok[u] = t < m && t != b;
+        i1[u] = ok[u] ? max(a, t) : 0;
+        j1[u] = ok[u] ? min(a, t) : 0;
+        i2[u] = ok[u] ? (t == a ? b : max(b, t)) : 0;
+        j2[u] = ok[u] ? (t == a ? b : min(b, t)) : 0;
+        if constexpr (kInLds) {
+          const bool in1 = inLds(i1[u], j1[u]), in2 = inLds(i2[u], j2[u]);
+          x[u] = Lp[in1 ? ldsAt(i1[u], j1[u]) : 0];
+          y[u] = Lp[in2 ? ldsAt(i2[u], j2[u]) : 0];
+          if (!in1 || !in2) {
+            const T gx = F[in1 ? 0 : at(i1[u], j1[u])], gy = F[in2 ? 0 : at(i2[u], j2[u])];
+            x[u] = in1 ? x[u] : gx;
+            y[u] = in2 ? y[u] : gy;
+          }
+        } else {
+          x[u] = F[at(i1[u], j1[u])];
+          y[u] = F[at(i2[u], j2[u])];
         }
-        put(i1, j1, y);
-        put(i2, j2, x);
-      } else {
-        const T x = F[at(i1, j1)], y = F[at(i2, j2)];
-        F[at(i1, j1)] = y;
-        F[at(i2, j2)] = x;
       }
+#pragma unroll
+      for (int u = 0; u < S; ++u)
+        if (ok[u]) {
+          put(i1[u], j1[u], y[u]);
+          put(i2[u], j2[u], x[u]);
+        }
     }
     if (tid == 0) {
       const int tp = fd.perm[io + a];
@@ -1273,6 +1297,48 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
     sync();
     ++k;
     ++p;
+  };
+  // out(i) = current column col of the held rows; returns the thread's max
+  // over its eligible rows but col.  Lane q keeps the weight of pivot q; RG
+  // groups of 64 rows per wave are in flight together.
+  auto currentColumn = [&](int col, auto&& out) -> double {
+    constexpr int RG = kWide ? 2 : 1;
+    const double wq = lane < p ? weight(lane, col) : 0.0;
+    double v = 0.0;
+    for (int i0 = k + 64 * wv; i0 < rEnd; i0 += RG * NT) {  // whole waves: the DPP operands come from every lane
+      int i[RG];
+      bool ok[RG];
+      double raw[RG], a0[RG], a1[RG];
+#pragma unroll
+      for (int g = 0; g < RG; ++g) {
+        ok[g] = i0 + g * NT + lane < rEnd;
+        i[g] = ok[g] ? i0 + g * NT + lane : rEnd - 1;
+        raw[g] = static_cast<double>(get(max(i[g], col), min(i[g], col)));
+        a0[g] = a1[g] = 0.0;
+      }
+#pragma unroll 1
+      for (int q = 0; q < p; q += 16) {
+        const double w16 = __shfl(wq, q + lr, 64);  // the weights past p are zero
+        double lv[RG][16];
+        if constexpr (kInLds) {
+#pragma unroll
+          for (int u = 0; u < 16; ++u) lv[0][u] = static_cast<double>(Lp[min(q + u, p - 1) * LD + (i[0] - k0)]);
+        } else {
+#pragma unroll
+          for (int g = 0; g < RG; ++g)
+            loadWiden<16>(lv[g], F, [&](int u) -> int64_t { return at(i[g], k0 + min(q + u, p - 1)); });
+        }
+#pragma unroll
+        for (int g = 0; g < RG; ++g) dotBcast16(a0[g], a1[g], w16, lv[g]);
+      }
+#pragma unroll
+      for (int g = 0; g < RG; ++g) {
+        const double c = raw[g] - (a0[g] + a1[g]);
+        if (ok[g]) out(i[g]) = c;
+        if (ok[g] && i[g] < nE && i[g] != col) v = fmax(v, fabs(c));
+      }
+    }
+    return v;
   };
   // one general step at pivot k (sigma test, swaps, 1x1 or 2x2, or a stop);
   // curK holds the current column k, lam = max |curK| over the eligible rows
@@ -1313,31 +1379,8 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
       stop = true;
       return;
     }
-    // curR = current column r; sigma = its max over the eligible rows but r
-    // (dense_kernel.hpp:628-633); lane q keeps the weight of pivot q
-    const double wq = lane < p ? weight(lane, r) : 0.0;
-    double sg = 0.0;
-    for (int i0 = k + 64 * wv; i0 < rEnd; i0 += NT) {  // whole waves: the DPP operands come from every lane
-      const bool ok = i0 + lane < rEnd;
-      const int i = ok ? i0 + lane : rEnd - 1;
-      const double raw = static_cast<double>(i >= r ? get(i, r) : get(r, i));
-      double a0 = 0.0, a1 = 0.0;
-#pragma unroll 1
-      for (int q = 0; q < p; q += 16) {
-        const double w16 = __shfl(wq, q + lr, 64);  // the weights past p are zero
-        double lv[16];
-        if constexpr (kInLds) {
-#pragma unroll
-          for (int u = 0; u < 16; ++u) lv[u] = static_cast<double>(Lp[min(q + u, p - 1) * LD + (i - k0)]);
-        } else {
-          loadWiden<16>(lv, F, [&](int u) -> int64_t { return at(i, k0 + min(q + u, p - 1)); });
-        }
-        dotBcast16(a0, a1, w16, lv);
-      }
-      const double c = raw - (a0 + a1);
-      if (ok) curR(i) = c;
-      if (ok && i < nE && i != r) sg = fmax(sg, fabs(c));
-    }
+    // sigma: the max of the current column r over the eligible rows but r (dense_kernel.hpp:628-633)
+    double sg = currentColumn(r, curR);
     sg = __ockl_wfred_max_f64(sg);
     const double tm = __ockl_wfred_max_f64(tmax);
     if (lane == 0) {
@@ -1411,19 +1454,21 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
       else
         return F[ok ? at(row, k0 + q) : 0];
     };
+    int lrL = lr;  // (see acceptChunk)
+    asm volatile("" : "+v"(lrL));
     T raw[NTL][4];
 #pragma unroll
     for (int t = 0; t < NTL; ++t)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int row = row0(t) + lr, col = 4 * u + lk;
+        const int row = row0(t) + lrL, col = 4 * u + lk;
         raw[t][u] = entry(row, c0 - k0 + col, row < rEnd && col < sw && row >= c0 + col);
       }
 #pragma unroll
     for (int t = 0; t < NTL; ++t)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int row = row0(t) + lr, col = 4 * u + lk;
+        const int row = row0(t) + lrL, col = 4 * u + lk;
         x[t][u] = row < rEnd && col < sw && row >= c0 + col ? static_cast<double>(raw[t][u]) : 0.0;
       }
     // operands of 16 pivots
@@ -1434,7 +1479,7 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
       for (int t = 0; t < NTL; ++t)
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const int row = row0(t) + lr, q = q0 + 4 * u + lk;
+          const int row = row0(t) + lrL, q = q0 + 4 * u + lk;
           l[t][u] = entry(row, q, row >= c0 && row < rEnd && q < p);
         }
 #pragma unroll
@@ -1454,7 +1499,7 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
       for (int u = 0; u < 4; ++u)
 #pragma unroll
         for (int t = 0; t < NTL; ++t) {
-          const int row = row0(t) + lr, q = q0 + 4 * u + lk;
+          const int row = row0(t) + lrL, q = q0 + 4 * u + lk;
           const double l = row >= c0 && row < rEnd && q < p ? static_cast<double>(lv[t][u]) : 0.0;
           x[t] = mfma64(w[u], l, x[t]);
         }
@@ -1481,7 +1526,24 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
     for (int t = 0; t < NTL; ++t) settle(x[t]);
   };
 
+  int passed = kAloneRun;  // columns that passed the first test since one failed
   while (k < nbEnd && !stop) {
+    if (kWide && passed < kAloneRun) {
+      double lam = __ockl_wfred_max_f64(currentColumn(k, curK));
+      if (lane == 0) redL[wv] = lam;
+      sync();
+#pragma unroll
+      for (int w = 0; w < NW; ++w) lam = fmax(lam, redL[w]);
+      const double akk = curK(k);
+      if (lam <= prm.zeroTol ? fabs(akk) > isolatedFloor : fabs(akk) >= kAlpha * lam) {
+        accept1([&](int i) { return curK(i); }, akk);
+        ++passed;
+      } else {
+        generalStep(lam);
+        passed = 0;
+      }
+      continue;
+    }
     const int c0 = k, sw = min(SW, nbEnd - k);
     if constexpr (!kInLds) {
       // weights of the earlier pivots at the block's rows
@@ -1599,10 +1661,14 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
       dc[u] = blk.d[4 * u + lk];
       rdc[u] = blk.rd[4 * u + lk];
     }
+    // (rows from an index that the compiler cannot match with the loads': their
+    // 4 CT addresses would stay in registers over the whole block)
+    int lrA = lr;
+    asm volatile("" : "+v"(lrA));
     auto acceptChunk = [&](int ch) {
 #pragma unroll
       for (int t = 0; t < CT; ++t) {
-        const int row0 = rowOf(ch, t), row = row0 + lr;
+        const int row0 = rowOf(ch, t), row = row0 + lrA;
         T lt[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) lt[u] = multiplier<T>(x[t][u], dc[u], rdc[u]);
@@ -1657,6 +1723,7 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
         ++npert;
       }
     }
+    if (kWide) passed = qs < min(kAloneRun, sw) ? 0 : kAloneRun;
     const double lamF = readLane(lam, min(qs, SW - 1));
     sync();
     k += qs;
