@@ -842,6 +842,9 @@ __device__ inline v4d mfma64(double a, double b, v4d c) { return __builtin_amdgc
 // distance along the longer way.  So every result of which only a part is
 // used, or which is read after a branch, is settled whole.
 __device__ inline void settle(v4d& x) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x)); }
+__device__ inline void settle(v4d (&x)[4]) {
+  asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]));
+}
 
 // Workgroup barrier that orders LDS accesses only: stores to global memory
 // stay in flight across it.
@@ -905,6 +908,63 @@ __device__ inline void substTile(v4d& x, const double (&op)[4]) {
   substStep<1>(x, op[1]);
   substStep<2>(x, op[2]);
   substStep<3>(x, op[3]);
+}
+
+// 4 x 4 transpose of the 16-lane rows of four registers: row g of v[k] and
+// row k of v[g] change places.
+__device__ inline void transposeRows(double (&v)[4]) {
+  uint32_t w[2][4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    w[0][k] = static_cast<uint32_t>(__double2loint(v[k]));
+    w[1][k] = static_cast<uint32_t>(__double2hiint(v[k]));
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const auto a = __builtin_amdgcn_permlane16_swap(w[h][0], w[h][1], false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(w[h][2], w[h][3], false, false);
+    const auto c = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+    const auto d = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+    w[h][0] = c[0];
+    w[h][1] = d[0];
+    w[h][2] = c[1];
+    w[h][3] = d[1];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = __hiloint2double(static_cast<int>(w[1][k]), static_cast<int>(w[0][k]));
+}
+
+// The same substitution of four tiles at once, with the same operations on
+// every row: transposed, a lane holds the four columns of one row of one
+// tile, so that the six dependent products serve four tiles and no lane
+// repeats another's.
+template <int S>
+__device__ inline void substStep4(v4d* x, double a) {
+  auto l = [&](int i, int k) { return readLane(a, 4 * S + i + 16 * k); };
+  double y[4] = {x[0][S], x[1][S], x[2][S], x[3][S]};
+  transposeRows(y);
+  y[1] = fma(l(1, 0), y[0], y[1]);
+  y[2] = fma(l(2, 1), y[1], fma(l(2, 0), y[0], y[2]));
+  y[3] = fma(l(3, 2), y[2], fma(l(3, 1), y[1], fma(l(3, 0), y[0], y[3])));
+  transposeRows(y);
+  if constexpr (S < 3) {
+    v4d d[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) d[t] = mfma64(a, y[t], x[t]);
+    settle(d);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = S + 1; r < 4; ++r) x[t][r] = d[t][r];
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t) x[t][S] = y[t];
+}
+__device__ inline void substTiles4(v4d* x, const double (&op)[4]) {
+  substStep4<0>(x, op[0]);
+  substStep4<1>(x, op[1]);
+  substStep4<2>(x, op[2]);
+  substStep4<3>(x, op[3]);
 }
 
 // Lane J of each 16-lane group in every lane of the group.
@@ -1611,15 +1671,21 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
     // substitution of the held rows and the maxima over the eligible rows below each pivot
     double vm[4] = {0.0, 0.0, 0.0, 0.0};
     auto solveChunk = [&](int ch) {
+      constexpr int ST = CT >= 4 ? 4 : 1;  // tiles substituted together
 #pragma unroll
-      for (int t = 0; t < CT; ++t) {
-        const int row0 = rowOf(ch, t);
-        if (row0 < rEnd && row0 + 16 > c0) {
-          substTile(x[t], op);
-          const int row = row0 + lr;
+      for (int t0 = 0; t0 < CT; t0 += ST) {
+        if (rowOf(ch, t0) < rEnd && rowOf(ch, t0 + ST - 1) + 16 > c0) {
+          if constexpr (ST == 4)
+            substTiles4(&x[t0], op);
+          else
+            substTile(x[t0], op);
 #pragma unroll
-          for (int u = 0; u < 4; ++u)
-            vm[u] = fmax(vm[u], row < nE && row > c0 + 4 * u + lk ? fabs(x[t][u]) : 0.0);
+          for (int t = t0; t < t0 + ST; ++t) {
+            const int row = rowOf(ch, t) + lr;
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              vm[u] = fmax(vm[u], row < nE && row > c0 + 4 * u + lk ? fabs(x[t][u]) : 0.0);
+          }
         }
       }
     };
