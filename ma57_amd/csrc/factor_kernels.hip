@@ -1111,13 +1111,15 @@ __global__ __launch_bounds__(256) void k_front_maxabs(const int* list, int count
 // the earlier multipliers, the interchanges and the general step's columns
 // cost no memory round trip.
 //
-// Where a wide panel's blocks (TPW >= 8 or streamed) keep fewer than four of
-// their columns, columns are formed one by one on the general step's buffers
-// until four in turn pass their test: a block of 4,000 rows costs 80 us
-// whatever it keeps, a column alone 15.  Random dense fronts (a failing column
-// in every second; blocks throughout -> here; sub-panels of four and eight
-// columns before the blocks): a panel of 4,000 rows 3.7 -> 1.9 ms (2.6),
-// 2,000 rows 2.0 -> 1.3 (1.9), 1,000 rows 1.26 -> 0.95 (1.3).
+// Where three blocks in turn of a panel with more than 256 rows keep few of
+// their columns (kPoorBlock), columns are formed one by one on the general
+// step's buffers until four in turn pass their test: a block costs the same
+// whatever it keeps (75 us at 4,000 rows, 19 at 1,000).  After one poor block already, fronts with a failing column in every
+// fifth lost more than they gained (192 systems, 1,024-row panels: 353 -> 422
+// us; after three 365).  Random dense fronts (a failing column in every
+// second), a panel of 4,000 rows: blocks throughout 3.7 ms, here 1.9 (sub-panels
+// of four and eight columns before the blocks: 2.6); 2,000 rows 2.0 -> 1.1
+// (1.9); 1,000 rows 1.26 -> 0.72 (1.33).
 //
 // Measured per panel of 64 columns (FP64, before: sub-panels of eight columns
 // in LDS, each thread factoring the 8 x 8 block, rows loaded slot by slot):
@@ -1127,10 +1129,12 @@ __global__ __launch_bounds__(256) void k_front_maxabs(const int* list, int count
 // 15,000 cycles there (6,000 of them the diagonal block), a general step
 // 8,000.
 constexpr int kPanelCols = 16;  // columns per block
-constexpr int kAloneRun = 4;    // a block that keeps fewer columns is followed by columns one by one
+constexpr int kAloneAfter = 3;  // poor blocks in turn before columns are taken one by one,
+constexpr int kAloneRun = 4;    // until so many have passed in turn
 template <int TPW, typename T>
 struct PanelShape {
   static constexpr int kRows = 128 * TPW;
+  static constexpr int kPoorBlock = TPW == 4 || TPW == 8 ? 2 : 4;  // columns kept
   // column stride in LDS: half the banks on from one column to the next, so
   // the four columns of an operand read do not collide
   static constexpr int kLd = kRows + 16;
@@ -1149,7 +1153,7 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
   constexpr int CT = TPW > 0 ? TPW : 8;                  // tiles per wave of a chunk
   constexpr int GT = CT < 4 ? CT : (TPW >= 16 ? 2 : 4);  // tiles whose loads are in flight together
   constexpr int LR = TPW > 0 ? Shape::kRows : 1;         // rows of the column buffers kept in LDS
-  constexpr bool kWide = TPW == 0 || TPW >= 8;           // columns one by one where the blocks keep few of theirs
+  constexpr bool kWide = TPW == 0 || TPW >= 4;           // columns one by one where the blocks keep few of theirs
   extern __shared__ double dynLds[];
   T* const Lp = reinterpret_cast<T*>(dynLds);  // panel column k0 + q, row k0 + i at [q * LD + i]
   __shared__ double bufK[LR], bufR[LR];        // current columns k and r of a general step, row k0 + i at [i]
@@ -1360,9 +1364,10 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
   };
   // out(i) = current column col of the held rows; returns the thread's max
   // over its eligible rows but col.  Lane q keeps the weight of pivot q; RG
-  // groups of 64 rows per wave are in flight together.
+  // groups of 64 rows per wave are in flight together (two where every panel
+  // has rows for them).
   auto currentColumn = [&](int col, auto&& out) -> double {
-    constexpr int RG = kWide ? 2 : 1;
+    constexpr int RG = TPW == 0 || TPW >= 16 ? 2 : 1;
     const double wq = lane < p ? weight(lane, col) : 0.0;
     double v = 0.0;
     for (int i0 = k + 64 * wv; i0 < rEnd; i0 += RG * NT) {  // whole waves: the DPP operands come from every lane
@@ -1586,7 +1591,9 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
     for (int t = 0; t < NTL; ++t) settle(x[t]);
   };
 
-  int passed = kAloneRun;  // columns that passed the first test since one failed
+  // columns that passed the first test since one failed; once two blocks in
+  // turn kept few of theirs it starts at zero
+  int passed = kAloneRun, poor = 0;
   while (k < nbEnd && !stop) {
     if (kWide && passed < kAloneRun) {
       double lam = __ockl_wfred_max_f64(currentColumn(k, curK));
@@ -1789,7 +1796,10 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
         ++npert;
       }
     }
-    if (kWide) passed = qs < min(kAloneRun, sw) ? 0 : kAloneRun;
+    if (kWide) {
+      poor = qs < min(Shape::kPoorBlock, sw) ? poor + 1 : 0;
+      if (poor == kAloneAfter) passed = poor = 0;
+    }
     const double lamF = readLane(lam, min(qs, SW - 1));
     sync();
     k += qs;
