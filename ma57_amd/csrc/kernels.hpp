@@ -79,7 +79,7 @@ void launchDiagInverse(const int* list, int count, const int* blockStart, int bl
 // the chain kernels take about 5 us a block)
 constexpr int kOwnMaxBlocks = 6;
 void launchFwdOwn(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* Z, double* Dl,
-                  const int64_t* gOff, const double* inv, const int64_t* invOff, hipStream_t st);
+                  const int64_t* gOff, int* err, const double* inv, const int64_t* invOff, hipStream_t st);
 // own rows, one workgroup per own block (blockStart: ceil(nF / kSolveBlock) per front), dependency flags
 void launchFwdChain(const int* list, int count, const int* blockStart, int blocks, const DevFronts& fd, int nrhs,
                     double* Z, double* Dl, const int64_t* gOff, unsigned* flags, const int64_t* flagOff,
@@ -93,7 +93,7 @@ void launchBwdAnc(const int* list, int count, const int* blockStart, int blocks,
                   hipStream_t st);
 void launchBwdOwn(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* X,
                   const double* Dl,
-                  const int64_t* gOff, const AncPart* parts, const double* inv, const int64_t* invOff,
+                  const int64_t* gOff, const AncPart* parts, int* err, const double* inv, const int64_t* invOff,
                   hipStream_t st);
 void launchBwdChain(const int* list, int count, const int* blockStart, int blocks, const DevFronts& fd, int nrhs,
                     double* X, double* Dl, const int64_t* gOff, const AncPart* parts, unsigned* flags,

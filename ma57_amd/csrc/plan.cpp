@@ -1220,7 +1220,8 @@ void Plan::solveCore(const double* dB, int64_t ldb, int nrhs, double* dX, int64_
     const SolveLevel& lv = solveLv_[L];
     profBegin(kProfFwd);
     launchFwdGather(dposInfo_.p + lv.posOff, lv.positions, nrhs, w.Bp, w.Dl, dmapRow_.p, stream_);
-    launchFwdOwn(lists + lv.own.list, lv.own.count, lv.own.maxBlocks, fd, nrhs, w.Z, w.Dl, dgOff_.p, dinv_.p, dinvOff_.p, stream_);
+    launchFwdOwn(lists + lv.own.list, lv.own.count, lv.own.maxBlocks, fd, nrhs, w.Z, w.Dl, dgOff_.p, err, dinv_.p,
+                 dinvOff_.p, stream_);
     launchFwdChain(lists + lv.chain.list, lv.chain.count, starts + lv.chain.start, lv.chain.blocks, fd, nrhs, w.Z,
                    w.Dl, dgOff_.p, dflagsF_.p, dflagOff_.p, dgen_.p, err, dinv_.p, dinvOff_.p, stream_);
     launchFwdDelta(lists + lv.delta.list, lv.delta.count, starts + lv.delta.start, lv.delta.blocks, fd, nrhs, w.Dl,
@@ -1233,8 +1234,8 @@ void Plan::solveCore(const double* dB, int64_t ldb, int nrhs, double* dX, int64_
     profBegin(kProfBwd);
     launchBwdAnc(lists + lv.anc.list, lv.anc.count, starts + lv.anc.start, lv.anc.blocks, fd, nrhs, w.Z, w.X, w.Dl,
                  dgOff_.p, dancPart_.p, err, stream_);
-    launchBwdOwn(lists + lv.own.list, lv.own.count, lv.own.maxBlocks, fd, nrhs, w.X, w.Dl, dgOff_.p, dancPart_.p, dinv_.p, dinvOff_.p,
-                 stream_);
+    launchBwdOwn(lists + lv.own.list, lv.own.count, lv.own.maxBlocks, fd, nrhs, w.X, w.Dl, dgOff_.p,
+                 dancPart_.p, err, dinv_.p, dinvOff_.p, stream_);
     launchBwdChain(lists + lv.chain.list, lv.chain.count, starts + lv.chain.start, lv.chain.blocks, fd, nrhs, w.X,
                    w.Dl, dgOff_.p, dancPart_.p, dflagsB_.p, dflagOff_.p, dgen_.p, err, dinv_.p, dinvOff_.p,
                    stream_);

@@ -690,17 +690,22 @@ __device__ inline v4d ownMma(double a, double b, v4d c) { return __builtin_amdgc
 // read's distance from it along the longer way only (20 wait states cover it).
 __device__ inline void ownSettle(v4d& x) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x)); }
 
-// NB: most own blocks of a listed front.  Forward (solve.hpp:349-361,
+// NB: most own blocks of a listed front (one that has more raises the error
+// word and is left alone).  Forward (solve.hpp:349-361,
 // :434-455): y_b = L_bb^{-1} (y0_b - sum_{j<b} L_bj y_j), then z = D^{-1} y.
 template <typename T, int NB>
 __global__ __launch_bounds__(256) void k_fwd_own(const int* list, int count, DevFronts fd, int nrhs,
                                                  double* __restrict__ Z, double* __restrict__ Dl,
                                                  const int64_t* __restrict__ gOff, const double* __restrict__ inv,
-                                                 const int64_t* __restrict__ invOff) {
+                                                 const int64_t* __restrict__ invOff, int* err) {
   if (static_cast<int>(blockIdx.x) >= count) return;
   const int s = list[blockIdx.x];
   const int m = fd.m[s], nf = fd.nF[s];
   const int nOwn = (nf + SB - 1) / SB;
+  if (nOwn > NB) {  // the front outgrew the plan
+    if (threadIdx.x == 0) raiseError(err, 2);
+    return;
+  }
   const int64_t io = fd.idxOff[s];
   const int* pk = fd.pkind + io;
   const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
@@ -836,11 +841,16 @@ template <typename T, int NB>
 __global__ __launch_bounds__(256) void k_bwd_own(const int* list, int count, DevFronts fd, int nrhs,
                                                  double* __restrict__ X, const double* __restrict__ Dl,
                                                  const int64_t* __restrict__ gOff, const AncPart* __restrict__ parts,
-                                                 const double* __restrict__ inv, const int64_t* __restrict__ invOff) {
+                                                 const double* __restrict__ inv, const int64_t* __restrict__ invOff,
+                                                 int* err) {
   if (static_cast<int>(blockIdx.x) >= count) return;
   const int s = list[blockIdx.x];
   const int m = fd.m[s], nf = fd.nF[s];
   const int nOwn = (nf + SB - 1) / SB;
+  if (nOwn > NB) {  // the front outgrew the plan
+    if (threadIdx.x == 0) raiseError(err, 2);
+    return;
+  }
   const int64_t io = fd.idxOff[s];
   const int* pk = fd.pkind + io;
   const GlobalIn<T> F = globalIn(static_cast<const T*>(fd.F[s]));
@@ -1740,8 +1750,10 @@ void launchDiagInverse(const int* list, int count, const int* blockStart, int bl
 static int ownThreads(int nrhs) { return 64 * std::min(4, (nrhs + 15) / 16); }
 template <typename T>
 static void fwdOwnT(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* Z, double* Dl,
-                    const int64_t* gOff, const double* inv, const int64_t* invOff, hipStream_t st) {
-  auto go = [&](auto kernel) { kernel<<<count, ownThreads(nrhs), 0, st>>>(list, count, fd, nrhs, Z, Dl, gOff, inv, invOff); };
+                    const int64_t* gOff, int* err, const double* inv, const int64_t* invOff, hipStream_t st) {
+  auto go = [&](auto kernel) {
+    kernel<<<count, ownThreads(nrhs), 0, st>>>(list, count, fd, nrhs, Z, Dl, gOff, inv, invOff, err);
+  };
   if (maxBlocks <= 2)
     go(k_fwd_own<T, 2>);
   else if (maxBlocks <= 4)
@@ -1750,12 +1762,12 @@ static void fwdOwnT(const int* list, int count, int maxBlocks, const DevFronts& 
     go(k_fwd_own<T, kOwnMaxBlocks>);
 }
 void launchFwdOwn(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* Z, double* Dl,
-                  const int64_t* gOff, const double* inv, const int64_t* invOff, hipStream_t st) {
+                  const int64_t* gOff, int* err, const double* inv, const int64_t* invOff, hipStream_t st) {
   if (count <= 0 || nrhs <= 0) return;
   if (fd.fp32)
-    fwdOwnT<float>(list, count, maxBlocks, fd, nrhs, Z, Dl, gOff, inv, invOff, st);
+    fwdOwnT<float>(list, count, maxBlocks, fd, nrhs, Z, Dl, gOff, err, inv, invOff, st);
   else
-    fwdOwnT<double>(list, count, maxBlocks, fd, nrhs, Z, Dl, gOff, inv, invOff, st);
+    fwdOwnT<double>(list, count, maxBlocks, fd, nrhs, Z, Dl, gOff, err, inv, invOff, st);
   hipCheck(hipGetLastError(), "launchFwdOwn");
 }
 void launchFwdChain(const int* list, int count, const int* blockStart, int blocks, const DevFronts& fd, int nrhs,
@@ -1791,10 +1803,10 @@ void launchBwdAnc(const int* list, int count, const int* blockStart, int blocks,
 }
 template <typename T>
 static void bwdOwnT(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* X,
-                    const double* Dl, const int64_t* gOff, const AncPart* parts, const double* inv,
+                    const double* Dl, const int64_t* gOff, const AncPart* parts, int* err, const double* inv,
                     const int64_t* invOff, hipStream_t st) {
   auto go = [&](auto kernel) {
-    kernel<<<count, ownThreads(nrhs), 0, st>>>(list, count, fd, nrhs, X, Dl, gOff, parts, inv, invOff);
+    kernel<<<count, ownThreads(nrhs), 0, st>>>(list, count, fd, nrhs, X, Dl, gOff, parts, inv, invOff, err);
   };
   if (maxBlocks <= 2)
     go(k_bwd_own<T, 2>);
@@ -1804,13 +1816,13 @@ static void bwdOwnT(const int* list, int count, int maxBlocks, const DevFronts& 
     go(k_bwd_own<T, kOwnMaxBlocks>);
 }
 void launchBwdOwn(const int* list, int count, int maxBlocks, const DevFronts& fd, int nrhs, double* X,
-                  const double* Dl, const int64_t* gOff, const AncPart* parts, const double* inv,
+                  const double* Dl, const int64_t* gOff, const AncPart* parts, int* err, const double* inv,
                   const int64_t* invOff, hipStream_t st) {
   if (count <= 0 || nrhs <= 0) return;
   if (fd.fp32)
-    bwdOwnT<float>(list, count, maxBlocks, fd, nrhs, X, Dl, gOff, parts, inv, invOff, st);
+    bwdOwnT<float>(list, count, maxBlocks, fd, nrhs, X, Dl, gOff, parts, err, inv, invOff, st);
   else
-    bwdOwnT<double>(list, count, maxBlocks, fd, nrhs, X, Dl, gOff, parts, inv, invOff, st);
+    bwdOwnT<double>(list, count, maxBlocks, fd, nrhs, X, Dl, gOff, parts, err, inv, invOff, st);
   hipCheck(hipGetLastError(), "launchBwdOwn");
 }
 void launchBwdChain(const int* list, int count, const int* blockStart, int blocks, const DevFronts& fd, int nrhs,
