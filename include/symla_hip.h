@@ -283,8 +283,10 @@ int symla_dense_factor(int n, double* A, int lda, int n_eligible, const symla_de
 /* Scheduling choices of a plan (no counterpart in the reference, whose
  * front kernel is one CPU routine): fronts of order <= small_front_max
  * (at most 192, default 64) are factored whole in LDS, larger ones by the
- * panel path; assembly runs in column tiles of assemble_tile (a power of two
- * in [16, 1024]).  With speculative_panel set, each panel of a front with
+ * panel path; assembly runs in tiles of at most assemble_tile columns (a power
+ * of two in [16, 1024]; no tile is wider than 64, and fronts of more than 128
+ * rows always use 16, so it only matters below 64 and for small fronts).
+ * With speculative_panel set, each panel of a front with
  * more than speculative_min_rows eligible rows is first factored as 1x1
  * pivots in order and the threshold tests checked for all its columns at
  * once; the exact pivot-by-pivot kernel continues from the first column that
@@ -293,7 +295,7 @@ int symla_dense_factor(int n, double* A, int lda, int n_eligible, const symla_de
  * (device) with nrhs fixed pseudo-random right-hand sides, best of reps, in
  * the given precision, by coordinate descent from the plan's current
  * tuning: each choice in turn over its candidates (small_front_max 0..192,
- * assemble_tile 32/64/128, the speculative step off or from 0/1,024/2,048/
+ * assemble_tile 16/32/64, the speculative step off or from 0/1,024/2,048/
  * 4,096 rows, the deferred contribution-block bound off or 1,024/2,048/
  * 4,096) with the others fixed, the fastest kept, until a sweep changes
  * nothing.  It keeps the fastest (returned in *chosen) and reports every

@@ -18,6 +18,7 @@ void launchResetPerm(const int* list, int count, const DevFronts& fd, hipStream_
 // tasks of monotone assembly (child rows in the parent's order): front, first
 // and last column + 1 (may pass the front's end), first row of a tile of
 // kAsmEntries entries; otherwise front and columns
+constexpr int kAsmMaxCols = 64;    // columns of the widest tile
 constexpr int kAsmEntries = 4096;  // FP64: 32 KiB of LDS, four workgroups per CU with the spare slots
 void launchAssemble(const int4* tasks, int ntasks, const DevFronts& fd, const double* aVals, int monotone,
                     hipStream_t st);

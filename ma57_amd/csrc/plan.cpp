@@ -399,7 +399,7 @@ void Plan::buildSchedule() {
       // assembly tiles of kAsmEntries entries, 16 columns by 256 rows (a
       // child's column is read in runs of rows); a front that fits fewer rows
       // gets more columns, so that a tiny one is one workgroup
-      const int w = std::min(tune_.asmTile, hm_[s] <= 64 ? 64 : hm_[s] <= 128 ? 32 : 16);
+      const int w = std::min(tune_.asmTile, hm_[s] <= 64 ? kAsmMaxCols : hm_[s] <= 128 ? 32 : 16);
       for (int c0 = 0; c0 < hm_[s]; c0 += w)
         for (int r0 = c0; r0 < hm_[s]; r0 += kAsmEntries / w) tasks.push_back(make_int4(s, c0, c0 + w, r0));
       if (hm_[s] <= tune_.smallMax) {
@@ -1840,8 +1840,10 @@ std::vector<Plan::TuneTrial> Plan::autotune(const double* dVals, int nrhs, int p
   o.precision = precision == 2 ? 1 : precision;  // SYMLA_PREC_BF16X3: FP32 fronts, BF16x3 contribution blocks
   o.bf16x3 = precision == 2;
   std::vector<TuneTrial> trials;
+  // (assembly tiles past kAsmMaxCols columns are one schedule)
   auto same = [](const Tuning& a, const Tuning& b) {
-    return a.smallMax == b.smallMax && a.asmTile == b.asmTile && a.specPanel == b.specPanel &&
+    return a.smallMax == b.smallMax && std::min(a.asmTile, kAsmMaxCols) == std::min(b.asmTile, kAsmMaxCols) &&
+           a.specPanel == b.specPanel &&
            a.specMinRows == b.specMinRows && a.cbMinRows == b.cbMinRows;
   };
   auto timeOf = [&](const Tuning& t) {
@@ -1868,7 +1870,7 @@ std::vector<Plan::TuneTrial> Plan::autotune(const double* dVals, int nrhs, int p
   Tuning cur = tune_;
   double curMs = timeOf(cur);
   const int smalls[] = {0, 32, 64, 96, 128, 192};
-  const int tiles[] = {32, 64, 128};
+  const int tiles[] = {16, 32, kAsmMaxCols};
   const int specs[] = {-1, 0, 1024, 2048, 4096};  // -1: no speculative step
   const int cbs[] = {-1, 1024, 2048, 4096};
   for (int sweep = 0; sweep < 3; ++sweep) {

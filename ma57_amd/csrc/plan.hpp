@@ -255,7 +255,9 @@ class Plan {
   bool hasGraph() const { return graphExec_ != nullptr; }
 
   // Scheduling choices: fronts of order <= smallMax take the LDS kernel,
-  // larger ones the panel path; assembly tiles hold at most asmTile columns.
+  // larger ones the panel path; assembly tiles hold at most asmTile columns
+  // (16 to 1,024; past kAsmMaxCols no difference, and fronts of more than 128
+  // rows have tiles of 16 columns whatever it says).
   struct Tuning {
     // fronts up to this order are factored whole in LDS; larger ones (also the
     // few mid-size fronts of the upper levels, where one workgroup per front
