@@ -68,7 +68,8 @@ struct DevFronts {
   int* kcur;             // next pivot position (panel path)
   int* pcount;           // pivots in the last panel (panel path)
   int* stopped;          // 1 when a front stopped on a delay
-  int* cbDone;           // 1 when the speculative panel also wrote the last panel's rows [nE, m)
+  int* cbDone;           // 1 when the last panel's rows [nE, m) are written too: by a speculative step that passed
+                         // whole, or by the panel kernel, which holds all rows of such a front
   double* pert;          // static mode: sum |perturbation|
   int* npert;            // static mode: perturbed pivots
   unsigned long long* schurFlops;  // algorithmic flops of the MFMA trailing updates (p*r*(r+1) per update)

@@ -880,8 +880,10 @@ __device__ inline void rows16(double v, double (&x)[4]) {
 //
 // (The inverse of the group's 4 x 4 unit block on the matrix cores in place
 // of the six dependent products is as accurate only while the multipliers
-// are bounded: static pivots, random dense fronts of 300 rows, componentwise
-// backward error 1600 u in the worst of six, against 1.5 u.)
+// are bounded.  Static pivots on random dense fronts of 192 rows, emulated,
+// componentwise backward error: 21 u, 292 u in the worst of six, against 1.8
+// and 2.1 u; measured at 300 rows, with the block's rows rounded a second time
+// as well: 46 and 1600 u against 1.4 and 2.0.)
 template <int S>
 __device__ inline void substStep(v4d& x, double a) {
   auto l = [&](int i, int k) { return readLane(a, 4 * S + i + 16 * k); };
@@ -1032,7 +1034,8 @@ struct Block16 {
 // 8000 cycles).  The block's multipliers that the front keeps are these, not
 // ones that the substitution forms again: all later products of the block's
 // columns use these, and where static pivots make them large a second
-// rounding of the same values is a backward error of its own.
+// rounding of the same values is a backward error of its own (emulated as
+// above: 17 u, 386 u at worst).
 template <typename T, typename PivotOf>
 __device__ inline void blockFactor16(double (&a)[16], Block16& B, PivotOf pivotOf) {
   const int lane = threadIdx.x & 63, i = lane & 15, k = lane >> 4;
@@ -1104,7 +1107,8 @@ __global__ __launch_bounds__(256) void k_front_maxabs(const int* list, int count
 // What bounds it: the dependent chain (16 reciprocals per block, the
 // barriers, memory round trips), then for many rows the one CU's FP64 rate:
 // 64 columns of R rows take about 2048 R multiply-adds.  TPW 16-row tiles
-// per wave stay in registers (128 TPW rows); TPW = 0 streams any number of
+// per wave stay in registers (128 TPW rows; the 2,048-row variant reloads some
+// 64 values that do not change during the panel from scratch); TPW = 0 streams any number of
 // rows eight tiles at a time, with the block's current values in the
 // workspace between the test and the multipliers.  A panel of few rows
 // (PanelShape::kInLds) lives in LDS from its first load to its write-back, so
@@ -2539,8 +2543,8 @@ __global__ __launch_bounds__(256) void k_spec_block(const int* list, int count, 
 // them by the block's four 16-column blocks and stores the multipliers in the
 // front.  What a block takes off the later columns is the stored multiplier
 // times its pivot.  All operands come from the record in lane order, in
-// flight together with the rows, so the pass is one memory round trip, 40
-// dependent-chain MFMAs (2,600 cycles) and the stores.  The column maxima of
+// flight together with the rows, so the pass is one memory round trip, 16
+// substitution steps with 36 MFMAs between them and the stores.  The column maxima of
 // the current values go to the record: over the eligible rows rounded up to
 // float (colmax[parity], the threshold test) and exact (emax), over the rows
 // [nE, m) exact (nmax).
@@ -3206,7 +3210,6 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 2 : 3) void k_schur(const int
       for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
         for (int bj = 0; bj < 2; ++bj) acc[bi][bj] = typename M::v4{0, 0, 0, 0};
-#pragma unroll 4
       for (int kk = 0; kk < pp; kk += 4) {
         const T a0 = As[wr + lr][kk + lk];
         const T a1 = As[wr + 16 + lr][kk + lk];
@@ -3534,8 +3537,7 @@ void launchSyrk(const int* list, int count, const int* tileStart, const int* til
                 const DevFronts& fd, hipStream_t st) {
   if (count <= 0 || totalTiles <= 0) return;
   // persistent workgroups: as many as are resident at once (LDS and
-  // registers allow two per CU in FP64, four in FP32 with the kernel's
-  // register bound), so that none starts after the others have taken their
+  // registers allow two per CU in FP64, three in FP32), so that none starts after the others have taken their
   // share of tiles
   static int resident[2] = {0, 0};
   int& res = resident[fd.fp32 ? 1 : 0];
