@@ -1125,13 +1125,14 @@ __global__ __launch_bounds__(256) void k_front_maxabs(const int* list, int count
 // of four and eight columns before the blocks: 2.6); 2,000 rows 2.0 -> 1.1
 // (1.9); 1,000 rows 1.26 -> 0.72 (1.33).
 //
-// Measured per panel of 64 columns (FP64, before: sub-panels of eight columns
-// in LDS, each thread factoring the 8 x 8 block, rows loaded slot by slot):
-// 30x30x30 27-point fronts, few failing columns, <= 128 rows 103 -> 24 us,
-// <= 512 rows 103 -> 55, <= 2048 rows 153 -> 129; 100x100 5-point fronts, a
-// failing column in about every eight, 210 -> 105 us.  A block takes about
-// 15,000 cycles there (6,000 of them the diagonal block), a general step
-// 8,000.
+// Measured per panel of 64 columns (before: sub-panels of eight columns in LDS,
+// each thread factoring the 8 x 8 block, rows loaded slot by slot): 30x30x30
+// 27-point fronts, FP32, few failing columns, <= 128 rows 103 -> 24 us, <= 512
+// rows 103 -> 56, <= 2048 rows 153 -> 114; 100x100 5-point fronts, FP64, a
+// failing column in about every eight, 210 -> 100 us; dense FP64 panels that
+// pass, 1,000 rows 165 -> 81, 2,000 273 -> 157, 4,000 (streamed) 620 -> 300 us.
+// A block of the 5-point fronts takes about 15,000 cycles (6,000 of them the
+// diagonal block), a general step 8,000.
 constexpr int kPanelCols = 16;  // columns per block
 constexpr int kAloneAfter = 3;  // poor blocks in turn before columns are taken one by one,
 constexpr int kAloneRun = 4;    // until so many have passed in turn
@@ -2409,8 +2410,8 @@ __device__ inline double roundUpToFloat(double v) {
 // operands.
 //
 // Bound by the dependent chain of 64 pivots: 4 x 6,000 cycles, 10 us of the
-// 22 on the 80^3 27-point workload (a barrier per two pivots on registers and
-// LDS took 37; 28 against 45 with static pivots).
+// 21 on the 80^3 27-point workload (a barrier per two pivots on registers and
+// LDS took 37; 29 against 45 with static pivots).
 template <typename T>
 __global__ __launch_bounds__(256) void k_spec_block(const int* list, int count, DevFronts fd, FactorParams prm,
                                                     double* wsBase, const int64_t* wsOff) {
@@ -2550,7 +2551,7 @@ __global__ __launch_bounds__(256) void k_spec_block(const int* list, int count, 
 // [nE, m) exact (nmax).
 //
 // (One row per thread with the coefficients broadcast from LDS took 31 us a
-// launch on the 80^3 27-point workload, this form 19.)
+// launch on the 80^3 27-point workload, this form 21.)
 template <typename T>
 __global__ __launch_bounds__(4 * kSpecRows) void k_spec_factor(const int* list, int count, const int* wgStart,
                                                                int parity, DevFronts fd, FactorParams prm,
