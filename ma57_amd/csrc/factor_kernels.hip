@@ -1525,7 +1525,7 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
         return F[ok ? at(row, k0 + q) : 0];
     };
     int lrL = lr;  // (see acceptChunk)
-    asm volatile("" : "+v"(lrL));
+    if constexpr (TPW == 0 || TPW >= 8) asm volatile("" : "+v"(lrL));
     T raw[NTL][4];
 #pragma unroll
     for (int t = 0; t < NTL; ++t)
@@ -1742,11 +1742,12 @@ __global__ __launch_bounds__(kPanelThreads) void k_panel(const int* list, int co
     // (rows from an index that the compiler cannot match with the loads': their
     // 4 CT addresses would stay in registers over the whole block)
     int lrA = lr;
-    asm volatile("" : "+v"(lrA));
+    if constexpr (TPW == 0 || TPW >= 8) asm volatile("" : "+v"(lrA));
     auto acceptChunk = [&](int ch) {
 #pragma unroll
       for (int t = 0; t < CT; ++t) {
         const int row0 = rowOf(ch, t), row = row0 + lrA;
+        if (row0 >= rEnd || row0 + 16 <= c0) continue;
         T lt[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) lt[u] = multiplier<T>(x[t][u], dc[u], rdc[u]);
