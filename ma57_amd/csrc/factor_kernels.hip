@@ -1127,9 +1127,9 @@ __global__ __launch_bounds__(256) void k_front_maxabs(const int* list, int count
 //
 // Measured per panel of 64 columns (before: sub-panels of eight columns in LDS,
 // each thread factoring the 8 x 8 block, rows loaded slot by slot): 30x30x30
-// 27-point fronts, FP32, few failing columns, <= 128 rows 103 -> 24 us, <= 512
-// rows 103 -> 56, <= 2048 rows 153 -> 114; 100x100 5-point fronts, FP64, a
-// failing column in about every eight, 210 -> 100 us; dense FP64 panels that
+// 27-point fronts, FP32, few failing columns, <= 128 rows 103 -> 23 us, <= 512
+// rows 103 -> 54, <= 2048 rows 153 -> 107; 100x100 5-point fronts, FP64, a
+// failing column in about every eight, 210 -> 98 us; dense FP64 panels that
 // pass, 1,000 rows 165 -> 81, 2,000 273 -> 157, 4,000 (streamed) 620 -> 300 us.
 // A block of the 5-point fronts takes about 15,000 cycles (6,000 of them the
 // diagonal block), a general step 8,000.
